@@ -1302,6 +1302,9 @@ uint32_t flat_rows_per_pass(uint32_t k) {
     return fit < 1u ? 1u : fit < regs ? fit : regs;
 }
 
+// Whether a CU's LDS holds k f32 activations as plan_job lays them out (with their per-16 sums and the queue counter).
+inline bool gemv_row_fits(uint32_t k) { return (size_t)k * 4 + (size_t)(k / 16) * 4 + 16 <= 160 * 1024 - 512; }
+
 // How m f32 K-quant rows are walked in slices of k: rows and super-blocks to a pass (LDS holds the one over the other).
 struct FlatSlices {
     uint32_t rows, slices, units;
@@ -1340,7 +1343,9 @@ int launch_flat_slices(hipStream_t s, const float* x, const uint8_t* w, float* y
         }
     return HQ_OK;
 }
-// Whether they are: more rows than a CU's LDS holds whole, enough windows in a slice, and faster.  us at 3 .. 8 rows, before /
+// Whether they are: rows that the one-row kernels take too (launch_t plans those first; longer ones stay with the chunk-staged
+// kernel, which has no limit on k, or are refused at every row count), more rows than a CU's LDS holds whole, enough
+// windows in a slice, and faster.  us at 3 .. 8 rows, before /
 // here: Q6_K 4096 x 14336 30 / 26, 34 / 31, 44 / 50, 46 / 48 (5120 rows and more are ahead up to six: 12288 x 12288 103 / 71,
 // 105 / 78, 106 / 101 at 5 .. 7; 8192 x 28672 151 / 139, 155 / 154, 157 / 188); Q4_K 4096 x 12288 20 / 22, 23 / 25, 29 / 28;
 // 4096 x 14336 23 / 22, 27 / 26, 33 / 30, 32 / 46; 12288 x 12288 43 / 38, 52 / 47, 73 / 56; 8192 x 28672 91 / 65 in three slices, 92 / 92
@@ -1354,6 +1359,7 @@ bool flat_slices_take(uint32_t m, uint32_t n, uint32_t k, uint32_t cus, FlatSlic
     *plan = p;
     const bool chunks = k % 1024u == 0;  // the small-batch kernel's
     if (TYPE == HQ_Q6_K ? chunks && m > (n >= 20u * cus ? 6u : 4u) : (uint64_t)n * k < (7u << 23) || (chunks && (m > 5u || p.slices > 3u))) return false;
+    if (!gemv_row_fits(k)) return false;
     const uint32_t whole = flat_rows_per_pass<TYPE, false>(k);
     if (TYPE == HQ_Q6_K && whole >= 3u && m <= 2u * whole) return false;
     return p.slices >= 2 && p.slices <= 8 && whole < p.rows &&

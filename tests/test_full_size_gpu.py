@@ -648,3 +648,29 @@ def test_several_f32_rows_in_slices_of_k_of_the_flat_walk(oracle, dev, t, n, k):
             ops.quantized_matmul_ggml(x[:m], w, y, GgmlQuantizedMatmulParams(m, n, k, t))
         assert torch.isfinite(y[:m]).all() and torch.isnan(y[m:]).all()
         assert_matmul_close(y[:m][:, torch.as_tensor(rows, device=dev)].cpu().numpy(), ref[:m], f"{m} rows, {n}x{k} t={t} in slices")
+
+
+@pytest.mark.parametrize("n,k,m", [(8192, 40960, 4), (8192, 40960, 6), (4096, 49152, 5), (16384, 53248, 4)])
+def test_f32_rows_longer_than_the_one_row_kernels_take(oracle, dev, n, k, m):
+    """Q6_K rows of more activations than a CU's LDS holds: four to six f32 rows run through the kernel that stages them in
+    chunks (the slices of the flat walk start from kernels that need a whole row), sampled weight rows against the oracle."""
+    t = HQ_Q6_K
+    w = _quantized(dev, n, k, t, 3 + m)
+    x = torch.randn(m, k, generator=torch.Generator(device=dev).manual_seed(m), device=dev)
+    y = torch.full((m + 1, n), float("nan"), device=dev)
+    ops.quantized_matmul_ggml(x, w, y, GgmlQuantizedMatmulParams(m, n, k, t))
+    assert torch.isfinite(y[:m]).all() and torch.isnan(y[m]).all()
+    rows = np.unique(np.concatenate([[0, 15, 16, n - 2, n - 1], np.random.default_rng(n).integers(0, n, 12)]))
+    ref = oracle.qmatmul_f64(x.cpu().numpy(), _rows_of(w, rows, k, t, oracle), m, rows.size, k, t)
+    assert_matmul_close(y[:m][:, torch.as_tensor(rows, device=dev)].cpu().numpy(), ref, f"{m} rows, {n}x{k}")
+
+
+@pytest.mark.parametrize("t", [HQ_Q4_K, HQ_Q6_K])
+def test_f32_rows_refused_for_one_are_refused_for_several(dev, t):
+    """k of no whole chunks beyond a CU's LDS has no kernel at any row count."""
+    n, k = 8192, 38656
+    w, x = torch.zeros(n * ops.ggml_row_bytes(t, k), dtype=torch.uint8, device=dev), torch.zeros(8, k, device=dev)
+    for m in (1, 3, 8):
+        with pytest.raises(ops.HqError) as e:
+            ops.quantized_matmul_ggml(x[:m], w, torch.empty(m, n, device=dev), GgmlQuantizedMatmulParams(m, n, k, t))
+        assert e.value.status == 2 and "LDS" in str(e.value)
