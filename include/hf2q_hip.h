@@ -365,9 +365,12 @@ HQ_API int hq_moe_weighted_reduce(void* stream, const float* y, const float* w, 
  * `scratch`: hq_moe_ffn_decode_scratch_bytes() bytes of device memory, 256-byte aligned, ZEROED ONCE before its first
  * use and then left to the library (it carries a call counter; calls that share a scratch must not overlap, and a
  * scratch serves one (n_experts, top_k) shape).  The workgroups of the launch hand results to each other through it
- * and wait for each other with bounded polling; if a wait ever runs out (it cannot, unless the device is shared with a
- * kernel that starves the launch for seconds) the second 32-bit word of the scratch becomes non-zero and the output is
- * undefined.  route_ids / route_weights: NULL, or where the routing is also written ([n_tokens * top_k] each). */
+ * and wait for each other with bounded polling.  Launches over scratches of their own may overlap (streams, processes): a
+ * workgroup whose wait runs out, because the others have no CU yet, works out what it misses by itself, with the same
+ * bits; the launch then takes a millisecond or two instead of tens of microseconds.  Only a last workgroup that does not
+ * start for about a million polls (a device taken by other kernels for seconds) makes the second 32-bit word of the scratch
+ * non-zero; the scratch must then be zeroed again.  route_ids / route_weights: NULL, or where the routing is also
+ * written ([n_tokens * top_k] each). */
 typedef struct hq_moe_ffn_layer {
     const void* router;            /* [n_experts, hidden] bf16 */
     const void* shared_gate_logit; /* [hidden] bf16, or NULL: the shared expert enters with weight 1 */
@@ -393,12 +396,13 @@ HQ_API int hq_moe_ffn_decode(void* stream, const hq_moe_ffn_layer* layer, const 
                       uint32_t* route_ids, float* route_weights);
 
 /* The hand-over state of a scratch of hq_moe_ffn_decode or hq_dense_ffn_decode: *error receives the scratch's error
- * word (0: every wait inside the launches so far ended by itself; non-zero: one ran into the polling limit, the output
- * of that call is undefined and the scratch must be zeroed again before its next use).  Waits for `stream` (a 4-byte
+ * word (0: all is well; non-zero: hq_dense_ffn_decode ran into the polling limit and the output of that call is undefined,
+ * or see hq_moe_ffn_decode; the scratch must be zeroed again before its next use).  Waits for `stream` (a 4-byte
  * copy to the host): call it where the serving loop
- * synchronises anyway.  hq_set_handover_spin_limit sets the polling limit of launches made after it (0: the default,
- * about a million polls, seconds): a tiny limit makes every wait give up at once, which is how the tests exercise the
- * bail-out path without hanging anything. */
+ * synchronises anyway.  hq_set_handover_spin_limit sets the polling limit of launches made after it (0: the defaults,
+ * about a million polls, seconds, in hq_dense_ffn_decode; a few hundred, after which a workgroup finishes alone, in
+ * hq_moe_ffn_decode, which takes lower limits only): a tiny limit makes every wait give up at once, which is how the tests
+ * exercise those paths without hanging anything. */
 HQ_API int hq_handover_status(void* stream, const void* scratch, uint32_t* error);
 HQ_API void hq_set_handover_spin_limit(uint32_t limit);
 
@@ -415,7 +419,9 @@ HQ_API void hq_set_handover_spin_limit(uint32_t limit);
  * hq_dense_ffn_decode_scratch_bytes() returns 0, and the separate calls do the work.
  * `scratch`: hq_dense_ffn_decode_scratch_bytes() bytes of device memory, 256-byte aligned, ZEROED ONCE before its first
  * use and then left to the library (call counter, error word, hand-over words); calls that share a scratch must not
- * overlap.  The waits inside the launch are bounded (hq_handover_status). */
+ * overlap.  The waits inside the launch are bounded (hq_handover_status).  The launch wants every CU and its workgroups wait
+ * for all others of it: a call must not overlap another call of this function on another stream, or both may run into
+ * the limit. */
 HQ_API size_t hq_dense_ffn_decode_scratch_bytes(uint32_t hidden, uint32_t inter, hq_ggml_type t_gate_up, hq_ggml_type t_down,
                                          hq_act_dtype xdt);
 HQ_API int hq_dense_ffn_decode(void* stream, const void* x, hq_act_dtype xdt, const void* w_gate, const void* w_up,

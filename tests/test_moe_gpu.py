@@ -630,6 +630,48 @@ def test_hand_over_waits_give_up_at_the_spin_limit_and_report_it(oracle, dev):
     assert torch.equal(out, good) and ops.handover_status(scratch) == 0
 
 
+def _moe_weights_on_device(dev, t, td, H, E, K, I, seed):
+    g = torch.Generator(device=dev)
+    g.manual_seed(seed)
+    rnd = lambda n, k, s: torch.randn(n * k, generator=g, device=dev).mul_(s)  # noqa: E731
+    qz = lambda n, k, ty: ops.quantize_ggml(rnd(n, k, 0.05), k, ty)  # noqa: E731
+    dense = lambda n: rnd(n, H, 0.1).view(n, H).to(torch.bfloat16)  # noqa: E731
+    return ops.MoeFfnWeightsGpuQ(dense(E), qz(E * I, H, t), qz(E * I, H, t), qz(E * H, I, td), dense(1), qz(I, H, t), qz(I, H, t), qz(H, I, td),
+                                 t, H, E, K, I, I, down_type=None if td == t else td)
+
+
+@pytest.mark.parametrize("T,E", [(1, 24), (1, 256), (2, 256), (3, 24), (8, 24), (8, 256), (11, 32)])
+@pytest.mark.parametrize("t,td,xdt", [(HQ_Q5_K, HQ_Q6_K, torch.float32), (HQ_Q4_K, HQ_Q4_K, torch.bfloat16), (HQ_Q6_K, HQ_Q6_K, torch.float32)])
+def test_moe_block_out_of_patience_finishes_alone(dev, t, td, xdt, T, E):
+    """A workgroup that does not get what it waits for works it out by itself (no workgroup of the launch has to be resident
+    for another one to finish).  With a limit of one poll nearly every workgroup takes that way: the same bits, no error
+    reported, routing included, and the calls behind it with the default limit find the scratch in order."""
+    from hf2q_amd import lib
+    H, K, I = 2048, 8, 512
+    w = _moe_weights_on_device(dev, t, td, H, E, K, I, seed=T + E)
+    x, res = torch.from_numpy(acts(51 + T, T, H)).to(dev).to(xdt), torch.from_numpy(acts(52, T, H)).to(dev)
+    s = ops.MoeFfnScratch(w, T, dev)
+    ref = torch.full((T, H), float("nan"), device=dev)
+    ids = torch.empty(T * K, dtype=torch.int32, device=dev)
+    for t0 in range(0, T, 8):
+        ops.build_moe_ffn_layer_gpu_q_into(x[t0:t0 + 8], w, s, ref[t0:t0 + 8], residual=res[t0:t0 + 8], batched=True)
+        ids[t0 * K:(t0 + 8) * K] = s.ids[:min(8, T - t0) * K]
+    L = lib.load()
+    for limit in (1, 0, 2, 1, 0):
+        out = torch.full((T, H), float("nan"), device=dev)
+        s.ids.fill_(-1)
+        try:
+            L.hq_set_handover_spin_limit(limit)
+            for _ in range(2):  # (back to back: the next call starts while the last workgroups of this one leave)
+                ops.build_moe_ffn_layer_gpu_q_into(x, w, s, out, residual=res)
+            torch.cuda.synchronize()
+        finally:
+            L.hq_set_handover_spin_limit(0)
+        assert ops.handover_status(s.fused) == 0
+        assert torch.isfinite(out).all() and torch.equal(out, ref), (limit, (out - ref).abs().max().item())
+        assert torch.equal(s.ids, ids)
+
+
 def _moe_weights_mixed(oracle, dev, t, td, H, E, K, I, SI, seed=0):
     w = _moe_weights(oracle, dev, t, H, E, K, I, SI, seed=seed)
     if td != t:
