@@ -636,7 +636,7 @@ __global__ __launch_bounds__(64 * WAVES_) void moe_fused_kernel(FusedArgs a) {
 #pragma unroll
                     for (int i = 0; i < POLL; ++i) {
                         const uint32_t e2 = base + tid + (uint32_t)i * THREADS;
-                        off[i] = 16u * (e2 < n2 ? e2 : tid);  // past the end: a word of the thread's own, not used
+                        off[i] = 16u * (e2 < n2 ? e2 : n2 - 1u);  // past the end: the token's last words, not used
                     }
                     // (the wait stands in the block of the loads: no register of theirs is touched before they are back)
                     if constexpr (POLL == 5)

@@ -672,6 +672,24 @@ def test_moe_block_out_of_patience_finishes_alone(dev, t, td, xdt, T, E):
         assert torch.equal(s.ids, ids)
 
 
+@pytest.mark.parametrize("T", [1, 2, 5, 8])
+@pytest.mark.parametrize("K,xdt", [(1, torch.float32), (1, torch.bfloat16), (2, torch.float32), (3, torch.bfloat16)])
+def test_moe_block_one_launch_of_a_small_top_k(dev, T, K, xdt):
+    """One routed expert per token: fewer hand-over words than a workgroup has threads (the words asked for stay inside the
+    token's, the last token's inside the scratch, and no workgroup waits for any other word)."""
+    H, E, I = 2048, 16, 512
+    w = _moe_weights_on_device(dev, HQ_Q4_K, HQ_Q4_K, H, E, K, I, seed=K)
+    x = torch.from_numpy(acts(61 + T, T, H)).to(dev).to(xdt)
+    s = ops.MoeFfnScratch(w, T, dev)
+    ref = torch.full((T, H), float("nan"), device=dev)
+    ops.build_moe_ffn_layer_gpu_q_into(x, w, s, ref, batched=True)
+    for _ in range(3):
+        out = torch.full((T, H), float("nan"), device=dev)
+        ops.build_moe_ffn_layer_gpu_q_into(x, w, s, out)
+        assert ops.handover_status(s.fused) == 0 and int(s.fused[0:4].view(torch.int32).item()) > 0
+        assert torch.isfinite(out).all() and torch.equal(out, ref)
+
+
 def _moe_weights_mixed(oracle, dev, t, td, H, E, K, I, SI, seed=0):
     w = _moe_weights(oracle, dev, t, H, E, K, I, SI, seed=seed)
     if td != t:
