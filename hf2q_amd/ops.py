@@ -1038,7 +1038,9 @@ def build_moe_ffn_layer_gpu_q_into(x: torch.Tensor, w: MoeFfnWeightsGpuQ, s: Moe
         # (a scratch made for fewer tokens than this call brings is too small for the one-launch form: separate dispatches then)
         layer = w.c_layer()
         need = _moe_ffn_decode_fused_bytes(x, layer)
-        if 0 < need <= s.fused.numel():
+        # (and Q6_K stacks that lie on even addresses only, which that form does not take)
+        stacks = (layer.expert_gate | layer.expert_up | layer.expert_down | layer.shared_gate | layer.shared_up | layer.shared_down)
+        if 0 < need <= s.fused.numel() and stacks % 16 == 0:
             # one launch for the whole block, the bits of the batched dispatches below
             return _moe_ffn_decode_fused(x, w, layer, s, out, residual)
     if fused:

@@ -690,6 +690,24 @@ def test_moe_block_one_launch_of_a_small_top_k(dev, T, K, xdt):
         assert torch.isfinite(out).all() and torch.equal(out, ref)
 
 
+@pytest.mark.parametrize("T,xdt", [(1, torch.float32), (5, torch.float32), (12, torch.float32), (1, torch.bfloat16)])
+def test_moe_block_over_q6k_stacks_on_even_addresses(dev, T, xdt):
+    """Q6_K blocks need two-byte alignment only; the one-launch form wants sixteen, so the block runs as separate dispatches."""
+    H, E, K, I = 2048, 16, 4, 512
+    w = _moe_weights_on_device(dev, HQ_Q6_K, HQ_Q6_K, H, E, K, I, seed=T)
+    x = torch.from_numpy(acts(71 + T, T, H)).to(dev).to(xdt)
+    s = ops.MoeFfnScratch(w, T, dev)
+    ref, out = (torch.full((T, H), float("nan"), device=dev) for _ in range(2))
+    ops.build_moe_ffn_layer_gpu_q_into(x, w, s, ref, fused=False)
+    for name in ("expert_gate", "expert_up", "expert_down", "shared_gate", "shared_up", "shared_down"):
+        q = getattr(w, name)
+        odd = torch.empty(q.numel() + 16, dtype=torch.uint8, device=dev)[2:2 + q.numel()]
+        setattr(w, name, odd.copy_(q))
+    assert w.expert_down.data_ptr() % 16 == 2
+    ops.build_moe_ffn_layer_gpu_q_into(x, w, s, out)
+    assert torch.isfinite(out).all() and torch.equal(out, ref)
+
+
 def _moe_weights_mixed(oracle, dev, t, td, H, E, K, I, SI, seed=0):
     w = _moe_weights(oracle, dev, t, H, E, K, I, SI, seed=seed)
     if td != t:
