@@ -989,8 +989,8 @@ def _moe_ffn_decode_fused(x, w, layer, s, out, residual) -> None:
     if s.fused is None:
         raise _l.HqError(_l.HQ_ERR_UNSUPPORTED, "no scratch for the one-launch MoE block (shape not supported)")
     L, st, xdt, H, K = _l.load(), _stream(), _act_dtype(x), w.hidden, w.top_k
-    if x.shape[1] != H or out.numel() < T * H or (residual is not None and residual.numel() < T * H) or s.ids.numel() < T * K:
-        raise ValueError(f"x must be [{T}, {H}], out and residual as large, and the scratch made for {T} tokens")
+    if x.numel() < T * H or out.numel() < T * H or (residual is not None and residual.numel() < T * H) or s.ids.numel() < T * K:
+        raise ValueError(f"x, out and residual must hold {T} rows of {H}, and the scratch be made for {T} tokens")
     xp, op, rp = _dev(x, "x"), _dev(out, "out"), _dev(residual, "residual") if residual is not None else None
     fp, ip, wp, fb, lp = _dev(s.fused, "scratch"), _dev(s.ids, "ids"), _dev(s.topk_w, "topk_w"), s.fused.numel(), ctypes.byref(layer)
     # more than eight tokens (up to _FUSED_CHUNKED_MAX_TOKENS): one launch per eight, one after the other over the same scratch

@@ -708,6 +708,19 @@ def test_moe_block_over_q6k_stacks_on_even_addresses(dev, T, xdt):
     assert torch.isfinite(out).all() and torch.equal(out, ref)
 
 
+@pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16])
+def test_moe_block_takes_activations_with_a_sequence_axis(dev, xdt):
+    """x, out and residual as [tokens, 1, hidden], as a decode step's hidden state comes."""
+    H, E, K, I, T = 2048, 16, 4, 512, 10
+    w = _moe_weights_on_device(dev, HQ_Q4_K, HQ_Q4_K, H, E, K, I, seed=3)
+    x, res = torch.from_numpy(acts(81, T, H)).to(dev).to(xdt), torch.from_numpy(acts(82, T, H)).to(dev)
+    s = ops.MoeFfnScratch(w, T, dev)
+    ref, out = (torch.full((T, 1, H), float("nan"), device=dev) for _ in range(2))
+    ops.build_moe_ffn_layer_gpu_q_into(x, w, s, ref.view(T, H), residual=res)
+    ops.build_moe_ffn_layer_gpu_q_into(x.view(T, 1, H), w, s, out, residual=res.view(T, 1, H))
+    assert torch.isfinite(out).all() and torch.equal(out, ref)
+
+
 def _moe_weights_mixed(oracle, dev, t, td, H, E, K, I, SI, seed=0):
     w = _moe_weights(oracle, dev, t, H, E, K, I, SI, seed=seed)
     if td != t:
