@@ -262,7 +262,7 @@ def quantized_matmul_id_swiglu_ggml(input: torch.Tensor, gate_stack: torch.Tenso
         params.n_experts, params.expert_stride, params.ggml_type))
 
 
-@dataclass(slots=True)
+@dataclass
 class QmatmulJob:
     """One product of a batched launch: the arguments of quantized_matmul_id_ggml (ids set) or of
     quantized_matmul_ggml (ids None, m <= 8).  With `input_up` the activations are

@@ -191,3 +191,12 @@ def test_flat_walk_plan_covers_every_row_with_no_empty_window():
     assert L.hq_gemv_flat_plan(16, 256, lib.HQ_Q4_K, 4096, *refs) == lib.HQ_ERR_INVALID_ARGUMENT   # a single unit per row
     assert L.hq_gemv_flat_plan(16, 512, lib.HQ_Q4_K, 0, *refs) == lib.HQ_ERR_INVALID_ARGUMENT
     assert L.hq_gemv_flat_plan(16, 512, lib.HQ_Q4_K, 4096, None, *refs[1:]) == lib.HQ_ERR_INVALID_ARGUMENT
+
+
+def test_a_batch_job_takes_attributes_and_weak_references():
+    import weakref
+
+    from hf2q_amd import ops
+    j = ops.QmatmulJob(None, None, None, 1, 1, 256)
+    j.label = "q"
+    assert weakref.ref(j)() is j and j.label == "q"
