@@ -120,7 +120,8 @@ struct MoeBufs {
 
 hq_ggml_type down_type(const hq_moe_ffn_layer& l) { return l.down_type ? (hq_ggml_type)l.down_type : l.ggml_type; }
 
-MoeBufs carve_moe(Carver& c, const hq_moe_ffn_layer& l, uint32_t T, hq_act_dtype xdt) {
+// exact_ws: with the workspace of routed products that have a grouped form of exact products; such calls run as GEMVs without.
+MoeBufs carve_moe(Carver& c, const hq_moe_ffn_layer& l, uint32_t T, hq_act_dtype xdt, bool exact_ws = true) {
     MoeBufs b{};
     const uint32_t K = l.top_k, E = l.n_experts, H = l.hidden, I = l.inter, SI = l.shared_inter;
     const hq_ggml_type t = l.ggml_type, td = down_type(l);
@@ -137,9 +138,11 @@ MoeBufs carve_moe(Carver& c, const hq_moe_ffn_layer& l, uint32_t T, hq_act_dtype
     b.sh_up = c.take<float>((size_t)T * SI);
     b.sh_act = c.take<float>((size_t)T * SI);
     b.sh_down = c.take<float>((size_t)T * H);
+    auto id_ws = [&](uint32_t nt, uint32_t k_top, uint32_t n, uint32_t k, uint64_t stride, hq_ggml_type ty) {
+        return !exact_ws && gemm_f16_grouped_exact(ty, k) ? 0 : hq_qmatmul_id_ggml_workspace_bytes(nt, k_top, n, k, E, stride, ty);
+    };
     b.id_ws_bytes = max3(hq_qmatmul_id_swiglu_ggml_workspace_bytes(T, K, I, H, E, l.expert_stride_gate_up, t),
-                         hq_qmatmul_id_ggml_workspace_bytes(T, K, I, H, E, l.expert_stride_gate_up, t),
-                         hq_qmatmul_id_ggml_workspace_bytes((uint32_t)TK, 1, H, I, E, l.expert_stride_down, td));
+                         id_ws(T, K, I, H, l.expert_stride_gate_up, t), id_ws((uint32_t)TK, 1, H, I, l.expert_stride_down, td));
     b.id_ws = b.id_ws_bytes ? c.bytes(b.id_ws_bytes) : nullptr;
     b.dense_ws_bytes = max3(hq_qmatmul_swiglu_ggml_workspace_bytes(T, SI, H, xdt, t), hq_qmatmul_ggml_workspace_bytes(T, SI, H, xdt, t),
                             hq_qmatmul_ggml_workspace_bytes(T, H, SI, HQ_F32, td));
@@ -325,7 +328,11 @@ int hq_moe_ffn_prefill(void* stream, const hq_moe_ffn_layer* layer, const hq_moe
     if (!route_ids != !route_weights) return fail(HQ_ERR_INVALID_ARGUMENT, "%s: route_ids and route_weights go together", fn);
     if (!is_aligned(scratch, 256)) return fail(HQ_ERR_INVALID_ARGUMENT, "%s: scratch must be 256-byte aligned", fn);
     Carver c{static_cast<uint8_t*>(scratch)};
-    const MoeBufs b = carve_moe(c, *layer, n_tokens, xdt);
+    MoeBufs b = carve_moe(c, *layer, n_tokens, xdt);
+    if (scratch_bytes < c.used) {  // (a size kept from before the exact grouped form: enough for everything else)
+        c = Carver{static_cast<uint8_t*>(scratch)};
+        b = carve_moe(c, *layer, n_tokens, xdt, false);
+    }
     if (scratch_bytes < c.used) return fail(HQ_ERR_INVALID_ARGUMENT, "%s: scratch of %zu bytes, %zu needed", fn, scratch_bytes, c.used);
     if (int rc = moe_steps(stream, *layer, row_scales, x, xdt, residual, out, n_tokens, b)) return rc;
     if (route_ids) {

@@ -200,3 +200,15 @@ def test_a_batch_job_takes_attributes_and_weak_references():
     j = ops.QmatmulJob(None, None, None, 1, 1, 256)
     j.label = "q"
     assert weakref.ref(j)() is j and j.label == "q"
+
+
+def test_workspaces_of_the_grouped_products_keep_their_sizes():
+    """A caller may hold a size it asked for once: the tile table of the forms that cut tiles of 64 rows or more is sized for those."""
+    L = lib.load()
+    row = {lib.HQ_Q4_K: 144, lib.HQ_Q5_K: 176, lib.HQ_Q6_K: 210}
+    pad = lambda b: (b + 255) // 256 * 256  # noqa: E731
+    for t in row:
+        for T, K, n, k, E in ((2048, 8, 1024, 2048, 256), (333, 8, 1408, 2816, 128), (2664, 1, 2048, 512, 64)):
+            pairs = T * K
+            want = pad(T * k * 2) + pad(T * 4) + pad(E * n * 4) + pad(pairs * 4) + pad(16 * (pairs // 64 + E)) + 256
+            assert L.hq_qmatmul_id_ggml_workspace_bytes(T, K, n, k, E, n * (k // 256) * row[t], t) == want

@@ -721,6 +721,25 @@ def test_moe_block_takes_activations_with_a_sequence_axis(dev, xdt):
     assert torch.isfinite(out).all() and torch.equal(out, ref)
 
 
+def test_moe_prefill_takes_a_scratch_without_the_exact_products_workspace(dev):
+    """Q8_0 expert rows that are no multiple of 128: with a scratch that lacks the grouped form's workspace (the size such a
+    layer asked for before it had that form) the down products run as GEMVs, to the same accuracy (f32 sums of 96 terms)."""
+    H, E, K, I, T, t = 512, 8, 4, 96, 64, HQ_Q8_0
+    w = _moe_weights_on_device(dev, t, t, H, E, K, I, seed=9)
+    x = torch.from_numpy(acts(91, T, H)).to(dev)
+    need = ops.moe_ffn_prefill_scratch_bytes(w, T, x.dtype)
+    ws = ops.quantized_matmul_id_workspace_bytes(ops.GgmlQuantizedMatmulIdParams(T * K, 1, H, I, E, H * ops.ggml_row_bytes(t, I), t))
+    gate = ops.quantized_matmul_id_workspace_bytes(ops.GgmlQuantizedMatmulIdParams(T, K, I, H, E, I * ops.ggml_row_bytes(t, H), t))
+    assert ws > gate
+    full, small = torch.full((T, H), float("nan"), device=dev), torch.full((T, H), float("nan"), device=dev)
+    ops.moe_ffn_prefill(x, w, full, torch.empty(need, dtype=torch.uint8, device=dev))
+    less = need - (ws + 255) // 256 * 256 + (gate + 255) // 256 * 256
+    ops.moe_ffn_prefill(x, w, small, torch.empty(less, dtype=torch.uint8, device=dev))
+    assert torch.isfinite(small).all() and (full - small).abs().max() <= 1e-5 * full.abs().max()
+    with pytest.raises(ops.HqError):
+        ops.moe_ffn_prefill(x, w, small, torch.empty(less - 256, dtype=torch.uint8, device=dev))
+
+
 def _moe_weights_mixed(oracle, dev, t, td, H, E, K, I, SI, seed=0):
     w = _moe_weights(oracle, dev, t, H, E, K, I, SI, seed=seed)
     if td != t:
