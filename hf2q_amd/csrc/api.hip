@@ -473,7 +473,7 @@ constexpr uint64_t kGroupedRowsPerExpert = 3;
 bool grouped_route(uint32_t n_tokens, uint32_t top_k, uint32_t n, uint32_t k, uint32_t n_experts, uint64_t expert_stride,
                    hq_ggml_type t) {
     const uint64_t pairs = (uint64_t)n_tokens * top_k;
-    // The form of exact products gives the GEMV's results at any row count: from one row per expert on it is the faster one
+    // The form of exact products has the GEMV's accuracy at any row count: from one row per expert on it is the faster one
     // (gate_up Q6_K GEMVs + Q8_0 down of 2816 x 704, 128 experts, top-8: 116 us with GEMVs against 123 at 11 tokens, 187
     // against 171 at 16, 472 against 327 at 47).
     if (gemm_f16_grouped_exact(t, k))
@@ -533,7 +533,7 @@ int qmatmul_id(const char* fn, void* stream, const void* x, hq_act_dtype xdt, co
     const uint64_t pairs = (uint64_t)n_tokens * top_k;
     if (pairs == 0) return HQ_OK;
     // Many rows per expert and a workspace from the caller: rows sorted by expert, tile GEMM per expert.
-    // (The exact form gives what the GEMVs give: a scratch too small for it, which such calls could pass before the form
+    // (The exact form is as accurate as the GEMVs: a scratch too small for it, which such calls could pass before the form
     // existed, leaves them to the GEMVs.)
     const size_t need = grouped_route(n_tokens, top_k, n, k, n_experts, expert_stride, t)
                             ? gemm_f16_grouped_workspace_bytes(n_tokens, top_k, n_experts, n, k, t) : 0;

@@ -124,8 +124,8 @@ int launch_gemm_f16_swiglu(hipStream_t s, const void* x, hq_act_dtype xdt, const
 // Grouped form of the tile GEMM for mul_mat_id with many routed rows: rows sorted by expert, one
 // tile = up to 256 rows of one expert; needs a contiguous stack (expert_stride = n rows) and a device
 // workspace of gemm_f16_grouped_workspace_bytes().
-// Whether (t, k) takes the grouped form whose products are exact (Q8_0 / Q4_0, k % 128 != 0): its results do not depend on
-// the number of rows, so the rows from which it runs are a matter of time alone.
+// Whether (t, k) takes the grouped form whose products are exact (Q8_0 / Q4_0, k % 128 != 0): it is as accurate as a GEMV per
+// row (the sums are taken in another order), so the rows from which it runs are a matter of time alone.
 bool gemm_f16_grouped_exact(hq_ggml_type t, uint32_t k);
 bool gemm_f16_grouped_supported(hq_ggml_type t, uint32_t n, uint32_t k, uint32_t n_experts, uint64_t expert_stride, uint64_t pairs);
 size_t gemm_f16_grouped_workspace_bytes(uint32_t n_tokens, uint32_t top_k, uint32_t n_experts, uint32_t n, uint32_t k,

@@ -504,8 +504,7 @@ def test_mul_mat_id_swiglu_has_no_form_for_other_types_and_small_calls(dev):
 ])
 def test_mul_mat_id_grouped_exact_rows_of_odd_length(oracle, dev, t, xdt, E, n, k, T, K):
     """Q8_0 / Q4_0 rows that are no multiple of 128 weights: the grouped form multiplies the integers exactly and scales every
-    block in f32, with f32 activations as two f16 parts (22 bits: 2^-23 per term, below the 2^-24 sqrt(k) of f32 sums at
-    these k).  Bound: 2e-5 of the output's rms per element, where the form that rounds weights to f16 shows 1e-3."""
+    block in f32, with f32 activations as three bf16 parts (all 24 bits).  Bound: 2e-5 of the output's rms per element, where the form that rounds weights to f16 shows 1e-3."""
     stack, ids, xv, xd, p = _grouped_setup(oracle, dev, t, E, n, k, T, K, xdt, seed=21)
     need = ops.quantized_matmul_id_workspace_bytes(p)
     assert need > 0, "this shape must take the grouped route"
@@ -524,6 +523,52 @@ def test_mul_mat_id_grouped_exact_rows_of_odd_length(oracle, dev, t, xdt, E, n, 
     ops.quantized_matmul_id_ggml(xd, sd, idd, y2, p, scratch=scratch)
     keep = np.setdiff1d(np.arange(T * K), [3])
     assert torch.isnan(y2[3]).all() and torch.equal(y2[keep], y[keep])
+
+
+@pytest.mark.parametrize("t", [HQ_Q8_0, HQ_Q4_0])
+@pytest.mark.parametrize("xdt", ["bf16", "f32"])
+def test_mul_mat_id_grouped_exact_rows_of_uneven_magnitudes(oracle, dev, t, xdt):
+    """Activations of 1e4 .. 1e8 that meet zero weights beside others of N(0, 1), and whole rows of 1e30 or 1e-25: every product is
+    exact, so the error is that of f32 sums of 22 block sums (2^-24 sqrt(22) = 2.8e-7 of the rms); bound 2e-6 per element."""
+    E, n, k, T, K = 8, 96, 704, 40, 2
+    _, ids, _, _, p = _grouped_setup(oracle, dev, t, E, n, k, T, K, xdt, seed=5)
+    w = weights(17, E * n, k)
+    w[:, 5::97] = 0.0
+    stack = oracle.quantize(w, k, t, threads=8)
+    x = acts(23, T, k)
+    x[:, 5::97] = np.array([1e4, 1e5, 1e6, 1e7, 1e8], np.float32)[np.arange(T) % 5][:, None]
+    x[7], x[8] = acts(24, 1, k)[0] * np.float32(1e30), acts(25, 1, k)[0] * np.float32(1e-25)
+    xd = torch.from_numpy(x).to(dev)
+    xd = xd.to(torch.bfloat16) if xdt == "bf16" else xd
+    xv = oracle.f32_to_bf16_bits(x) if xdt == "bf16" else x
+    ref = oracle.qmatmul_id_f64(xv, stack, ids, T, K, n, k, E, p.expert_stride, t)
+    scratch = torch.empty(ops.quantized_matmul_id_workspace_bytes(p), dtype=torch.uint8, device=dev)
+    y = torch.full((T * K, n), float("nan"), device=dev)
+    ops.quantized_matmul_id_ggml(xd, torch.from_numpy(stack).to(dev), torch.from_numpy(ids.view(np.int32)).to(dev), y, p, scratch=scratch)
+    err = np.abs(y.cpu().numpy().astype(np.float64) - ref).max(axis=1) / np.sqrt(np.mean(ref * ref, axis=1))
+    assert err.max() <= 2e-6, err.max()
+
+
+@pytest.mark.parametrize("t", [HQ_Q8_0, HQ_Q4_0])
+def test_mul_mat_id_grouped_exact_rows_keep_inf_and_nan(oracle, dev, t):
+    """inf and nan activations (a nan of low bits among them) give results that are not finite where a GEMV per row does, and
+    nowhere else (the Q4_0 GEMV takes eight times the sum of the activations away, nan where this form has inf)."""
+    E, n, k, T, K = 4, 64, 96, 40, 2
+    stack, ids, _, _, p = _grouped_setup(oracle, dev, t, E, n, k, T, K, "f32", seed=6)
+    x = acts(29, T, k)
+    x[3, 11], x[4, 40], x[5, 95], x[6, 0] = np.inf, -np.inf, np.nan, 1e36
+    x.view(np.uint32)[9, 33] = 0x7f800001
+    xd, sd, idd = torch.from_numpy(x).to(dev), torch.from_numpy(stack).to(dev), torch.from_numpy(ids.view(np.int32)).to(dev)
+    scratch = torch.empty(ops.quantized_matmul_id_workspace_bytes(p), dtype=torch.uint8, device=dev)
+    y, g = (torch.zeros(T * K, n, device=dev) for _ in range(2))
+    ops.quantized_matmul_id_ggml(xd, sd, idd, y, p, scratch=scratch)
+    ops.quantized_matmul_id_ggml(xd, sd, idd, g, p)
+    assert torch.equal(torch.isfinite(y), torch.isfinite(g)) and torch.isnan(y).any() and torch.isinf(y).any()
+    if t == HQ_Q8_0:
+        assert torch.equal(torch.isnan(y), torch.isnan(g)) and torch.equal(y[torch.isinf(y)], g[torch.isinf(g)])
+    for r in range(T * K):
+        fin = torch.isfinite(g[r])
+        assert (y[r][fin] - g[r][fin]).abs().max() <= 4e-6 * g[r][fin].abs().max() if fin.any() else True
 
 
 def test_mul_mat_id_grouped_routing_properties(oracle, dev):
