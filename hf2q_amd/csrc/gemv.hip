@@ -1702,6 +1702,8 @@ int launch_jobs_t(hipStream_t s, const GemvArgs* jobs, uint32_t n_jobs) {
 // Where the small-batch kernel has its stage-once form (gemv_rows_stream_fast: Q6_K 151936 x 4096 134 us, Q4_K 65536 x 4096
 // 41 us, Q4_K / Q6_K 12288 x 4096 13 / 21 us for any 3 .. 8 rows) it is ahead from five rows on, and from three on
 // matrices of 32768 rows or more (three and four rows in passes: 55 / 62 us on the 65536-row Q4_K matrix).
+// (Q6_K 32768 x 12288, five to seven rows: the small-batch kernel in slices of k takes 90 us against 146, but its error is
+// 1.2e-6 of the result where these passes have 1.4e-7: they stay.)
 // The flat walk's plan for an n x k matrix of type t on `waves` waves (host arithmetic).
 void gemv_flat_plan(hq_ggml_type t, uint32_t n, uint32_t k, uint32_t waves, uint32_t* units_per_row, uint32_t* rows_per_task,
                     uint32_t* windows_per_task, uint32_t* units_per_window, uint32_t* window_capacity) {
@@ -1717,8 +1719,6 @@ void gemv_flat_plan(hq_ggml_type t, uint32_t n, uint32_t k, uint32_t waves, uint
 
 bool gemv_stream_passes_preferred(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32_t n, uint32_t k) {
     if (xdt != HQ_BF16 || m < 3) return false;
-    // (Q6_K 32768 x 12288: five rows 146 us in such passes, 90 in slices of k of the small-batch kernel)
-    if (m >= 5 && n >= 32768) return false;
     uint32_t cus = 0;
     if (cu_count(&cus)) return false;
     if (gemv_rows_stream_fast(t, xdt, m, n, k) && (m >= 5 || n >= 32768)) return false;

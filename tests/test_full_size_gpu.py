@@ -674,3 +674,18 @@ def test_f32_rows_refused_for_one_are_refused_for_several(dev, t):
         with pytest.raises(ops.HqError) as e:
             ops.quantized_matmul_ggml(x[:m], w, torch.empty(m, n, device=dev), GgmlQuantizedMatmulParams(m, n, k, t))
         assert e.value.status == 2 and "LDS" in str(e.value)
+
+
+@pytest.mark.parametrize("n,k,m", [(32768, 12288, 5), (32771, 12288, 7), (65536, 8192, 6)])
+def test_bf16_rows_over_long_q6k_rows_keep_f32_products(oracle, dev, n, k, m):
+    """Five to seven bf16 rows over Q6_K rows too long for the small-batch kernel's one-launch form run in passes whose products
+    are f32: error of the sampled rows at most 4e-7 of the result (f32 sums over 16 lanes and 48 pieces: 2^-24 sqrt(48) = 4.1e-7)."""
+    t = HQ_Q6_K
+    w = _quantized(dev, n, k, t, 31)
+    x = torch.randn(m, k, generator=torch.Generator(device=dev).manual_seed(k), device=dev).to(torch.bfloat16)
+    y = torch.full((m, n), float("nan"), device=dev)
+    ops.quantized_matmul_ggml(x, w, y, GgmlQuantizedMatmulParams(m, n, k, t))
+    rows = np.arange(n // 2, n // 2 + 64)
+    ref = oracle.qmatmul_f64(oracle.f32_to_bf16_bits(x.float().cpu().numpy()), _rows_of(w, rows, k, t, oracle), m, rows.size, k, t).reshape(m, -1)
+    got = y[:, n // 2:n // 2 + 64].cpu().numpy().astype(np.float64)
+    assert np.linalg.norm(got - ref) <= 4e-7 * np.linalg.norm(ref)
