@@ -982,7 +982,8 @@ int launch_gemv_rows(hipStream_t s, const void* x, hq_act_dtype xdt, const void*
     // k whose activations leave no room for the piece buffers: slices of k, one launch each, the later ones adding to y.
     // Q6_K 152064 x 5120 at 5 f32 rows 383 us in one launch without the transposed fetch, 167 in two slices (bf16 240 -> 165);
     // 151936 x 4096 f32 241 -> 140; Q4_K 248320 x 5120 f32 289 -> 169.
-    if (n >= kSliceMinRows) {
+    // (Q4_K / Q5_K of less than 4096 weights per row gain nothing: Q5_K 152064 x 3584 91 us in one launch, 96 in two slices; Q4_K 80, 80)
+    if (n >= kSliceMinRows && (k >= 4096 || (t != HQ_Q4_K && t != HQ_Q5_K))) {
         const uint32_t nsb = k / 256u;
         for (uint32_t slices = 2; k % 256u == 0 && slices <= kMaxSlices && nsb >= 2u * slices; ++slices) {
             const uint32_t per = (nsb + slices - 1u) / slices * 256u;
