@@ -473,13 +473,25 @@ constexpr uint64_t kGroupedRowsPerExpert = 3;
 bool grouped_route(uint32_t n_tokens, uint32_t top_k, uint32_t n, uint32_t k, uint32_t n_experts, uint64_t expert_stride,
                    hq_ggml_type t) {
     const uint64_t pairs = (uint64_t)n_tokens * top_k;
-    // The form of exact products has the GEMV's accuracy at any row count: from one row per expert on it is the faster one
-    // (gate_up Q6_K GEMVs + Q8_0 down of 2816 x 704, 128 experts, top-8: 116 us with GEMVs against 123 at 11 tokens, 187
-    // against 171 at 16, 472 against 327 at 47).
+    // (the form of exact products: what a workspace is asked for; exact_ahead says whether the call uses it)
     if (gemm_f16_grouped_exact(t, k))
         return pairs >= 64 && pairs >= n_experts && gemm_f16_grouped_supported(t, n, k, n_experts, expert_stride, pairs);
     return pairs >= 256 && pairs >= kGroupedRowsPerExpert * n_experts &&
            gemm_f16_grouped_supported(t, n, k, n_experts, expert_stride, pairs);
+}
+// The form of exact products has the GEMV's accuracy at any row count, so that its line is a matter of time.  GEMVs cost the
+// products (0.25 .. 0.6 us per million), this form about 12 us, 1 us per 64 of k and the weights of the experts met, once.
+// us, GEMVs / this form, f32 rows: from 64 rows on where there are two per expert (8 experts of 2816 x 704 Q8_0 at 64 rows 35 / 22,
+// 32 of 2048 x 736 37 / 36), else from 128 rows and 2^27 products on (64 experts of 2816 x 704 at 64 rows 36 / 48, at 88 46 / 51, at 128 77 / 51; 60 of
+// 2048 x 1440 Q4_0 49 / 72, 88 / 90, 89 / 90; 128 of 2816 x 704 at 128 82 / 73; 256 of 2048 x 352 at 256 113 / 69; 100 of 1024 x 608 Q4_0 at 128 25 / 38); and from 2^26
+// products on (8 experts of 1024 x 96 at 512 rows 13 / 18, of 512 x 352 at 256 21 / 25, at 512 33 / 26; 64 of 512 x 224 at 256
+// 14 / 17; 16 of 4096 x 96 at 128 13 / 15, at 256 18 / 16).  bf16 rows, whose GEMVs take half the time at long k, later there (60
+// experts of 2048 x 1440 Q4_0 at 128 / 192 / 256 rows 45 / 62 / 80 as GEMVs, 79 / 79 / 80 in this form; 16 of 512 x 1440 Q8_0 at
+// 192 / 256 / 512 29 / 36 / 64, 36 / 37 / 40).
+bool exact_ahead(hq_act_dtype xdt, uint64_t pairs, uint32_t n, uint32_t k, uint32_t n_experts) {
+    const uint64_t products = pairs * n * k;
+    if (pairs < 2ull * n_experts ? pairs < 128 || products < 1ull << 27 : products < 1ull << 26) return false;
+    return xdt != HQ_BF16 || k < 1024 || (pairs >= 4ull * n_experts && products >= 3ull << 26);
 }
 }  // namespace
 
@@ -538,7 +550,7 @@ int qmatmul_id(const char* fn, void* stream, const void* x, hq_act_dtype xdt, co
     const size_t need = grouped_route(n_tokens, top_k, n, k, n_experts, expert_stride, t)
                             ? gemm_f16_grouped_workspace_bytes(n_tokens, top_k, n_experts, n, k, t) : 0;
     const bool fits = scratch && scratch_bytes >= need && reinterpret_cast<uintptr_t>(scratch) % 256 == 0;
-    if (scratch && need && (fits || !gemm_f16_grouped_exact(t, k))) {
+    if (scratch && need && (!gemm_f16_grouped_exact(t, k) || (fits && exact_ahead(xdt, pairs, n, k, n_experts)))) {
         if (scratch_bytes < need)
             return fail(HQ_ERR_INVALID_ARGUMENT, "%s: scratch of %zu bytes, %zu needed", fn, scratch_bytes, need);
         if (reinterpret_cast<uintptr_t>(scratch) % 256)

@@ -223,8 +223,8 @@ HQ_API int hq_qmatmul_perm021_ggml_ws(void* stream, const void* x_perm, hq_act_d
  * GEMM of the m > 8 route (the reference's mul_mm_id, forward_mlx.rs:5237-5245);
  * that form needs a contiguous stack (expert_stride = one expert's bytes).
  * Q8_0 / Q4_0 rows whose k is no multiple of 128 have a grouped form that
- * keeps every product exact, as the GEMVs do; it runs from one routed row per
- * expert (and 64 rows) on.
+ * keeps every product exact, as the GEMVs do; it runs from about one routed row
+ * per expert and 64 .. 128 rows on, small products excepted.
  * With scratch == NULL every size takes the GEMV form. */
 HQ_API int hq_qmatmul_id_ggml(void* stream, const void* x, hq_act_dtype xdt, const void* w_stack,
                        const uint32_t* ids, float* y, void* scratch, size_t scratch_bytes,

@@ -530,7 +530,7 @@ def test_mul_mat_id_grouped_exact_rows_of_odd_length(oracle, dev, t, xdt, E, n, 
 def test_mul_mat_id_grouped_exact_rows_of_uneven_magnitudes(oracle, dev, t, xdt):
     """Activations of 1e4 .. 1e8 that meet zero weights beside others of N(0, 1), and whole rows of 1e30 or 1e-25: every product is
     exact, so the error is that of f32 sums of 22 block sums (2^-24 sqrt(22) = 2.8e-7 of the rms); bound 2e-6 per element."""
-    E, n, k, T, K = 8, 96, 704, 40, 2
+    E, n, k, T, K = 8, 1202, 704, 40, 2
     _, ids, _, _, p = _grouped_setup(oracle, dev, t, E, n, k, T, K, xdt, seed=5)
     w = weights(17, E * n, k)
     w[:, 5::97] = 0.0
@@ -542,9 +542,10 @@ def test_mul_mat_id_grouped_exact_rows_of_uneven_magnitudes(oracle, dev, t, xdt)
     xd = xd.to(torch.bfloat16) if xdt == "bf16" else xd
     xv = oracle.f32_to_bf16_bits(x) if xdt == "bf16" else x
     ref = oracle.qmatmul_id_f64(xv, stack, ids, T, K, n, k, E, p.expert_stride, t)
-    scratch = torch.empty(ops.quantized_matmul_id_workspace_bytes(p), dtype=torch.uint8, device=dev)
+    scratch = torch.full((ops.quantized_matmul_id_workspace_bytes(p),), 255, dtype=torch.uint8, device=dev)
     y = torch.full((T * K, n), float("nan"), device=dev)
     ops.quantized_matmul_id_ggml(xd, torch.from_numpy(stack).to(dev), torch.from_numpy(ids.view(np.int32)).to(dev), y, p, scratch=scratch)
+    assert (scratch != 255).any(), "the grouped form did not run"
     err = np.abs(y.cpu().numpy().astype(np.float64) - ref).max(axis=1) / np.sqrt(np.mean(ref * ref, axis=1))
     assert err.max() <= 2e-6, err.max()
 
@@ -553,22 +554,51 @@ def test_mul_mat_id_grouped_exact_rows_of_uneven_magnitudes(oracle, dev, t, xdt)
 def test_mul_mat_id_grouped_exact_rows_keep_inf_and_nan(oracle, dev, t):
     """inf and nan activations (a nan of low bits among them) give results that are not finite where a GEMV per row does, and
     nowhere else (the Q4_0 GEMV takes eight times the sum of the activations away, nan where this form has inf)."""
-    E, n, k, T, K = 4, 64, 96, 40, 2
+    E, n, k, T, K = 4, 2200, 96, 160, 2
     stack, ids, _, _, p = _grouped_setup(oracle, dev, t, E, n, k, T, K, "f32", seed=6)
     x = acts(29, T, k)
     x[3, 11], x[4, 40], x[5, 95], x[6, 0] = np.inf, -np.inf, np.nan, 1e36
     x.view(np.uint32)[9, 33] = 0x7f800001
     xd, sd, idd = torch.from_numpy(x).to(dev), torch.from_numpy(stack).to(dev), torch.from_numpy(ids.view(np.int32)).to(dev)
-    scratch = torch.empty(ops.quantized_matmul_id_workspace_bytes(p), dtype=torch.uint8, device=dev)
+    scratch = torch.full((ops.quantized_matmul_id_workspace_bytes(p),), 255, dtype=torch.uint8, device=dev)
     y, g = (torch.zeros(T * K, n, device=dev) for _ in range(2))
     ops.quantized_matmul_id_ggml(xd, sd, idd, y, p, scratch=scratch)
     ops.quantized_matmul_id_ggml(xd, sd, idd, g, p)
+    assert (scratch != 255).any(), "the grouped form did not run"
     assert torch.equal(torch.isfinite(y), torch.isfinite(g)) and torch.isnan(y).any() and torch.isinf(y).any()
     if t == HQ_Q8_0:
         assert torch.equal(torch.isnan(y), torch.isnan(g)) and torch.equal(y[torch.isinf(y)], g[torch.isinf(g)])
     for r in range(T * K):
         fin = torch.isfinite(g[r])
         assert (y[r][fin] - g[r][fin]).abs().max() <= 4e-6 * g[r][fin].abs().max() if fin.any() else True
+
+
+@pytest.mark.parametrize("t", [HQ_Q8_0, HQ_Q4_0])
+@pytest.mark.parametrize("xdt", ["bf16", "f32"])
+@pytest.mark.parametrize("E,n,k,T,K,takes", [
+    (16, 610, 704, 40, 4, ("f32", "bf16")),     # tiles of 32 routed rows, a ragged last weight-row tile
+    (6, 131, 736, 500, 3, ("f32", "bf16")),     # bf16: tiles of 128, f32: of 64; an odd number of blocks
+    (8, 1030, 160, 70, 8, ("f32", "bf16")),     # tiles of 64
+    (64, 1500, 704, 64, 2, ("f32", "bf16")),    # two rows per expert
+    (60, 1100, 704, 88, 1, ()),                 # fewer than two rows per expert and than 128 rows: GEMVs
+    (8, 1024, 96, 512, 1, ()),                  # fewer than 2^26 products: GEMVs
+    (40, 1300, 1440, 128, 1, ("f32",)),         # bf16 rows of long k: GEMVs below four rows per expert
+])
+def test_mul_mat_id_exact_form_by_size(oracle, dev, t, xdt, E, n, k, T, K, takes):
+    """Where the grouped form of exact products runs and where a GEMV per row does, although a workspace for it is there: the same
+    accuracy.  Per element: f32 sums of at most 45 block sums, 2^-24 sqrt(45) = 4e-7 of the rms as standard deviation; the Q4_0
+    GEMVs sum nibbles 0 .. 15 and take eight times the activations' sum away, partial sums of twice the size: 8e-7.  Bound 6e-6 over
+    up to half a million elements."""
+    stack, ids, xv, xd, p = _grouped_setup(oracle, dev, t, E, n, k, T, K, xdt, seed=E)
+    need = ops.quantized_matmul_id_workspace_bytes(p)
+    assert need > 0
+    scratch = torch.full((need,), 255, dtype=torch.uint8, device=dev)
+    y = torch.full((T * K, n), float("nan"), device=dev)
+    ops.quantized_matmul_id_ggml(xd, torch.from_numpy(stack).to(dev), torch.from_numpy(ids.view(np.int32)).to(dev), y, p, scratch=scratch)
+    assert bool((scratch != 255).any()) == (xdt in takes)
+    ref = oracle.qmatmul_id_f64(xv, stack, ids, T, K, n, k, E, p.expert_stride, t)
+    err = np.abs(y.cpu().numpy().astype(np.float64) - ref)
+    assert err.max() <= 6e-6 * np.sqrt(np.mean(ref * ref)), err.max()
 
 
 def test_mul_mat_id_grouped_routing_properties(oracle, dev):
