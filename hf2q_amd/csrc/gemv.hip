@@ -1149,16 +1149,19 @@ bool flat_takes_small(uint64_t n_total, uint32_t k, uint32_t cus, size_t lds) {
 template <int TYPE>
 constexpr int kFlatDepth = kIsX2<TYPE> ? 1 : TYPE == HQ_Q8_0 ? HQ_FLAT_D_Q80 : TYPE == HQ_Q4_0 ? HQ_FLAT_D_Q40 : 1;
 
+// Waves per CU of the flat walk: 16; 12 for Q6_K (measured with both activation types: f32 262144 x 2816 123 -> 117 us, 8192 x 28672
+// 43.8 -> 38.9, 4096 x 14336 14.9 -> 13.0; bf16 112 against 121 with 16) and for Q8_0 block pairs, whose windows are
+// copied through LDS (12288 x 4096 12.0 -> 11.1 us, 4096 x 14336 14.2 -> 13.1, 262144 x 2816 127.3 -> 123.1; 5120 x 17408
+// 19.6 -> 20.3); Q4_K, Q5_K and Q4_0 are faster or equal with 16
+template <int TYPE>
+constexpr int kFlatWaves = kBaseType<TYPE> == HQ_Q6_K || TYPE == HQ_Q8_0_X2 ? 12 : 16;
+
 template <int TYPE, bool X_BF16>
 int launch_flat(hipStream_t s, const void* x, const uint8_t* w0, const uint8_t* w1, float* y0, float* y1, uint32_t n, uint32_t k,
                 uint32_t nm, uint32_t cus, bool swiglu = false) {
     if constexpr (kBlock32<TYPE>)
         if (walk_doubled<TYPE, X_BF16>((uint64_t)n * nm, k)) return launch_flat<kX2 + TYPE, X_BF16>(s, x, w0, w1, y0, y1, n, k, nm, cus, swiglu);
-    // waves per CU: 16; 12 for Q6_K (measured with both activation types: f32 262144 x 2816 123 -> 117 us, 8192 x 28672
-    // 43.8 -> 38.9, 4096 x 14336 14.9 -> 13.0; bf16 112 against 121 with 16) and for Q8_0 block pairs, whose windows are
-    // copied through LDS (12288 x 4096 12.0 -> 11.1 us, 4096 x 14336 14.2 -> 13.1, 262144 x 2816 127.3 -> 123.1; 5120 x 17408
-    // 19.6 -> 20.3); Q4_K, Q5_K and Q4_0 are faster or equal with 16
-    constexpr int W = kBaseType<TYPE> == HQ_Q6_K || TYPE == HQ_Q8_0_X2 ? 12 : 16;
+    constexpr int W = kFlatWaves<TYPE>;
     using X = FlatX<TYPE, X_BF16>;
     const FArgs fa{x, w0, w1, y0, y1, n, k, nm, swiglu ? 1u : 0u, flat_geom(k, kUnitElems<TYPE>, kUnitsPerWindow<TYPE>, n, nm, cus * W),
                    kBaseType<TYPE> == HQ_Q6_K ? N4 : M4, kBaseType<TYPE> == HQ_Q5_K ? M1 : kBaseType<TYPE> == HQ_Q6_K ? N2 : M2, MAGIC};
@@ -1366,7 +1369,9 @@ bool flat_slices_take(uint32_t m, uint32_t n, uint32_t k, uint32_t cus, FlatSlic
            (uint64_t)n * (k / kUnitElems<TYPE>) < 0x7fff0000ull / 8u && flat_takes<TYPE>(n, (p.units - 1u) * kUnitElems<TYPE>, cus, 0);
 }
 
-// m activation rows over one matrix or two: as many to a pass as registers and a CU's LDS hold, in passes of even sizes.
+// m activation rows over one matrix or two: as many to a pass as registers and a CU's LDS hold, in passes of even sizes.  Windows
+// and super-tasks are those of the one-row walk (whose waves per CU they are planned for), so that a row's bits do not
+// depend on the rows beside it.
 template <int TYPE, bool X_BF16>
 int launch_flat_passes(hipStream_t s, const void* x, const uint8_t* w0, const uint8_t* w1, float* y0, float* y1, uint32_t m, uint32_t n, uint32_t k,
                        uint32_t nm, uint32_t cus, bool swiglu = false) {
@@ -1374,7 +1379,7 @@ int launch_flat_passes(hipStream_t s, const void* x, const uint8_t* w0, const ui
         if (walk_doubled<TYPE, X_BF16>((uint64_t)n * nm, k)) return launch_flat_passes<kX2 + TYPE, X_BF16>(s, x, w0, w1, y0, y1, m, n, k, nm, cus, swiglu);
     const size_t row_lds = FlatX<TYPE, X_BF16>::lds_bytes(k);
     const uint32_t most = flat_rows_per_pass<TYPE, X_BF16>(k);
-    FArgs fa{x, w0, w1, y0, y1, n, k, nm, swiglu ? 1u : 0u, flat_geom(k, kUnitElems<TYPE>, kUnitsPerWindow<TYPE>, n, nm, cus * kFlatRowsWaves<TYPE>),
+    FArgs fa{x, w0, w1, y0, y1, n, k, nm, swiglu ? 1u : 0u, flat_geom(k, kUnitElems<TYPE>, kUnitsPerWindow<TYPE>, n, nm, cus * kFlatWaves<TYPE>),
              kBaseType<TYPE> == HQ_Q6_K ? N4 : M4, kBaseType<TYPE> == HQ_Q5_K ? M1 : kBaseType<TYPE> == HQ_Q6_K ? N2 : M2, MAGIC};
     for (uint32_t r = 0, passes = (m + most - 1u) / most; r < m; --passes) {
         const uint32_t rows = (m - r + passes - 1u) / passes;

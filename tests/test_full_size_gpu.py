@@ -575,7 +575,7 @@ def test_tq_attention_full_size_over_an_encoded_cache(oracle, dev):
 
 @pytest.mark.parametrize("t", [HQ_Q4_K, HQ_Q5_K, HQ_Q6_K, HQ_Q8_0, HQ_Q4_0])
 @pytest.mark.parametrize("xdt", ["bf16", "f32"])
-@pytest.mark.parametrize("n,k", [(4101, 2816), (4099, 4096), (2049, 11264), (16390, 1024)])
+@pytest.mark.parametrize("n,k", [(4101, 2816), (4099, 4096), (2049, 11264), (16390, 1024), (18944, 3584), (8192, 2816), (4096, 14336)])
 def test_gate_and_up_of_several_rows_share_a_pass(dev, t, xdt, n, k):
     """Two to eight activation rows per pass of the flat walk (rows that straddle windows, whole windows, several windows per row,
     several rows per window; a ragged last task; k = 11264 in f32, where a CU's LDS holds three rows): the bits of a call per row."""
@@ -689,3 +689,25 @@ def test_bf16_rows_over_long_q6k_rows_keep_f32_products(oracle, dev, n, k, m):
     ref = oracle.qmatmul_f64(oracle.f32_to_bf16_bits(x.float().cpu().numpy()), _rows_of(w, rows, k, t, oracle), m, rows.size, k, t).reshape(m, -1)
     got = y[:, n // 2:n // 2 + 64].cpu().numpy().astype(np.float64)
     assert np.linalg.norm(got - ref) <= 4e-7 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("t", [HQ_Q8_0, HQ_Q4_0])
+@pytest.mark.parametrize("xdt", ["bf16", "f32"])
+@pytest.mark.parametrize("n,k", [(4101, 2848), (8200, 4128), (20000, 480)])
+def test_gate_and_up_of_several_rows_of_an_odd_number_of_blocks(oracle, dev, t, xdt, n, k):
+    """32-weight blocks that cannot be walked in pairs (89, 129 and 15 to a row): the bits of a call per row, and one row's products
+    and SwiGLU against the oracle."""
+    wg, wu = _quantized(dev, n, k, t, 25), _quantized(dev, n, k, t, 26)
+    x = torch.randn(8, k, generator=torch.Generator(device=dev).manual_seed(n), device=dev)
+    x = x.to(torch.bfloat16) if xdt == "bf16" else x
+    ref = torch.full((8, n), float("nan"), device=dev)
+    for r in range(8):
+        ops.quantized_matmul_swiglu_decode(x[r:r + 1], wg, wu, ref[r:r + 1], GgmlQuantizedMatmulParams(1, n, k, t))
+    for m in range(2, 9):
+        y = torch.full((9, n), float("nan"), device=dev)
+        ops.quantized_matmul_swiglu_decode(x[:m], wg, wu, y, GgmlQuantizedMatmulParams(m, n, k, t))
+        assert torch.equal(y[:m], ref[:m]) and torch.isnan(y[m:]).all(), m
+    rows = np.unique(np.concatenate([[0, 63, 64, n - 1], np.random.default_rng(n).integers(0, n, 40)]))
+    xin = oracle.f32_to_bf16_bits(x.float().cpu().numpy()) if xdt == "bf16" else x.cpu().numpy()
+    g, u = (oracle.qmatmul_f64(xin, _rows_of(w, rows, k, t, oracle), 8, rows.size, k, t).reshape(8, -1) for w in (wg, wu))
+    assert_matmul_close(ref[:, torch.as_tensor(rows, device=dev)].cpu().numpy(), g / (1 + np.exp(-g)) * u, f"{n}x{k} t={t} {xdt}")
