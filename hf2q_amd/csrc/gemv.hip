@@ -1396,7 +1396,9 @@ int launch_flat_passes(hipStream_t s, const void* x, const uint8_t* w0, const ui
 }
 
 // Several dense products of one type in one launch (q, k and v of a decode step, rows of a small batch): every product gets
-// a share of the workgroups in proportion to its windows and walks its matrix with them as gemv_flat_kernel does with all.
+// a share of the workgroups in proportion to its windows and walks its matrix with them as gemv_flat_kernel does with all (its
+// windows, and so the order of its sums, are planned for that share: with those of the whole device 4096 + 1024 + 1024 rows x
+// 2816 Q8_0 took 8.2 us instead of 7.8, 8192 + 1024 + 1024 Q6_K 10.2 instead of 9.2).
 // The products are about a window per wave, so what counts is that all are under way at once and that no wave walks more
 // than a window or two: one launch of 256 workgroups of 16 waves.
 // q / k / v of 4096 + 1024 + 1024 rows x 2816, Q5_K, f32 activations: 16.5 us through gemv_jobs_kernel, whose lane groups fit
@@ -1684,11 +1686,14 @@ int launch_jobs_t(hipStream_t s, const GemvArgs* jobs, uint32_t n_jobs) {
             return launch_stream<TYPE>(s, SArgs{j0.x, j0.w, j1.w, j0.y, j1.y, j0.n, j0.n + j1.n, j0.k, TYPE == HQ_Q6_K ? N4 : M4, TYPE == HQ_Q5_K ? M1 : TYPE == HQ_Q6_K ? N2 : M2, MAGIC}, cus);
     }
     {
+        // gate and up of an FFN: walked side by side as hq_qmatmul_swiglu_decode walks them, for any number of rows (its bits; us at
+        // 2 / 5 / 8 rows as products of a batch and so: 18944 x 3584 Q5_K f32 39 / 91 / 141 and 29 / 48 / 80, 4096 x 4096 Q8_0 bf16
+        // 17 / 31 / 43 and 12 / 17 / 22; Q4_0 2048 x 1024 f32 4.5 / 6.8 / 7.5 and 5.0 / 7.3 / 9.7)
         const GemvArgs &j0 = jobs[0], &j1 = jobs[1];
-        auto plain = [](const GemvArgs& j) { return j.pairs == 1 && !j.x2 && !j.ids && !j.route_logits; };
-        if (n_jobs == 2 && plain(j0) && plain(j1) && j0.x == j1.x && j0.k == j1.k && j0.n == j1.n &&
+        auto dense = [](const GemvArgs& j) { return !j.x2 && !j.ids && !j.route_logits; };
+        if (n_jobs == 2 && dense(j0) && dense(j1) && j0.pairs == j1.pairs && j0.x == j1.x && j0.k == j1.k && j0.n == j1.n &&
             flat_takes<TYPE>((uint64_t)j0.n * 2, j0.k, cus, FlatX<TYPE, X_BF16>::lds_bytes(j0.k)))
-            return launch_flat<TYPE, X_BF16>(s, j0.x, j0.w, j1.w, j0.y, j1.y, j0.n, j0.k, 2, cus);
+            return launch_flat_passes<TYPE, X_BF16>(s, j0.x, j0.w, j1.w, j0.y, j1.y, j0.pairs, j0.n, j0.k, 2, cus);
     }
     if (flat_jobs_take<TYPE, X_BF16>(jobs, n_jobs, cus)) return launch_flat_jobs<TYPE, X_BF16>(s, jobs, n_jobs, cus);
     const uint64_t per_simd = slots / (4ull * cus);

@@ -31,7 +31,8 @@ constexpr uint32_t kUnitElems = (kLaneUnit<TYPE> ? 32u : 256u) * (kIsX2<TYPE> ? 
 // Whether rows of type t are walked with doubled pieces (kX2 + t): the 32-weight block types (Q8_0 12288 x 4096: 15.9 ->
 // 12.4 us; the K-quants, whose pieces are larger and whose arithmetic is heavier, lose 7 .. 50 % to the registers a
 // doubled piece takes), rows of whole doubled units, about a window per wave of the device or more.  The same rule
-// wherever the walk is used, so that every caller gets the same sums.
+// wherever the walk goes over one matrix or two side by side, so that those callers get the same sums; a batch of other
+// products (launch_flat_jobs), whose matrices are smaller, walks single units.
 template <int TYPE, bool X_BF16>
 inline bool walk_doubled(uint64_t n_total, uint32_t k) {
     static_assert(!kIsX2<TYPE>, "asked of the base type");

@@ -189,7 +189,7 @@ HQ_API int hq_qmatmul_swiglu_ggml_ws(void* stream, const void* x, hq_act_dtype x
 /* The same on the decode route (m <= 8 activation rows): one launch, for as many rows as a CU's LDS holds, walks the same
  * weight rows of both matrices and stores silu(gate) * up -- the two f32 products never go to memory and the hq_silu_mul dispatch between them and the
  * down projection disappears (gpu_ffn.rs:1231-1306 at batch 1).  The bits of hq_qmatmul_batch_ggml(gate, up) followed by
- * hq_silu_mul.  Any type, f32 or bf16 activations, any k of whole blocks; matrices too small for the streaming GEMV
+ * hq_silu_mul, for every m.  Any type, f32 or bf16 activations, any k of whole blocks; matrices too small for the streaming GEMV
  * (hq_qmatmul_swiglu_decode_supported() == 0) return HQ_ERR_UNSUPPORTED and take the separate calls. */
 HQ_API int hq_qmatmul_swiglu_decode_supported(uint32_t n, uint32_t k, hq_ggml_type t, hq_act_dtype xdt);
 HQ_API int hq_qmatmul_swiglu_decode(void* stream, const void* x, hq_act_dtype xdt, const void* w_gate, const void* w_up, float* y,

@@ -711,3 +711,26 @@ def test_gate_and_up_of_several_rows_of_an_odd_number_of_blocks(oracle, dev, t, 
     xin = oracle.f32_to_bf16_bits(x.float().cpu().numpy()) if xdt == "bf16" else x.cpu().numpy()
     g, u = (oracle.qmatmul_f64(xin, _rows_of(w, rows, k, t, oracle), 8, rows.size, k, t).reshape(8, -1) for w in (wg, wu))
     assert_matmul_close(ref[:, torch.as_tensor(rows, device=dev)].cpu().numpy(), g / (1 + np.exp(-g)) * u, f"{n}x{k} t={t} {xdt}")
+
+
+@pytest.mark.parametrize("t", [HQ_Q4_K, HQ_Q5_K, HQ_Q6_K, HQ_Q8_0, HQ_Q4_0])
+@pytest.mark.parametrize("xdt", ["bf16", "f32"])
+@pytest.mark.parametrize("n,k", [(4101, 2816), (18944, 3584), (12288, 4096), (2048, 2048), (2049, 11264)])
+def test_gate_and_up_as_a_batch_and_with_their_swiglu_in_one_call(dev, t, xdt, n, k):
+    """hq_qmatmul_swiglu_decode has the bits of hq_qmatmul_batch_ggml(gate, up) followed by hq_silu_mul, one row to eight."""
+    wg, wu = _quantized(dev, n, k, t, 35), _quantized(dev, n, k, t, 36)
+    x = torch.randn(8, k, generator=torch.Generator(device=dev).manual_seed(n), device=dev)
+    x = x.to(torch.bfloat16) if xdt == "bf16" else x
+    for m in range(1, 9):
+        y, g, u = (torch.full((m, n), float("nan"), device=dev) for _ in range(3))
+        ops.quantized_matmul_swiglu_decode(x[:m], wg, wu, y, GgmlQuantizedMatmulParams(m, n, k, t))
+        ops.quantized_matmul_batch_ggml([ops.QmatmulJob(x[:m], wg, g, m, n, k), ops.QmatmulJob(x[:m], wu, u, m, n, k)], t)
+        want = torch.full((m, n), float("nan"), device=dev)
+        if (m * n) % 4 == 0:
+            ops.dispatch_silu_mul(g, u, want)
+        else:  # (hq_silu_mul takes whole vectors of four)
+            pad = torch.zeros(3, (m * n + 3) // 4 * 4, device=dev)
+            pad[0, :m * n], pad[1, :m * n] = g.view(-1), u.view(-1)
+            ops.dispatch_silu_mul(pad[0], pad[1], pad[2])
+            want = pad[2, :m * n].view(m, n)
+        assert torch.isfinite(y).all() and torch.equal(y, want), m
