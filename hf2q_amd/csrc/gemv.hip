@@ -1402,7 +1402,10 @@ int launch_flat_passes(hipStream_t s, const void* x, const uint8_t* w0, const ui
 // The products are about a window per wave, so what counts is that all are under way at once and that no wave walks more
 // than a window or two: one launch of 256 workgroups of 16 waves.
 // q / k / v of 4096 + 1024 + 1024 rows x 2816, Q5_K, f32 activations: 16.5 us through gemv_jobs_kernel, whose lane groups fit
-// rows of eleven super-blocks badly and whose many workgroups each stage the activations again; 7.0 us here (bf16: 8.8 -> 6.9).
+// rows of eleven super-blocks badly and whose many workgroups each stage the activations again; 7.0 us here (bf16: 8.8 -> 6.9).  In
+// that kernel / here, us at one and two rows: Q8_0 f32 12.8 / 7.6 and 15.4 / 10.8, Q4_0 bf16 8.7 / 5.6 and 13.1 / 7.5, Q6_K bf16 9.0 / 6.7 and
+// 11.4 / 9.1; x 4096: Q4_K f32 10.5 / 6.2 and 14.7 / 8.3, bf16 7.4 / 7.4 and 9.6 / 9.7, Q8_0 11.6 / 9.9 and 15.9 / 14.0.  Eight entries,
+// a row each: three rows of three products stay with that kernel.
 constexpr uint32_t MAX_FLAT_JOBS = 8;
 struct FJobs {
     FArgs j[MAX_FLAT_JOBS];
@@ -1444,6 +1447,7 @@ bool flat_jobs_take(const GemvArgs* jobs, uint32_t n_jobs, uint32_t cus) {
         const GemvArgs& j = jobs[i];
         rows += j.pairs;
         if (j.x2 || j.ids || j.route_logits || rows > MAX_FLAT_JOBS) return false;
+        if (kBlock32<TYPE> && j.k < 1024) return false;  // (three products of 512 x 512 Q4_0, f32: 3.6 us against 3.3 in gemv_jobs_kernel; at two rows 4.0 and 3.4)
         const size_t lds = X::lds_bytes(j.k);
         if (!flat_takes<TYPE>(j.n, j.k, cus, lds) && !flat_takes_small<TYPE, X_BF16>(j.n, j.k, cus, lds)) return false;
     }
