@@ -1286,7 +1286,7 @@ __global__ __launch_bounds__(64 * kFlatRowsWaves<TYPE>) void gemv_flat_slice_ker
     });
 }
 
-// Rows per pass at most: eight; six of f32 K-quant rows, whose two halves' sums of more would spill.
+// Rows per pass at most: eight; six of f32 K-quant rows, which keep the sums of two halves each.
 template <int TYPE, bool X_BF16>
 constexpr int kFlatMaxRows = X_BF16 || kBlock32<kBaseType<TYPE>> ? 8 : 6;
 template <int TYPE, bool X_BF16, int NR = kFlatMaxRows<TYPE, X_BF16>>
@@ -1349,7 +1349,8 @@ int launch_flat_slices(hipStream_t s, const float* x, const uint8_t* w, float* y
 // Whether they are: rows that the one-row kernels take too (launch_t plans those first; longer ones stay with the chunk-staged
 // kernel, which has no limit on k, or are refused at every row count), more rows than a CU's LDS holds whole, enough
 // windows in a slice, and faster.  us at 3 .. 8 rows, before /
-// here: Q6_K 4096 x 14336 30 / 26, 34 / 31, 44 / 50, 46 / 48 (5120 rows and more are ahead up to six: 12288 x 12288 103 / 71,
+// here: Q6_K 4096 x 14336 30 / 26, 34 / 31, 45 / 51, 46 / 49 (beyond a group of sixteen rows per CU the small-batch kernel takes two rounds
+// and slices are ahead up to six: 4352 x 14336 67 / 55, 70 / 55 at 5, 6, 4352 x 12288 67 / 37, 68 / 42, 12288 x 12288 103 / 71,
 // 105 / 78, 106 / 101 at 5 .. 7; 8192 x 28672 151 / 139, 155 / 154, 157 / 188); Q4_K 4096 x 12288 20 / 22, 23 / 25, 29 / 28;
 // 4096 x 14336 23 / 22, 27 / 26, 33 / 30, 32 / 46; 12288 x 12288 43 / 38, 52 / 47, 73 / 56; 8192 x 28672 91 / 65 in three slices, 92 / 92
 // in four, 95 / 109.  Where k is no multiple of 1024 the small-batch kernel does not run and the line is passes over whole rows:
@@ -1361,7 +1362,7 @@ bool flat_slices_take(uint32_t m, uint32_t n, uint32_t k, uint32_t cus, FlatSlic
     const FlatSlices p = flat_slices<TYPE>(m, k);
     *plan = p;
     const bool chunks = k % 1024u == 0;  // the small-batch kernel's
-    if (TYPE == HQ_Q6_K ? chunks && m > (n >= 20u * cus ? 6u : 4u) : (uint64_t)n * k < (7u << 23) || (chunks && (m > 5u || p.slices > 3u))) return false;
+    if (TYPE == HQ_Q6_K ? chunks && m > (n > 16u * cus ? 6u : 4u) : (uint64_t)n * k < (7u << 23) || (chunks && (m > 5u || p.slices > 3u))) return false;
     if (!gemv_row_fits(k)) return false;
     const uint32_t whole = flat_rows_per_pass<TYPE, false>(k);
     if (TYPE == HQ_Q6_K && whole >= 3u && m <= 2u * whole) return false;
