@@ -22,8 +22,8 @@
 // polled `patience` times without success stops waiting for the others and works out what it misses by itself -- the
 // logits for its own use, the activations of its token for everybody -- with the same arithmetic: duplicates have the same
 // bits.  Started workgroups therefore always finish, whatever else is resident; only workgroup 0 then stays until all have
-// started, which takes one CU from the others.  (What that costs where nobody runs out of patience: 0.3 us of 16 at one
-// token -- Q5_K + Q6_K, f32: 16.9 -> 17.2 -- and nothing that can be told from the runs' spread from two tokens on.)
+// started, which takes one CU from the others.  (What that costs where nobody runs out of patience: 0.3 .. 0.8 us of 15 .. 17
+// at one token, nothing that can be told from the runs' spread from two tokens on.)
 //
 // Row arithmetic is that of the separate dispatches — the same piece dot products, the same reduction order, the
 // same SwiGLU rounding, the same order of the weighted sum — so the block's output has the bits of
@@ -146,7 +146,7 @@ struct FusedBlock {
     float* lds_w;        // K + 1: slot K = shared gate
     float* lds_part;     // S * 64 down partials of one unit
     uint32_t* lds_gath;  // 64 * WAVES: the workgroup's SwiGLU activations
-    uint32_t* lds_late;  // 1: whether a thread ran out of patience
+    uint32_t* lds_late;  // whether a thread ran out of patience; the call's tag
     uint32_t *s_epoch, *s_err;
     uint64_t *s_lg, *s_act;
 
@@ -444,7 +444,7 @@ __device__ __forceinline__ void finish_alone(uint4* smem, uint32_t tid, uint32_t
         __syncthreads();
     }
     // Workgroup 0 leaves behind the start of all others: one that read the new call count would take it for its own.  Every
-    // workgroup has stored its logits only when all its waves had read the old one.
+    // workgroup has stored its logits only when it had read the old one.
     if (b == 0 && tid < 64u)
         for (uint32_t r = lane; r < k.n_rows; r += 64u) {
             uint32_t v;
@@ -468,8 +468,10 @@ __global__ __launch_bounds__(64 * WAVES_) void moe_fused_kernel(FusedArgs a) {
     float* const lds_lg = k.lds_lg;
     uint32_t* const lds_gath = k.lds_gath;
 
-    const uint32_t tag = ld_dev(k.s_epoch) + 1u;
-    const uint64_t tag_hi = (uint64_t)tag << 32;
+    // One wave reads the call count for the workgroup (2048 reads of that word instead of 256 take longer, and every wave would have
+    // to have its own before the logits may leave).
+    uint32_t tag0 = 0;
+    if (wv == 0) tag0 = ld_dev(k.s_epoch) + 1u;
 
     // the token's activations, requested first and staged while the logits travel
     XRaw<X_BF16> xraw;
@@ -477,15 +479,18 @@ __global__ __launch_bounds__(64 * WAVES_) void moe_fused_kernel(FusedArgs a) {
 
     // ---- phase 1: router logits and the shared-gate logit, one (row, token) per wave and turn ----
     // Workgroup b takes the rows b, b + G, ... for every token (G <= n_rows: it has at least one row), its waves the
-    // (row, token) pairs in turn.  It delivers logits of EVERY token, and none before all its waves have read the call count: once a
+    // (row, token) pairs in turn.  It delivers logits of EVERY token, and none before it has read the call count: once a
     // token's logits are complete, every workgroup has read it, and workgroup 0 may store the new one.
     const uint32_t pairs1 = (k.n_rows - b + G - 1u) / G * T;
+    uint32_t tag;
+    uint64_t tag_hi;
     {
         typename FusedBlock<TG, TD, WAVES_, X_BF16>::LogitIn in;
         if (wv < pairs1) k.fetch_logit(in, b + G * (wv / T), wv % T);
-        if (tid == 0) *k.lds_late = 0;
-        asm volatile("" : : "v"(tag));  // (the fetches are under way)
+        if (tid == 0) k.lds_late[0] = 0, k.lds_late[1] = tag0;  // (the fetches are under way)
         __syncthreads();
+        tag = (uint32_t)__builtin_amdgcn_readfirstlane((int)k.lds_late[1]);
+        tag_hi = (uint64_t)tag << 32;
         for (uint32_t q = wv; q < pairs1;) {
             const uint32_t r = b + G * (q / T), t = q % T;
             const float v = k.dot_logit(in);
@@ -505,8 +510,8 @@ __global__ __launch_bounds__(64 * WAVES_) void moe_fused_kernel(FusedArgs a) {
         lds_lg[i] = __uint_as_float(v);
     }
     __syncthreads();
-    // (looked at where something is to leave the workgroup: until then the phases run on with what there is, whatever it is)
-    uint32_t late = *k.lds_late;
+    // (lds_late is looked at where something is to leave the workgroup: until then the phases run on with what there is, whatever it
+    // is.  It is read ahead of a barrier behind which it may be set again, so all waves read the same.)
     k.route();
     uint32_t m4, m2, magic;
     asm volatile("v_mov_b32 %0, %3\n\tv_mov_b32 %1, %4\n\tv_mov_b32 %2, %5"
@@ -526,7 +531,7 @@ __global__ __launch_bounds__(64 * WAVES_) void moe_fused_kernel(FusedArgs a) {
     const uint32_t rows2_wg = jb * WAVES < P ? (P - jb * WAVES + NTW - 1u) / NTW : 0u;  // of the workgroup's first wave: the most
     const bool gather = rows2_wg <= 64u;
     auto flush = [&](uint32_t first, uint32_t count) {
-        if (lane < count && !late) st_dev(&s_act[(size_t)tok * P + tw + (first + lane) * NTW], tag_hi | keep);
+        if (lane < count && !*k.lds_late) st_dev(&s_act[(size_t)tok * P + tw + (first + lane) * NTW], tag_hi | keep);
     };
     {
         const uint32_t mine = rows2;
@@ -589,8 +594,8 @@ __global__ __launch_bounds__(64 * WAVES_) void moe_fused_kernel(FusedArgs a) {
     // from the loop's conditions), or it would make the next phase's fetches wait for each other for the sake of the
     // registers they share with these.
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    bool late = __builtin_amdgcn_readfirstlane((int)*k.lds_late) != 0;
     __syncthreads();  // the staged activations are dead from here on: their LDS holds the SwiGLU activations next
-    late = (uint32_t)__builtin_amdgcn_readfirstlane((int)late);  // the same in all waves
 
     // ---- phases 3 + 4: unit (column slice c of the token): the down rows of the slice for every slot of the token, then
     // the weighted sum over the slots in slot order, the shared expert last (the order of moe_weighted_reduce_kernel) ----
@@ -677,7 +682,6 @@ __global__ __launch_bounds__(64 * WAVES_) void moe_fused_kernel(FusedArgs a) {
                 }
             }
             __syncthreads();
-            late = *k.lds_late;
             k.sum_acts();
             __syncthreads();
             float xf[64], sx[4];
@@ -705,8 +709,8 @@ __global__ __launch_bounds__(64 * WAVES_) void moe_fused_kernel(FusedArgs a) {
             // (every fetch has been consumed: a free wait that tells the compiler so, or it would make the next unit's first
             // fetches wait for the output store below)
             __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+            late = __builtin_amdgcn_readfirstlane((int)*k.lds_late) != 0;
             __syncthreads();
-            late = (uint32_t)__builtin_amdgcn_readfirstlane((int)late);
             if (late) break;
             k.store_unit(c);
             __syncthreads();  // lds_act / lds_part are rewritten by the next unit
