@@ -262,11 +262,8 @@ def quantized_matmul_id_swiglu_ggml(input: torch.Tensor, gate_stack: torch.Tenso
         params.n_experts, params.expert_stride, params.ggml_type))
 
 
-@dataclass
-class QmatmulJob:
-    """One product of a batched launch: the arguments of quantized_matmul_id_ggml (ids set) or of
-    quantized_matmul_ggml (ids None, m <= 8).  With `input_up` the activations are
-    silu(input) * input_up, formed while they are staged."""
+@dataclass(slots=True)
+class _QmatmulJobFields:
     input: torch.Tensor
     weight: torch.Tensor
     output: torch.Tensor
@@ -283,6 +280,14 @@ class QmatmulJob:
     route_logits: torch.Tensor | None = None
     route_ids: torch.Tensor | None = None
     route_weights: torch.Tensor | None = None
+
+
+class QmatmulJob(_QmatmulJobFields):
+    """One product of a batched launch: the arguments of quantized_matmul_id_ggml (ids set) or of
+    quantized_matmul_ggml (ids None, m <= 8).  With `input_up` the activations are
+    silu(input) * input_up, formed while they are staged."""
+
+    # (the fields lie in slots of the base, 0.1 us less per job of the 0.7 it takes to build one; further attributes go beside them)
 
 
 # hq_qmatmul_job packed in one go: a third of the host time of filling a ctypes structure.
