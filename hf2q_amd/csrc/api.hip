@@ -215,10 +215,10 @@ static int check_matmul_common(const char* fn, const void* x, hq_act_dtype xdt, 
 #endif
 namespace {
 
-// Rows past the GEMV limit.  Every type has small tiles (Q4_K / Q5_K: 64 token rows, the others 128) whose one launch
-// for any m <= 128 costs about what one to two chunks of kGemvMaxRows rows through the small-batch kernel cost
-// (measured at 12288 x 4096: Q4_K 34 us against 15.5 us per chunk; Q6_K 44 against 32; Q8_0 43 against 33; Q4_0 33
-// against 30), so Q4_K / Q5_K run two chunks before the tiles take over and the other types one.  Where a type has no
+// Rows past the GEMV limit.  Every type has small tiles (64 token rows, 128, 256) whose one launch
+// for any m <= 64 costs about what one to two chunks of kGemvMaxRows rows through the small-batch kernel cost
+// (measured at 12288 x 4096: Q4_K 34 us against 15.5 us per chunk; with tiles of 128, Q6_K 44 against 32; Q8_0 43 against 33;
+// Q4_0 33 against 30), so Q4_K / Q5_K run two chunks before the tiles take over and the other types one.  Where a type has no
 // small-batch kernel for this k (K-quants with k % 1024 != 0) two rounds of per-row GEMVs run first.
 uint32_t chunked_rows_limit(uint32_t k, hq_ggml_type t) {
     if (!gemv_rows_supported(t, kGemvMaxRows, k) && !gemv_rows32_supported(t, kGemvMaxRows, k)) return 2 * kGemvMaxRows;
@@ -703,7 +703,7 @@ int hq_moe_ffn_decode(void* stream, const hq_moe_ffn_layer* l, const void* x, hq
     if (!moe_fused_supported(n_tokens, l->hidden, l->n_experts, l->top_k, l->inter, l->shared_inter, l->ggml_type, t_down, xdt))
         return fail(HQ_ERR_UNSUPPORTED,
                     "%s: takes 1..8 tokens of bf16 or f32 activations, K-quant experts (one type, or Q4_K / Q5_K gate / up with a Q6_K down), "
-                    "hidden 2048, expert and shared FFN width 512, <= 256 experts (got %u tokens, dtype %d, types %d / %d, hidden %u, "
+                    "hidden 2048, expert and shared FFN width 512, <= 256 experts, top-k within a workgroup's LDS (24 of 256 experts) (got %u tokens, dtype %d, types %d / %d, hidden %u, "
                     "inter %u / %u, %u experts, top-%u); run the block as separate dispatches",
                     fn, n_tokens, (int)xdt, (int)l->ggml_type, (int)t_down, l->hidden, l->inter, l->shared_inter, l->n_experts, l->top_k);
     if (!x || !out || !scratch || !l->router || !l->expert_gate || !l->expert_up || !l->expert_down || !l->shared_gate ||

@@ -360,7 +360,7 @@ HQ_API int hq_moe_weighted_reduce(void* stream, const float* y, const float* w, 
  * (hq_dense_gemv_bf16_pair, hq_qmatmul_batch_ggml twice with the routing and the SwiGLU folded in,
  * hq_moe_weighted_reduce).  Takes 1..8 tokens of bf16 or f32 activations, K-quant experts (Q4_K, Q5_K or Q6_K for all three
  * matrices, or Q4_K / Q5_K gate / up with a Q6_K down: layer->down_type), hidden 2048, expert and shared FFN
- * width 512, n_tokens <= n_experts <= 256, top_k <= 64; anything else is HQ_ERR_UNSUPPORTED (hq_moe_ffn_decode_scratch_bytes
+ * width 512, n_tokens <= n_experts <= 256, a top_k whose activations fit 64 KB of LDS (up to 24 of 256 experts); anything else is HQ_ERR_UNSUPPORTED (hq_moe_ffn_decode_scratch_bytes
  * returns 0 for it) and runs as the separate dispatches.
  * `scratch`: hq_moe_ffn_decode_scratch_bytes() bytes of device memory, 256-byte aligned, ZEROED ONCE before its first
  * use and then left to the library (it carries a call counter; calls that share a scratch must not overlap, and a
