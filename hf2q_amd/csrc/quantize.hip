@@ -71,62 +71,86 @@ __global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float* __restr
     }
 }
 
+// A candidate's code of a value, as a float.  FAST: v_rndne_f32 and one v_med3_f32, the same number as the magic add and
+// the integer clamp wherever |f| < 2^22; the searches below check that bound (kFastLimit, with room for the rounding of
+// the check itself) and run again in the literal form for a wave that meets anything else (infinities, NaN, a range that
+// has collapsed).
+constexpr float kFastLimit = 2097152.f;  // 2^21
+template <bool FAST, int LO, int HI>
+__device__ __forceinline__ float code_of(float f) {
+    if constexpr (FAST) return __builtin_amdgcn_fmed3f(__builtin_rintf(f), (float)LO, (float)HI);
+    return (float)max(LO, min(HI, nearest_int(f)));
+}
+
 // ------------------------------------------------------------------ Q4_K, Q5_K
 // common.rs:174-286 make_qkx2_quants with n = 32, use_mad = false and
 // nmax = 15, rmin = -1, rdelta = 0.1, nstep = 20 (Q4_K, the arguments of q4_k.rs:120-132) or
 // nmax = 31, rmin = -0.5, rdelta = 0.1, nstep = 15 (Q5_K, q5_k.rs).
-// L comes back packed four codes per word.
 // V3 = true is common.rs:294-408 make_qkx3_quants as the importance-matrix paths call it (q4_k.rs:262-274,
 // q5_k.rs:283-295): rmin = -0.9, rdelta = 0.05, nstep = 36, and the early return on max <= min.
-template <int nmax, bool V3 = false>
-__device__ float qkx2_search_32(const float (&x)[32], const float (&wt)[32], uint32_t (&Lp)[8], float& the_min) {
+//
+// Bound by VALU instructions: a candidate costs eight per element for the sums (sub, mul, rndne, med3, mul, three fma)
+// and four for the error, over codes that stay in registers as floats.  The codes themselves are not kept: the best
+// candidate is remembered by its scale and minimum (`best`), from which qkx2_codes() works them out for the rare
+// super-block that needs them.  12288 x 4096, Q4_K 498 -> 397 us, Q5_K 406 -> 316, with an importance matrix 953 -> 741 and
+// 986 -> 732 (seventeen instructions and packed codes before; keeping x - min as well, for a round of 32 subtractions less,
+// leaves room for two waves per SIMD instead of three: 408 us).
+struct Candidate {
+    float iscale, mn;
+    bool flat;  // all values alike: every code is zero
+};
+template <int nmax, bool V3, bool FAST>
+__device__ float qkx2_search_32(const float (&x)[32], const float (&wt)[32], Candidate& best, float& the_min, bool& ok) {
     constexpr int nstep = V3 ? 36 : nmax == 15 ? 20 : 15;
     constexpr float rmin = V3 ? -0.9f : nmax == 15 ? -1.f : -0.5f;
     constexpr float rdelta = V3 ? 0.05f : 0.1f;
     float mn = x[0], mx = x[0];
     float sum_w = wt[0];
     float sum_x = sum_w * x[0];
+    float mag = fabsf(x[0]);
 #pragma unroll
     for (int i = 1; i < 32; ++i) {
         if (x[i] < mn) mn = x[i];
         if (x[i] > mx) mx = x[i];
         sum_w += wt[i];
         sum_x = fmaf(wt[i], x[i], sum_x);
+        if constexpr (FAST) mag += fabsf(x[i]);
     }
+    if constexpr (FAST) ok = mag < __builtin_inff();  // (false for NaN)
+    const float x_min = mn;
     if (mn > 0.f) mn = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) Lp[i] = 0;
-    if (V3 ? (mx <= mn) : (mx == mn)) {
+    best = {0.f, 0.f, V3 ? (mx <= mn) : (mx == mn)};
+    if (best.flat) {
         the_min = -mn;
         return 0.f;
     }
     float iscale = (float)nmax / (mx - mn);
     float scale = 1.f / iscale;
     float best_error = 0.f;
+    best.iscale = iscale;
+    best.mn = mn;
 #pragma unroll
     for (int i = 0; i < 32; ++i) {
-        int l = nearest_int(iscale * (x[i] - mn));
-        l = max(0, min(nmax, l));
-        Lp[i >> 2] |= (uint32_t)l << (8 * (i & 3));
-        float diff = fmaf(scale, (float)l, mn) - x[i];
+        const float y = x[i] - mn;
+        float diff = fmaf(scale, code_of<FAST, 0, nmax>(iscale * y), mn) - x[i];
         diff = diff * diff;
         best_error = fmaf(wt[i], diff, best_error);
     }
+    // the largest |iscale * (x - mn)|, which is monotone in x
+    auto in_range = [&]() { return fabsf(iscale) * fmaxf(fabsf(x_min - mn), fabsf(mx - mn)) < kFastLimit; };
+    if constexpr (FAST) ok = ok && in_range();
     for (int is = 0; is <= nstep; ++is) {
         iscale = (rmin + rdelta * (float)is + (float)nmax) / (mx - mn);
+        if constexpr (FAST) ok = ok && in_range();
         float sum_l = 0.f, sum_l2 = 0.f, sum_xl = 0.f;
-        uint32_t La[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) La[i] = 0;
+        float lf[32];
 #pragma unroll
         for (int i = 0; i < 32; ++i) {
-            int l = nearest_int(iscale * (x[i] - mn));
-            l = max(0, min(nmax, l));
-            La[i >> 2] |= (uint32_t)l << (8 * (i & 3));
-            const float lf = (float)l, w = wt[i];
-            sum_l = fmaf(w, lf, sum_l);
-            sum_l2 = fmaf(w * lf, lf, sum_l2);
-            sum_xl = fmaf(w * lf, x[i], sum_xl);
+            lf[i] = code_of<FAST, 0, nmax>(iscale * (x[i] - mn));
+            const float wl = wt[i] * lf[i];
+            sum_l = fmaf(wt[i], lf[i], sum_l);
+            sum_l2 = fmaf(wl, lf[i], sum_l2);
+            sum_xl = fmaf(wl, x[i], sum_xl);
         }
         const float D = fmaf(sum_w, sum_l2, -sum_l * sum_l);
         if (D > 0.f) {
@@ -139,14 +163,13 @@ __device__ float qkx2_search_32(const float (&x)[32], const float (&wt)[32], uin
             float cur_error = 0.f;
 #pragma unroll
             for (int i = 0; i < 32; ++i) {
-                const float lf = (float)((La[i >> 2] >> (8 * (i & 3))) & 0xffu);
-                float diff = fmaf(this_scale, lf, this_min) - x[i];
+                float diff = fmaf(this_scale, lf[i], this_min) - x[i];
                 diff = diff * diff;
                 cur_error = fmaf(wt[i], diff, cur_error);
             }
             if (cur_error < best_error) {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) Lp[i] = La[i];
+                best.iscale = iscale;
+                best.mn = mn;
                 best_error = cur_error;
                 scale = this_scale;
                 mn = this_min;
@@ -154,6 +177,25 @@ __device__ float qkx2_search_32(const float (&x)[32], const float (&wt)[32], uin
         }
     }
     the_min = -mn;
+    return scale;
+}
+// The codes of the chosen candidate, packed four per word.
+template <int nmax>
+__device__ __forceinline__ void qkx2_codes(const float (&x)[32], const Candidate& best, uint32_t (&Lp)[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) Lp[i] = 0;
+    if (best.flat) return;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+        const int l = max(0, min(nmax, nearest_int(best.iscale * (x[i] - best.mn))));
+        Lp[i >> 2] |= (uint32_t)l << (8 * (i & 3));
+    }
+}
+template <int nmax, bool V3>
+__device__ __forceinline__ float qkx2_search(const float (&x)[32], const float (&wt)[32], Candidate& best, float& the_min) {
+    bool ok = true;
+    float scale = qkx2_search_32<nmax, V3, true>(x, wt, best, the_min, ok);
+    if (__any(!ok)) scale = qkx2_search_32<nmax, V3, false>(x, wt, best, the_min, ok);
     return scale;
 }
 
@@ -260,6 +302,7 @@ __global__ __launch_bounds__(256) void quantize_q4_k_kernel(const float* __restr
         x[4 * i + 3] = t.w;
     }
     uint32_t Lp[8];
+    Candidate best;
     float the_min, scale;
     uint32_t ls, lm, d16, dmin16;
     if constexpr (IM) {
@@ -282,25 +325,19 @@ __global__ __launch_bounds__(256) void quantize_q4_k_kernel(const float* __restr
             wt[i] = qw[i] * sqrtf(sigma2 + x[i] * x[i]);
             sumw += wt[i];
         }
-        scale = qkx2_search_32<NMAX, true>(x, wt, Lp, the_min);
+        scale = qkx2_search<NMAX, true>(x, wt, best, the_min);
         s_scale[tid] = scale;
         s_min[tid] = the_min;
         s_sw[tid] = sumw;
         __syncthreads();
-        if (j == 0) {  // the super-block's codes and d / dmin: make_qp_quants over its eight sub-blocks (q4_k.rs:277-278)
-            uint32_t Ls[8], Lm[8];
-            const float d_blk = qp_quants_8(&s_scale[lb * 8], &s_sw[lb * 8], Ls);
-            const float dmin_blk = qp_quants_8(&s_min[lb * 8], &s_sw[lb * 8], Lm);
-            for (int t = 0; t < 8; ++t) {
-                const uint32_t a = Ls[t] > 63u ? 63u : Ls[t], b = Lm[t] > 63u ? 63u : Lm[t];
-                s_code[lb * 8 + t] = a | (b << 8);
-            }
-            s_d[lb * 2] = d_blk;
-            s_d[lb * 2 + 1] = dmin_blk;
+        if (j < 2) {  // the super-block's codes and d / dmin: make_qp_quants over its eight sub-blocks (q4_k.rs:277-278)
+            uint32_t L[8];
+            s_d[lb * 2 + j] = qp_quants_8(j ? &s_min[lb * 8] : &s_scale[lb * 8], &s_sw[lb * 8], L);
+            for (int t = 0; t < 8; ++t) reinterpret_cast<uint8_t*>(&s_code[lb * 8 + t])[j] = (uint8_t)(L[t] > 63u ? 63u : L[t]);
         }
         __syncthreads();
         ls = s_code[tid] & 0xffu;
-        lm = s_code[tid] >> 8;
+        lm = s_code[tid] >> 8 & 0xffu;
         d16 = f32_to_f16_bits(s_d[lb * 2]);
         dmin16 = f32_to_f16_bits(s_d[lb * 2 + 1]);
     } else {
@@ -311,7 +348,7 @@ __global__ __launch_bounds__(256) void quantize_q4_k_kernel(const float* __restr
 #pragma unroll
         for (int i = 0; i < 32; ++i) wt[i] = av_x + fabsf(x[i]);
 
-        scale = qkx2_search_32<NMAX>(x, wt, Lp, the_min);
+        scale = qkx2_search<NMAX, false>(x, wt, best, the_min);
         s_scale[tid] = scale;
         s_min[tid] = the_min;
         __syncthreads();
@@ -347,6 +384,8 @@ __global__ __launch_bounds__(256) void quantize_q4_k_kernel(const float* __restr
             l = max(0, min(NMAX, l));
             Lp[i >> 2] |= (uint32_t)l << (8 * (i & 3));
         }
+    } else {
+        qkx2_codes<NMAX>(x, best, Lp);
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) s_L[tid * 8 + i] = Lp[i];
@@ -362,7 +401,7 @@ __global__ __launch_bounds__(256) void quantize_q4_k_kernel(const float* __restr
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             sc[t] = s_code[lb * 8 + t] & 0xffu;
-            mi[t] = s_code[lb * 8 + t] >> 8;
+            mi[t] = s_code[lb * 8 + t] >> 8 & 0xffu;
         }
         uint32_t q[12];
 #pragma unroll
@@ -450,10 +489,12 @@ __global__ __launch_bounds__(256) void quantize_q4_0_kernel(const float* __restr
 // ------------------------------------------------------------------ Q6_K
 // common.rs:61-167 make_qx_quants with rmse_type = 1: n = 16, nmax = 32 for Q6_K (q6_k.rs:58; W: the sub-block's slice
 // of the importance matrix as the weights, else x^2), n = 32, nmax = 8 with weights for Q4_0's importance-matrix path
-// (q4_0.rs:75).  Codes come back as L = l + nmax, one per byte.
-template <int N, int nmax, bool W>
-__device__ float qx_search(const float (&x)[N], const float* qw, uint32_t (&Lp)[N / 4]) {
-    float mx = 0.f, amax = 0.f;
+// (q4_0.rs:75).  Six VALU instructions per element and candidate (mul, rndne, med3, mul, two fma; w and w * x are kept);
+// the best candidate is remembered by its scale, `best_iscale` (qx_codes() makes codes of it).  Q6_K 12288 x 4096: 272 -> 203 us
+// (eleven instructions and packed codes before).
+template <int N, int nmax, bool W, bool FAST>
+__device__ float qx_search_n(const float (&x)[N], const float* qw, float& best_iscale, bool& flat, bool& ok) {
+    float mx = 0.f, amax = 0.f, mag = 0.f;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
         const float ax = fabsf(x[i]);
@@ -461,47 +502,63 @@ __device__ float qx_search(const float (&x)[N], const float* qw, uint32_t (&Lp)[
             amax = ax;
             mx = x[i];
         }
+        if constexpr (FAST) mag += ax;
     }
-#pragma unroll
-    for (int i = 0; i < N / 4; ++i) Lp[i] = 0;
-    if (amax < kGroupMaxEps) return 0.f;
-    float iscale = -(float)nmax / mx;
-    float sumlx = 0.f, suml2 = 0.f;
+    if constexpr (FAST) ok = mag < __builtin_inff();  // (false for NaN)
+    best_iscale = 0.f;
+    flat = amax < kGroupMaxEps;
+    if (flat) return 0.f;
+    float w[N], wx[N];
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-        int l = nearest_int(iscale * x[i]);
-        l = max(-nmax, min(nmax - 1, l));
-        Lp[i >> 2] |= (uint32_t)(l + nmax) << (8 * (i & 3));
-        const float w = W ? qw[i] : x[i] * x[i];
-        sumlx = fmaf(w * x[i], (float)l, sumlx);
-        suml2 = fmaf(w * (float)l, (float)l, suml2);
+        w[i] = W ? qw[i] : x[i] * x[i];
+        wx[i] = w[i] * x[i];
     }
+    auto sums = [&](float iscale, float& sumlx, float& suml2) {
+        if constexpr (FAST) ok = ok && fabsf(iscale) * amax < kFastLimit;
+        sumlx = 0.f;
+        suml2 = 0.f;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const float l = code_of<FAST, -nmax, nmax - 1>(iscale * x[i]);
+            sumlx = fmaf(wx[i], l, sumlx);
+            suml2 = fmaf(w[i] * l, l, suml2);
+        }
+    };
+    float sumlx, suml2;
+    best_iscale = -(float)nmax / mx;
+    sums(best_iscale, sumlx, suml2);
     float scale = suml2 != 0.f ? sumlx / suml2 : 0.f;
     float best = scale * sumlx;
     for (int is = -9; is <= 9; ++is) {
         if (is == 0) continue;
-        iscale = -((float)nmax + 0.1f * (float)is) / mx;
-        sumlx = 0.f;
-        suml2 = 0.f;
-        uint32_t La[N / 4];
-#pragma unroll
-        for (int i = 0; i < N / 4; ++i) La[i] = 0;
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            int l = nearest_int(iscale * x[i]);
-            l = max(-nmax, min(nmax - 1, l));
-            La[i >> 2] |= (uint32_t)(l + nmax) << (8 * (i & 3));
-            const float w = W ? qw[i] : x[i] * x[i];
-            sumlx = fmaf(w * x[i], (float)l, sumlx);
-            suml2 = fmaf(w * (float)l, (float)l, suml2);
-        }
+        const float iscale = -((float)nmax + 0.1f * (float)is) / mx;
+        sums(iscale, sumlx, suml2);
         if (suml2 > 0.f && sumlx * sumlx > best * suml2) {
-#pragma unroll
-            for (int i = 0; i < N / 4; ++i) Lp[i] = La[i];
+            best_iscale = iscale;
             scale = sumlx / suml2;
             best = scale * sumlx;
         }
     }
+    return scale;
+}
+// Codes of the chosen candidate as L = l + nmax, one per byte (all zero bytes where nothing was searched).
+template <int N, int nmax>
+__device__ __forceinline__ void qx_codes(const float (&x)[N], float iscale, bool flat, uint32_t (&Lp)[N / 4]) {
+#pragma unroll
+    for (int i = 0; i < N / 4; ++i) Lp[i] = 0;
+    if (flat) return;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int l = max(-nmax, min(nmax - 1, nearest_int(iscale * x[i])));
+        Lp[i >> 2] |= (uint32_t)(l + nmax) << (8 * (i & 3));
+    }
+}
+template <int N, int nmax, bool W>
+__device__ __forceinline__ float qx_search(const float (&x)[N], const float* qw, float& best_iscale, bool& flat) {
+    bool ok = true;
+    float scale = qx_search_n<N, nmax, W, true>(x, qw, best_iscale, flat, ok);
+    if (__any(!ok)) scale = qx_search_n<N, nmax, W, false>(x, qw, best_iscale, flat, ok);
     return scale;
 }
 
@@ -536,7 +593,10 @@ __global__ __launch_bounds__(256) void quantize_q4_0_im_kernel(const float* __re
 #pragma unroll
     for (int i = 0; i < 32; ++i) wt[i] = qw[i] * sqrtf(s2 + x[i] * x[i]);
     uint32_t Lp[8];
-    const float d = qx_search<32, 8, true>(x, wt, Lp);
+    float iscale;
+    bool flat;
+    const float d = qx_search<32, 8, true>(x, wt, iscale, flat);
+    qx_codes<32, 8>(x, iscale, flat, Lp);
     uint8_t* o = out + b * Q4_0_BYTES;
     *reinterpret_cast<uint16_t*>(o) = (uint16_t)f32_to_f16_bits(d);
     // byte j = code j | code (j + 16) << 4: words 0..3 hold codes 0..15, words 4..7 codes 16..31
@@ -574,7 +634,9 @@ __global__ __launch_bounds__(256) void quantize_q6_k_kernel(const float* __restr
         x[4 * i + 3] = t.w;
     }
     uint32_t Lp[4];
-    const float scale = qx_search<16, 32, IM>(x, IM ? imatrix + (size_t)(blk % blocks_per_row) * 256 + 16 * ib : nullptr, Lp);
+    float search_iscale;
+    bool flat;
+    const float scale = qx_search<16, 32, IM>(x, IM ? imatrix + (size_t)(blk % blocks_per_row) * 256 + 16 * ib : nullptr, search_iscale, flat);
     s_scale[tid] = scale;
     __syncthreads();
 
@@ -606,6 +668,8 @@ __global__ __launch_bounds__(256) void quantize_q6_k_kernel(const float* __restr
                 l = max(-32, min(31, l));
                 Lp[i >> 2] |= (uint32_t)(l + 32) << (8 * (i & 3));
             }
+        } else {
+            qx_codes<16, 32>(x, search_iscale, flat, Lp);
         }
     } else {
 #pragma unroll

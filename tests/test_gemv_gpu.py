@@ -286,6 +286,28 @@ def test_imatrix_quantizer_byte_equal_to_oracle(oracle, dev, t):
         assert not np.array_equal(got, ops.quantize_ggml(torch.from_numpy(x).to(dev), npr, t).cpu().numpy())
 
 
+@pytest.mark.parametrize("t", [HQ_Q4_K, HQ_Q5_K, HQ_Q6_K, HQ_Q4_0])
+@pytest.mark.parametrize("npr", [256, 768, 4352])
+def test_quantizer_byte_equal_to_oracle_at_range_edges(oracle, dev, t, npr):
+    """Where the searches leave their fast rounding (codes beyond 2^21: a range that collapses beside its minimum), at the
+    ends of f32's exponents, and rows of one block, of less than and of more than one tile of Q4_0's row sums; row counts
+    that are no whole groups of sixteen."""
+    rng = np.random.default_rng(240 + t + npr)
+    wide = rng.standard_normal((5, npr)) * 10.0 ** rng.uniform(-12, 12, (5, npr))
+    narrow = -1.0 - 1e-6 * rng.random((3, npr))
+    one = np.full((2, npr), -1.0)
+    one[:, 7::32] = np.nextafter(np.float32(-1.0), np.float32(0.0))
+    spike = rng.standard_normal((3, npr)) * 1e-3
+    spike[:, 5::64] = 3e8
+    x = np.concatenate([wide, narrow, one, spike, rng.standard_normal((4, npr)) * 1e-30, rng.standard_normal((2, npr)) * 0.02]).astype(np.float32)
+    for im in (None, (10.0 ** rng.uniform(-2, 2, npr)).astype(np.float32)):
+        want = oracle.quantize(x, npr, t, im, threads=8)
+        got = ops.quantize_ggml(torch.from_numpy(x).to(dev), npr, t, imatrix=None if im is None else torch.from_numpy(im).to(dev)).cpu().numpy()
+        bb = oracle.BLOCK_BYTES[t]
+        bad = np.nonzero((got.reshape(-1, bb) != want.reshape(-1, bb)).any(axis=1))[0]
+        assert bad.size == 0, f"{bad.size} blocks differ, first {bad[:5]}"
+
+
 def test_imatrix_quantizer_rejects_bad_arguments(dev):
     x = torch.zeros(1024, device=dev)
     with pytest.raises(ValueError):
