@@ -1212,11 +1212,15 @@ int launch_flat(hipStream_t s, const void* x, const uint8_t* w0, const uint8_t* 
 // Gate + up + SwiGLU of 17408 x 5120 Q5_K, f32: 56 / 84 / 138 / 220 us at 2 / 3 / 5 / 8 rows as a pass per row -> 38 / 47 / 64 /
 // 107; Q4_K 12288 x 4096 bf16: 23 / 34 / 56 / 88 -> 17 / 21 / 27 / 38; Q8_0 37 / 55 / 91 / 145 -> 21 / 24 / 32 / 44.  One matrix,
 // Q6_K 5120 x 6144 f32: 15 / 22 -> 10 / 12 at 2 / 3 rows.
+//
+// PAIRED (K-quants): two pieces meet every activation read from LDS (run_rows_paired), by twelve waves per CU.
+template <int TYPE, bool PAIRED = false>
+constexpr int kFlatRowsWaves = PAIRED || kBaseType<TYPE> == HQ_Q6_K || kBlock32<kBaseType<TYPE>> ? 12 : 16;
 template <int TYPE>
-constexpr int kFlatRowsWaves = kBaseType<TYPE> == HQ_Q6_K || kBlock32<kBaseType<TYPE>> ? 12 : 16;
-template <int TYPE, bool X_BF16, int NR>
-__global__ __launch_bounds__(64 * kFlatRowsWaves<TYPE>) void gemv_flat_rows_kernel(FArgs a) {
-    constexpr uint32_t W = kFlatRowsWaves<TYPE>;
+constexpr bool kFlatPairs = !kIsX2<TYPE> && !kBlock32<TYPE>;
+template <int TYPE, bool X_BF16, int NR, bool PAIRED>
+__global__ __launch_bounds__((64 * kFlatRowsWaves<TYPE, PAIRED>)) void gemv_flat_rows_kernel(FArgs a) {
+    constexpr uint32_t W = kFlatRowsWaves<TYPE, PAIRED>;
     using X = FlatX<TYPE, X_BF16>;
     extern __shared__ uint4 smem[];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
@@ -1229,10 +1233,10 @@ __global__ __launch_bounds__(64 * kFlatRowsWaves<TYPE>) void gemv_flat_rows_kern
         X::stage(static_cast<const uint8_t*>(a.x) + (size_t)r * a.k * (X_BF16 ? 2 : 4), a.k, smem + r * x_pitch, lds_s + r * s_pitch, tid, 64u * W);
     FlatWalk<TYPE, X_BF16> wk;
     wk.init(a.w0, a.w1, a.n, a.nm, a.g, wv * gridDim.x + blockIdx.x, W * gridDim.x);
-    wk.prime();
+    if constexpr (!PAIRED) wk.prime();
     __syncthreads();
     wk.load_masks(a.m4, a.m2, a.magic);
-    wk.template run_rows<NR>(smem, lds_s, x_pitch, s_pitch, [&](uint32_t cnt, const float* k0, const float* k1, uint32_t row) {
+    auto out = [&](uint32_t cnt, const float* k0, const float* k1, uint32_t row) {
         if (lane < cnt && row < a.n) {
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
@@ -1241,10 +1245,13 @@ __global__ __launch_bounds__(64 * kFlatRowsWaves<TYPE>) void gemv_flat_rows_kern
                 } else {
                     a.y0[(size_t)r * a.n + row] = k0[r];
                     if (a.nm == 2u) a.y1[(size_t)r * a.n + row] = k1[r];
+                    if (PAIRED && a.nm == 1u && row + wk.pair_rows() < a.n) a.y0[(size_t)r * a.n + row + wk.pair_rows()] = k1[r];
                 }
             }
         }
-    });
+    };
+    if constexpr (PAIRED) wk.template run_rows_paired<NR>(smem, lds_s, x_pitch, s_pitch, out);
+    else wk.template run_rows<NR>(smem, lds_s, x_pitch, s_pitch, out);
 }
 
 // The same over elements k0 .. k0 + f.k - 1 of rows of k_row f32 activations, later slices adding to y: for rows so long that a
@@ -1256,9 +1263,9 @@ struct FSliceArgs {
     FArgs f;  // k, x, w0 and the geometry: of the slice
     uint32_t k_row, add;
 };
-template <int TYPE, int NR>
-__global__ __launch_bounds__(64 * kFlatRowsWaves<TYPE>) void gemv_flat_slice_kernel(FSliceArgs s) {
-    constexpr uint32_t W = kFlatRowsWaves<TYPE>;
+template <int TYPE, int NR, bool PAIRED>
+__global__ __launch_bounds__((64 * kFlatRowsWaves<TYPE, PAIRED>)) void gemv_flat_slice_kernel(FSliceArgs s) {
+    constexpr uint32_t W = kFlatRowsWaves<TYPE, PAIRED>;
     using X = FlatX<TYPE, false>;
     extern __shared__ uint4 smem[];
     const FArgs& a = s.f;
@@ -1272,18 +1279,35 @@ __global__ __launch_bounds__(64 * kFlatRowsWaves<TYPE>) void gemv_flat_slice_ker
     FlatWalk<TYPE, false, 1, false, false, false, true> wk;
     wk.init(a.w0, a.w0, a.n, 1u, a.g, wv * gridDim.x + blockIdx.x, W * gridDim.x);
     wk.pitch_u = s.k_row / kUnitElems<TYPE>;
-    wk.prime();
+    if constexpr (!PAIRED) wk.prime();
     __syncthreads();
     wk.load_masks(a.m4, a.m2, a.magic);
-    wk.template run_rows<NR>(smem, lds_s, x_pitch, s_pitch, [&](uint32_t cnt, const float* k0, const float*, uint32_t row) {
+    auto out = [&](uint32_t cnt, const float* k0, const float* k1, uint32_t row) {
         if (lane < cnt && row < a.n) {
 #pragma unroll
             for (int r = 0; r < NR; ++r) {
                 float* y = a.y0 + (size_t)r * a.n + row;
                 *y = s.add ? *y + k0[r] : k0[r];
+                if (PAIRED && row + wk.pair_rows() < a.n) {
+                    y += wk.pair_rows();
+                    *y = s.add ? *y + k1[r] : k1[r];
+                }
             }
         }
-    });
+    };
+    if constexpr (PAIRED) wk.template run_rows_paired<NR>(smem, lds_s, x_pitch, s_pitch, out);
+    else wk.template run_rows<NR>(smem, lds_s, x_pitch, s_pitch, out);
+}
+
+// Two pieces at a time: both matrices' where there are two, else (three rows or more) where every wave has two super-tasks to
+// pair.  Gate + up at five f32 rows, Q5_K: 17408 x 5120 62 -> 48 us, 12288 x 4096 32 -> 28, 4101 x 2816 15.6 -> 12.6, at two 36 -> 32,
+// 19.5 -> 18.9, 9.4 -> 8.7; bf16 55 -> 48, 29 -> 27, 14.4 -> 12.9.  One matrix, Q6_K f32 28000 x 5120: 31 -> 32 at two rows, 47 -> 45 at five.
+// Q6_K under bf16 rows from four to six: 20 -> 23 us at two rows of 14336 x 4096, 31 -> 30 at five, and the registers of seven
+// rows and eight no longer fit (41 -> 45 at eight, 12288 x 4096).
+template <int TYPE, bool X_BF16, int NR>
+inline bool flat_paired(const FArgs& fa, uint32_t cus) {
+    if (TYPE == HQ_Q6_K && X_BF16 && (NR < 4 || NR > 6)) return false;
+    return fa.nm == 2u || (NR >= 3 && (fa.n >> fa.g.log_r) >= 2u * 12u * cus);
 }
 
 // Rows per pass at most: eight; six of f32 K-quant rows, which keep the sums of two halves each.
@@ -1293,9 +1317,15 @@ template <int TYPE, bool X_BF16, int NR = kFlatMaxRows<TYPE, X_BF16>>
 int launch_flat_rows(hipStream_t s, const FArgs& fa, uint32_t rows, size_t lds, uint32_t cus) {
     if constexpr (NR > 2)
         if (rows < (uint32_t)NR) return launch_flat_rows<TYPE, X_BF16, NR - 1>(s, fa, rows, lds, cus);
-    auto kern = gemv_flat_rows_kernel<TYPE, X_BF16, NR>;
+    auto kern = gemv_flat_rows_kernel<TYPE, X_BF16, NR, false>;
+    uint32_t waves = kFlatRowsWaves<TYPE>;
+    if constexpr (kFlatPairs<TYPE>)
+        if (flat_paired<TYPE, X_BF16, NR>(fa, cus)) {
+            kern = gemv_flat_rows_kernel<TYPE, X_BF16, NR, true>;
+            waves = kFlatRowsWaves<TYPE, true>;
+        }
     if (int rc = ensure_lds_limit(reinterpret_cast<const void*>(kern), lds, "hipFuncSetAttribute(gemv flat rows LDS)")) return rc;
-    hipLaunchKernelGGL(kern, dim3(cus), dim3(64 * kFlatRowsWaves<TYPE>), lds, s, fa);
+    hipLaunchKernelGGL(kern, dim3(cus), dim3(64 * waves), lds, s, fa);
     return check_launch("gemv flat rows kernel launch");
 }
 
@@ -1327,9 +1357,10 @@ template <int TYPE, int NR = kFlatMaxRows<TYPE, false>>
 int launch_flat_slice(hipStream_t s, const FSliceArgs& fa, uint32_t rows, size_t lds, uint32_t cus) {
     if constexpr (NR > 1)
         if (rows < (uint32_t)NR) return launch_flat_slice<TYPE, NR - 1>(s, fa, rows, lds, cus);
-    auto kern = gemv_flat_slice_kernel<TYPE, NR>;
+    const bool paired = flat_paired<TYPE, false, NR>(fa.f, cus);
+    auto kern = paired ? gemv_flat_slice_kernel<TYPE, NR, true> : gemv_flat_slice_kernel<TYPE, NR, false>;
     if (int rc = ensure_lds_limit(reinterpret_cast<const void*>(kern), lds, "hipFuncSetAttribute(gemv flat slice LDS)")) return rc;
-    hipLaunchKernelGGL(kern, dim3(cus), dim3(64 * kFlatRowsWaves<TYPE>), lds, s, fa);
+    hipLaunchKernelGGL(kern, dim3(cus), dim3(64 * (paired ? kFlatRowsWaves<TYPE, true> : kFlatRowsWaves<TYPE>)), lds, s, fa);
     return check_launch("gemv flat slice kernel launch");
 }
 template <int TYPE>

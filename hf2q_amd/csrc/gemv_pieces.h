@@ -295,13 +295,15 @@ __device__ __forceinline__ float dot_f32(const Piece<HQ_Q5_K>& p, int c, const f
 // The same dot products in two halves of 32 activations each (xh: the half's activations), for callers that cannot
 // afford all 64 in registers: half h leaves its raw sums in out[], dot_f32_finish combines both halves' sums.  The
 // operations and their order are those of dot_f32: the same bits.
-__device__ __forceinline__ void dot_f32_half(const Piece<HQ_Q4_K>& p, int, int h, const float* xh, float* out) {
+// half_word: the four weights of half h that meet activations 4 j .. 4 j + 3 of it, one per byte.
+__device__ __forceinline__ uint32_t half_word(const Piece<HQ_Q4_K>& p, int, int h, int j) {
+    const uint32_t w = j < 4 ? word(p.q0, j) : word(p.q1, j - 4);
+    return (h ? w >> 4 : w) & 0x0f0f0f0fu;
+}
+__device__ __forceinline__ void dot_f32_half(const Piece<HQ_Q4_K>& p, int c, int h, const float* xh, float* out) {
     float acc = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const uint32_t w = j < 4 ? word(p.q0, j) : word(p.q1, j - 4);
-        acc = dot4((h ? w >> 4 : w) & 0x0f0f0f0fu, xh + 4 * j, acc);
-    }
+    for (int j = 0; j < 8; ++j) acc = dot4(half_word(p, c, h, j), xh + 4 * j, acc);
     out[0] = acc;
 }
 __device__ __forceinline__ float dot_f32_finish(const Piece<HQ_Q4_K>& p, int c, const float* lo, const float* hi, const float* sx) {
@@ -312,15 +314,16 @@ __device__ __forceinline__ float dot_f32_finish(const Piece<HQ_Q4_K>& p, int c, 
     acc += d * (float)sc1 * hi[0] - dmin * (float)m1 * (sx[2] + sx[3]);
     return acc;
 }
+__device__ __forceinline__ uint32_t half_word(const Piece<HQ_Q5_K>& p, int c, int h, int j) {
+    constexpr uint32_t N4 = 0x0f0f0f0fu, N1 = 0x10101010u;
+    const uint32_t w = j < 4 ? word(p.q0, j) : word(p.q1, j - 4);
+    const uint32_t hs = (j < 4 ? word(p.h0, j) : word(p.h1, j - 4)) >> (2 * c);
+    return h ? ((w >> 4) & N4) | ((hs << 3) & N1) : (w & N4) | ((hs << 4) & N1);
+}
 __device__ __forceinline__ void dot_f32_half(const Piece<HQ_Q5_K>& p, int c, int h, const float* xh, float* out) {
     float acc = 0.f;
-    constexpr uint32_t N4 = 0x0f0f0f0fu, N1 = 0x10101010u;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const uint32_t w = j < 4 ? word(p.q0, j) : word(p.q1, j - 4);
-        const uint32_t hs = (j < 4 ? word(p.h0, j) : word(p.h1, j - 4)) >> (2 * c);
-        acc = dot4(h ? ((w >> 4) & N4) | ((hs << 3) & N1) : (w & N4) | ((hs << 4) & N1), xh + 4 * j, acc);
-    }
+    for (int j = 0; j < 8; ++j) acc = dot4(half_word(p, c, h, j), xh + 4 * j, acc);
     out[0] = acc;
 }
 __device__ __forceinline__ float dot_f32_finish(const Piece<HQ_Q5_K>& p, int c, const float* lo, const float* hi, const float* sx) {
@@ -332,19 +335,19 @@ __device__ __forceinline__ float dot_f32_finish(const Piece<HQ_Q5_K>& p, int c, 
     return acc;
 }
 // Q6_K: half 0 = the runs of the low nibbles (r0, r1), half 1 = those of the high nibbles (r2, r3).
-__device__ __forceinline__ void dot_f32_half(const Piece<HQ_Q6_K>& p, int, int h, const float* xh, float* out) {
-    float ra = 0.f, rb = 0.f;
+__device__ __forceinline__ uint32_t half_word(const Piece<HQ_Q6_K>& p, int, int h, int j) {
     constexpr uint32_t N4 = 0x0f0f0f0fu, N2 = 0x30303030u;
+    const uint32_t a = j < 4 ? word(p.qa, j) : word(p.qb, j - 4), v = word(p.qh, j & 3);
+    // low nibbles: two-bit fields 0 (qa) and 1 (qb) of qh; high nibbles: fields 2 and 3
+    const uint32_t two = h == 0 ? (j < 4 ? v << 4 : v << 2) : j < 4 ? v : v >> 2;
+    return ((h ? a >> 4 : a) & N4) | (two & N2);
+}
+__device__ __forceinline__ void dot_f32_half(const Piece<HQ_Q6_K>& p, int c, int h, const float* xh, float* out) {
+    float ra = 0.f, rb = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const uint32_t a = word(p.qa, j), b = word(p.qb, j), v = word(p.qh, j);
-        if (h == 0) {
-            ra = dot4((a & N4) | ((v << 4) & N2), xh + 4 * j, ra);
-            rb = dot4((b & N4) | ((v << 2) & N2), xh + 16 + 4 * j, rb);
-        } else {
-            ra = dot4(((a >> 4) & N4) | (v & N2), xh + 4 * j, ra);
-            rb = dot4(((b >> 4) & N4) | ((v >> 2) & N2), xh + 16 + 4 * j, rb);
-        }
+        ra = dot4(half_word(p, c, h, j), xh + 4 * j, ra);
+        rb = dot4(half_word(p, c, h, j + 4), xh + 16 + 4 * j, rb);
     }
     out[0] = ra;
     out[1] = rb;

@@ -192,6 +192,21 @@ struct FlatX1 {
         }
     }
 
+    // f32 K-quant pieces: chunk j (activations 4 j .. 4 j + 3) of half h of the lane's 64 lies at half_base() + half_chunk(h, j).
+    static __device__ __forceinline__ const uint4* half_base(const uint4* lds_x, uint32_t ur, int c) {
+        static_assert(!PAIR && !kBlock32<TYPE>, "f32 activations of a K-quant");
+        if constexpr (TYPE == HQ_Q6_K) return lds_x + ur * 81u + (uint32_t)(c >> 1) * 40u + (uint32_t)(c & 1) * 4u;
+        return lds_x + (ur * 4u + (uint32_t)c) * (G + 1u);
+    }
+    static constexpr __device__ __forceinline__ int half_chunk(int h, int j) {
+        return TYPE == HQ_Q6_K ? 16 * h + 8 * (j >> 2) + (j & 3) : 8 * h + j;
+    }
+    static __device__ __forceinline__ void load_sums(const float* lds_s, uint32_t ur, int c, float* sx) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            sx[r] = TYPE == HQ_Q6_K ? lds_s[ur * 16u + (uint32_t)(c >> 1) * 8u + (uint32_t)(c & 1) + 2u * r] : lds_s[(ur * 4u + (uint32_t)c) * 4u + r];
+    }
+
     // f32 K-quant pieces in two halves of 32 activations (see dot_f32_half); h = 0 also loads the four run sums.
     static __device__ __forceinline__ void load_half(const uint4* lds_x, const float* lds_s, uint32_t ur, int c, int h, uint32_t* xh,
                                                      float* sx) {
@@ -628,6 +643,133 @@ struct FlatWalk {
                     }
                     ++q_cur;
                 }
+            }
+        }
+        if (done & 63u) out(done & 63u, keep0, keep1, keep_row);
+    }
+
+    // run_rows over two pieces at a time that meet the same activations: the same window of both matrices (nm == 2), or of two
+    // super-tasks one after the other in the wave's sequence (nm == 1), so that an activation read from LDS serves twice the
+    // weights.  K-quants.  The operations and their order per row are those of run_rows: the same bits.  out's keep1: the second
+    // matrix's sums, or those of the rows pair_rows() further on (past the matrix's end where the sequence has none left).
+    __device__ __forceinline__ uint32_t pair_rows() const { return nm == 2u ? 0u : seq_stride << g.log_r; }
+    __device__ __forceinline__ void fetch_pair(Piece<TYPE>& pa, Piece<TYPE>& pb) {
+        const uint32_t sid = seq_first + f_q * seq_stride;
+        const uint32_t wu = g.uwe * f_w + lv, su = g.bu << g.log_r, last = nrows * g.bu - 1u;
+        const uint32_t first = (sid << g.log_r) * g.bu + (wu < su ? wu : su - 1u), second = first + pair_rows() * g.bu;
+        uint32_t ua = first < last ? first : last, ub = second < last ? second : last;
+        if constexpr (SLICE) {
+            ua += __umulhi(ua, g.magic) * (pitch_u - g.bu);
+            ub += __umulhi(ub, g.magic) * (pitch_u - g.bu);
+        }
+        pa.load(w0 + (size_t)ua * BB, c);
+        pb.load((nm == 2u ? w1 : w0) + (size_t)ub * BB, c);
+        if (f_w + 1u < g.st) {
+            ++f_w;
+        } else if (f_q + 3u - nm < count) {  // (past the end: the last task again, not used)
+            f_w = 0;
+            f_q += 3u - nm;
+        }
+    }
+    template <int NR, typename OUT>
+    __device__ __forceinline__ void run_rows_paired(const uint4* lds_x, const float* lds_s, uint32_t x_pitch, uint32_t s_pitch, OUT&& out) {
+        static_assert(D == 1 && !DYN && !COPY && !kLaneUnit<TYPE> && !kIsX2<TYPE>, "the plain walk of a K-quant");
+        uint32_t c_w = 0, done = 0, keep_row = 0;
+        float keep0[NR] = {}, keep1[NR] = {}, acc0[NR] = {}, acc1[NR] = {};
+        const int last_lane = (int)(g.uwe * LPU - 1u);
+        const bool one_row = g.log_r == 0u;
+        Piece<TYPE> pa, pb;
+        if (q_cur < count) fetch_pair(pa, pb);
+        while (q_cur < count) {
+            const uint32_t lu_raw = g.uwe * c_w + lv, su = g.bu << g.log_r;
+            const bool in_task = lu_raw < su;
+            const uint32_t lu = in_task ? lu_raw : su - 1u;
+            uint32_t lrow = __umulhi(lu, g.magic);
+            const uint32_t ur = lu - lrow * g.bu;
+            float part0[NR], part1[NR];
+            if constexpr (X::PAIR) {
+#pragma unroll
+                for (int r = 0; r < NR; ++r) {
+                    uint32_t xr[X::XW];
+                    float sx[4];
+                    X::load(lds_x + r * x_pitch, lds_s + r * s_pitch, ur, c, xr, sx);
+                    part0[r] = dot_pair(pa, c, xr, sx, m4, m2, magic);
+                    part1[r] = dot_pair(pb, c, xr, sx, m4, m2, magic);
+                    asm volatile("" : "+v"(part0[r]), "+v"(part1[r]));
+                }
+            } else {
+                // sums of the two halves (Q6_K: of two runs in each), in the order of dot_f32_half
+                constexpr int CH = TYPE == HQ_Q6_K ? 2 : 1;
+                float s0[2][NR][CH] = {}, s1[2][NR][CH] = {};
+                const uint4* base = X::half_base(lds_x, ur, c);
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        uint32_t wa = half_word(pa, c, h, j), wb = half_word(pb, c, h, j);
+                        asm("" : "+v"(wa), "+v"(wb));  // (see dot4)
+                        const float a[4] = {ubyte0(wa), ubyte1(wa), ubyte2(wa), ubyte3(wa)}, b[4] = {ubyte0(wb), ubyte1(wb), ubyte2(wb), ubyte3(wb)};
+                        const int ch = CH == 2 ? j >> 2 : 0;
+#pragma unroll
+                        for (int r = 0; r < NR; ++r) {
+                            const float4 x = *reinterpret_cast<const float4*>(base + r * x_pitch + X::half_chunk(h, j));
+                            s0[h][r][ch] = fmaf(a[3], x.w, fmaf(a[2], x.z, fmaf(a[1], x.y, fmaf(a[0], x.x, s0[h][r][ch]))));
+                            s1[h][r][ch] = fmaf(b[3], x.w, fmaf(b[2], x.z, fmaf(b[1], x.y, fmaf(b[0], x.x, s1[h][r][ch]))));
+                        }
+                    }
+#pragma unroll
+                for (int r = 0; r < NR; ++r) {
+                    float sx[4];
+                    X::load_sums(lds_s + r * s_pitch, ur, c, sx);
+                    part0[r] = dot_f32_finish(pa, c, s0[0][r], s0[1][r], sx);
+                    part1[r] = dot_f32_finish(pb, c, s1[0][r], s1[1][r], sx);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < NR; ++r) asm volatile("" : "+v"(part0[r]), "+v"(part1[r]));  // the refill follows the arithmetic that frees its registers
+            fetch_pair(pa, pb);
+            const uint32_t row0 = (seq_first + q_cur * seq_stride) << g.log_r;
+            if (one_row) {
+#pragma unroll
+                for (int r = 0; r < NR; ++r) {
+                    acc0[r] += active && in_task ? part0[r] : 0.f;
+                    acc1[r] += active && in_task ? part1[r] : 0.f;
+                }
+                if (c_w + 1u == g.st) {
+                    const bool mine = lane == (done & 63u);
+#pragma unroll
+                    for (int r = 0; r < NR; ++r) {
+                        const float v0 = group_sum(acc0[r], 6), v1 = group_sum(acc1[r], 6);
+                        acc0[r] = acc1[r] = 0.f;
+                        keep0[r] = mine ? v0 : keep0[r];
+                        keep1[r] = mine ? v1 : keep1[r];
+                    }
+                    keep_row = mine ? row0 : keep_row;
+                }
+            } else {
+                const uint32_t r_lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)lrow);
+                const uint32_t r_hi = (uint32_t)__builtin_amdgcn_readlane((int)lrow, last_lane);
+                lrow = active && in_task ? lrow : 0xffffffffu;
+                for (uint32_t q = r_lo; q <= r_hi; ++q) {
+                    const bool mine = lane == ((done + q) & 63u);
+#pragma unroll
+                    for (int r = 0; r < NR; ++r) {
+                        const float v0 = group_sum(lrow == q ? part0[r] : 0.f, 6), v1 = group_sum(lrow == q ? part1[r] : 0.f, 6);
+                        keep0[r] = mine ? keep0[r] + v0 : keep0[r];
+                        keep1[r] = mine ? keep1[r] + v1 : keep1[r];
+                    }
+                    keep_row = mine ? row0 + q : keep_row;
+                }
+            }
+            if (++c_w == g.st) {
+                c_w = 0;
+                done += 1u << g.log_r;
+                if ((done & 63u) == 0u) {
+                    out(64u, keep0, keep1, keep_row);
+#pragma unroll
+                    for (int r = 0; r < NR; ++r) keep0[r] = keep1[r] = 0.f;
+                }
+                q_cur += 3u - nm;
             }
         }
         if (done & 63u) out(done & 63u, keep0, keep1, keep_row);
