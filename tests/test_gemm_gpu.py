@@ -75,6 +75,14 @@ def test_small_tiles_and_k_slices_match_f64_oracle(oracle, dev, t, m, n, k):
     assert np.array_equal(y, y2)
 
 
+@pytest.mark.parametrize("t,k", [(HQ_Q6_K, 256), (HQ_Q6_K, 768), (HQ_Q8_0, 128), (HQ_Q8_0, 384), (HQ_Q4_0, 128), (HQ_Q4_0, 384)])
+@pytest.mark.parametrize("m,n", [(70, 1), (70, 33), (70, 127), (40, 31), (300, 65)])
+def test_tile_weight_rows_that_end_inside_a_wave(oracle, dev, t, k, m, n):
+    """The 2-byte aligned types fetch 32 weight rows per wave together: matrices that end inside a wave's rows, one run of k."""
+    y, ref = _run(oracle, dev, t, "bf16", m, n, k)
+    assert_matmul_close_f16_tile(y, ref, f"weight rows t={t} {m}x{n}x{k}")
+
+
 @pytest.mark.parametrize("t", [HQ_Q4_K, HQ_Q8_0, HQ_Q6_K, HQ_Q5_K, HQ_Q4_0])
 def test_gemm_adversarial_blocks(oracle, dev, t):
     """Every scale / min / nibble bit pattern (raw random bytes with finite f16 fields)."""
