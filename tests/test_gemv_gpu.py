@@ -503,6 +503,26 @@ def test_mul_mat_id_swiglu_grouped(oracle, dev, t, xdt, E, n, k, T, K):
     assert np.sqrt(np.mean((got - ref) ** 2)) <= 1.5e-3 * np.sqrt(np.mean(ref * ref))
 
 
+@pytest.mark.parametrize("t", [HQ_Q4_K, HQ_Q5_K])
+@pytest.mark.parametrize("rows", [(95, 96, 97, 1, 33), (193, 0, 64, 32, 3)])
+def test_mul_mat_id_swiglu_grouped_at_tile_edges(oracle, dev, t, rows):
+    """Experts whose rows end at, before and behind tiles of 96: the bits of two grouped calls followed by silu_mul."""
+    E, n, k, T = len(rows), 136, 512, sum(rows)
+    gate, _, _, xd, p = _grouped_setup(oracle, dev, t, E, n, k, T, 1, "f32", seed=3)
+    up, _, _, _, _ = _grouped_setup(oracle, dev, t, E, n, k, T, 1, "f32", seed=4)
+    ids = np.random.default_rng(5).permutation(np.repeat(np.arange(E, dtype=np.int32), rows))
+    gd, ud, idd = torch.from_numpy(gate).to(dev), torch.from_numpy(up).to(dev), torch.from_numpy(ids).to(dev)
+    scratch = torch.empty(ops.quantized_matmul_id_swiglu_workspace_bytes(p), dtype=torch.uint8, device=dev)
+    yg, yu = torch.empty(T, n, device=dev), torch.empty(T, n, device=dev)
+    ops.quantized_matmul_id_ggml(xd, gd, idd, yg, p, scratch=scratch)
+    ops.quantized_matmul_id_ggml(xd, ud, idd, yu, p, scratch=scratch)
+    sep = torch.empty_like(yg)
+    ops.dispatch_silu_mul(yg, yu, sep)
+    y = torch.full((T, n), float("nan"), device=dev)
+    ops.quantized_matmul_id_swiglu_ggml(xd, gd, ud, idd, y, p, scratch)
+    assert torch.equal(y, sep)
+
+
 def test_mul_mat_id_swiglu_has_no_form_for_other_types_and_small_calls(dev):
     p = GgmlQuantizedMatmulIdParams(64, 4, 128, 512, 8, 128 * ops.ggml_row_bytes(HQ_Q6_K, 512), HQ_Q6_K)
     assert ops.quantized_matmul_id_workspace_bytes(p) > 0 and ops.quantized_matmul_id_swiglu_workspace_bytes(p) == 0
