@@ -1060,3 +1060,27 @@ int hq_moe_weighted_reduce(void* stream, const float* y, const float* w, const f
 }
 
 }  // extern "C"
+
+namespace hq {
+
+bool grouped_shared_supported(uint32_t n_tokens, uint32_t top_k, uint32_t n, uint32_t k, uint32_t n_experts, uint64_t expert_stride,
+                              hq_ggml_type t, bool swiglu) {
+    return grouped_route(n_tokens, top_k, n, k, n_experts, expert_stride, t) && !gemm_f16_grouped_exact(t, k) &&
+           (!swiglu || gemm_f16_grouped_swiglu_supported(t));
+}
+
+int grouped_with_shared(const char* fn, void* stream, const void* x, hq_act_dtype xdt, const void* w_stack, const void* w_stack2,
+                        const float* scales, const float* scales2, const uint32_t* ids, float* y, void* workspace, uint32_t n_tokens,
+                        uint32_t top_k, uint32_t n, uint32_t k, uint32_t n_experts, uint64_t expert_stride, hq_ggml_type t, const SharedExpert& sh) {
+    for (const void* w : {w_stack, sh.w})
+        if (int rc = check_matmul_common(fn, x, xdt, w, y, n, k, t)) return rc;
+    if (w_stack2)
+        for (const void* w : {w_stack2, sh.w2})
+            if (int rc = check_matmul_common(fn, x, xdt, w, y, n, k, t)) return rc;
+    for (const float* sc : {scales, scales2, sh.w_scales, sh.w_scales2})
+        if (!is_aligned(sc, 4)) return fail(HQ_ERR_INVALID_ARGUMENT, "%s: row scales must be 4-byte aligned", fn);
+    return launch_gemm_f16_grouped((hipStream_t)stream, x, xdt, w_stack, ids, y, workspace, n_tokens, top_k, n, k, n_experts, expert_stride, t,
+                                   scales, w_stack2, scales2, &sh);
+}
+
+}  // namespace hq

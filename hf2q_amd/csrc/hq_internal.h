@@ -133,10 +133,25 @@ size_t gemm_f16_grouped_workspace_bytes(uint32_t n_tokens, uint32_t top_k, uint3
 // w_stack2 (Q4_K / Q5_K, see gemm_f16_grouped_swiglu_supported): y = silu(W[ids] . x) * (W2[ids] . x), the gate and up
 // projections of a MoE block and their SwiGLU as one grouped product; workspace for stacks = 2.
 bool gemm_f16_grouped_swiglu_supported(hq_ggml_type t);
+// One more expert of the same shape that every token goes to (a MoE layer's shared expert), multiplied by the same launch: its
+// `rows` output rows follow the routed ones in y.  Its activations are the tokens', or (own_rows) `rows` more rows of x behind the
+// routed ones.  The row scales, of the stacks as well, are the caller's; not for exact products.
+struct SharedExpert {
+    const void *w, *w2;
+    const float *w_scales, *w_scales2;
+    uint32_t rows, own_rows;
+};
+// (api.hip: with the argument checks of the public calls that it stands for)
+bool grouped_shared_supported(uint32_t n_tokens, uint32_t top_k, uint32_t n, uint32_t k, uint32_t n_experts, uint64_t expert_stride,
+                              hq_ggml_type t, bool swiglu);
+int grouped_with_shared(const char* fn, void* stream, const void* x, hq_act_dtype xdt, const void* w_stack, const void* w_stack2,
+                        const float* scales, const float* scales2, const uint32_t* ids, float* y, void* workspace, uint32_t n_tokens,
+                        uint32_t top_k, uint32_t n, uint32_t k, uint32_t n_experts, uint64_t expert_stride, hq_ggml_type t, const SharedExpert& sh);
+size_t gemm_f16_grouped_shared_workspace_bytes(uint32_t x_rows, uint32_t pairs, uint32_t shared, uint32_t n_experts, uint32_t k);
 int launch_gemm_f16_grouped(hipStream_t s, const void* x, hq_act_dtype xdt, const void* w_stack, const uint32_t* ids, float* y,
                             void* workspace, uint32_t n_tokens, uint32_t top_k, uint32_t n, uint32_t k, uint32_t n_experts,
                             uint64_t expert_stride, hq_ggml_type t, const float* w_scales = nullptr,
-                            const void* w_stack2 = nullptr, const float* w_scales2 = nullptr);
+                            const void* w_stack2 = nullptr, const float* w_scales2 = nullptr, const SharedExpert* sh = nullptr);
 
 // MoE glue (moe.hip)
 int launch_dense_gemv_bf16(hipStream_t s, const void* x, hq_act_dtype xdt, const void* w, float* y, uint32_t m,
