@@ -124,41 +124,79 @@ __global__ __launch_bounds__(256) void moe_weighted_reduce_kernel(const float* _
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 
-// The same product for many activation rows (the router of a prefill chunk: 2048 tokens x 256 experts), bf16
-// activations: both operands go from memory straight into the matrix cores.  One workgroup per tile of 32 token rows x
-// 64 weight rows, its four waves a quarter of k each; a wave reads one activation fragment and two weight fragments per
-// k-step (eight k-steps of loads in flight) for two MFMAs -- the loads are row-strided, a cache line per lane, and their
-// line look-ups are what bounds the kernel, so fewer of them per MFMA is what counts.  The partial tiles are added in
+// The same product for many activation rows (the router of a prefill chunk: 2048 tokens x 256 experts) on the matrix cores.
+// One workgroup per tile of 32 token rows x 32 weight rows, its four waves a quarter of k each; the partial tiles are added in
 // wave order through LDS.  The bf16 products are exact and the sums f32.  The weights are the MFMA's first operand, so
-// a lane ends up with sixteen outputs of ONE token (lane % 32) per weight tile, four runs of four consecutive n.  Rows
+// a lane ends up with sixteen outputs of ONE token (lane % 32), four runs of four consecutive n.  Rows
 // past m or n repeat the last one and are not stored.  k % 16 == 0.
 // f32 activations are split into three bf16 terms each (truncations of x, of x - hi and of the rest: every step exact, 24
-// significant bits in all), so an activation fragment costs three MFMAs per weight tile and the products stay exact.
+// significant bits in all), so an activation fragment costs three MFMAs and the products stay exact.
+//
+// Four k-steps (64 values of every row) at a time a wave fetches both operands as 16-byte pieces, consecutive lanes consecutive
+// pieces of a row, and passes them on through LDS of its own while the next ones are in flight.  Bound by the chain of conversions
+// and products of one wave: tiles of 64 weight rows, a wave per SIMD, took 25 us over f32 rows at 1999 tokens x 256 x 2048 and 20
+// at 59 (26 and 23 with fragments straight from memory, a row per lane); these 21 and 12.  Three batches in flight: no gain.
 template <bool X_BF16>
 __global__ __launch_bounds__(256) void dense_gemm_bf16_kernel(const void* __restrict__ xv, const uint16_t* __restrict__ w,
                                                               float* __restrict__ y, uint32_t m, uint32_t n, uint32_t k) {
-    __shared__ float part[3][2][16][64];
-    const uint32_t lane = threadIdx.x & 63u, l32 = lane & 31u, lg = lane >> 5, wave = threadIdx.x >> 6;
-    const uint32_t tiles_n = (n + 63u) / 64u;
-    const uint32_t m0 = (blockIdx.x / tiles_n) * 32u, n0 = (blockIdx.x % tiles_n) * 64u;
-    const uint32_t xr = m0 + l32 < m ? m0 + l32 : m - 1u;
-    // this lane's k-group of eight values: one uint4 of bf16, or two of f32
-    const uint4* xp = X_BF16 ? reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(xv) + (size_t)xr * k) + lg
-                             : reinterpret_cast<const uint4*>(static_cast<const float*>(xv) + (size_t)xr * k) + 2u * lg;
-    // k-step st of the activations: 1 (bf16) or 3 (f32) fragments
+    // A wave's share: 32 rows of x, then 32 of w; rows are padded by 16 bytes, so that the sixteen rows that sixteen lanes read lie in
+    // different 16-byte slots of 256 bytes.  The partial tiles of waves 1 .. 3 lie over the shares after the products.
+    constexpr uint32_t ST = 4, XB = X_BF16 ? 2 : 4;                                     // k-steps at a time; bytes per activation
+    constexpr uint32_t XP = ST * 16 * XB + 16, WP = ST * 16 * 2 + 16, SHARE = 32 * XP + 32 * WP;
+    constexpr uint32_t XL = ST * XB, WL = ST * 2;                                       // pieces per row and batch
+    constexpr int XN = 32 * XL / 64, WN = 32 * WL / 64;                                 // fetches per lane and batch
+    static_assert(3 * 16 * 64 * 4 <= 4 * SHARE, "the partial tiles fit the shares");
+    __shared__ __attribute__((aligned(16))) uint8_t smem[4 * SHARE];
+    const uint32_t lane = threadIdx.x & 63u, l32 = lane & 31u, lg = lane >> 5;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t tiles_n = (n + 31u) / 32u;
+    // (workgroup b runs on XCD b % 8: the tiles of the same token rows are on one XCD, whose L2 they share)
+    const uint32_t slot = blockIdx.x >> 3, m0 = ((slot / tiles_n) * 8u + (blockIdx.x & 7u)) * 32u, n0 = (slot % tiles_n) * 32u;
+    if (m0 >= m) return;
+    uint8_t *lx = smem + wave * SHARE, *lw = lx + 32 * XP;
+    const uint32_t steps = k / 16u, per = (steps + 3u) / 4u;
+    const uint32_t first = wave * per, end = first + per < steps ? first + per : steps;
+
+    typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
+    u32x4_t px[XN], pw[WN];
+    // (pieces of k-steps past the wave's last one: the last one's again, not used)
+    auto fetch = [&](uint32_t st) {
+        const uint32_t left = end - st;  // >= 1
+        const uint32_t xc = lane % XL, wc = lane % WL, xs = XL / ST, wsn = WL / ST;  // pieces per k-step
+        const uint32_t xq = xc / xs < left ? xc : xc % xs + (left - 1u) * xs, wq = wc / wsn < left ? wc : wc % wsn + (left - 1u) * wsn;
+#pragma unroll
+        for (uint32_t i = 0; i < (uint32_t)XN; ++i) {
+            const uint32_t r = m0 + i * (64u / XL) + lane / XL;
+            px[i] = *reinterpret_cast<const u32x4_t*>(static_cast<const uint8_t*>(xv) + ((size_t)(r < m ? r : m - 1u) * k + 16u * st) * XB + 16u * xq);
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < (uint32_t)WN; ++i) {
+            const uint32_t r = n0 + i * (64u / WL) + lane / WL;
+            pw[i] = *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint8_t*>(w) + ((size_t)(r < n ? r : n - 1u) * k + 16u * st) * 2 + 16u * wq);
+        }
+    };
+    auto store = [&] {  // (one wave's LDS instructions are served in order)
+#pragma unroll
+        for (uint32_t i = 0; i < (uint32_t)XN; ++i) *reinterpret_cast<u32x4_t*>(lx + (i * (64u / XL) + lane / XL) * XP + 16u * (lane % XL)) = px[i];
+#pragma unroll
+        for (uint32_t i = 0; i < (uint32_t)WN; ++i) *reinterpret_cast<u32x4_t*>(lw + (i * (64u / WL) + lane / WL) * WP + 16u * (lane % WL)) = pw[i];
+        asm volatile("" ::: "memory");
+    };
+    // k-step u of the batch, this lane's k-group of eight values: 1 (bf16) or 3 (f32) fragments
     constexpr int XT = X_BF16 ? 1 : 3;
-    auto x_frags = [&](uint32_t st, bf16x8_t* f) {
+    auto x_frags = [&](uint32_t u, bf16x8_t* f) {
+        const uint4* p = reinterpret_cast<const uint4*>(lx + l32 * XP + u * (16u * XB) + lg * (8u * XB));
         if constexpr (X_BF16) {
-            f[0] = __builtin_bit_cast(bf16x8_t, xp[2u * st]);
+            f[0] = __builtin_bit_cast(bf16x8_t, p[0]);
         } else {
-            const uint4 v0 = xp[4u * st], v1 = xp[4u * st + 1u];
-            const uint32_t u[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+            const uint4 v0 = p[0], v1 = p[1];
+            const uint32_t v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
             uint32_t t[3][8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const uint32_t hi = u[i] & 0xffff0000u;
+                const uint32_t hi = v[i] & 0xffff0000u;
                 // (inf / nan stay in the first term alone: inf - inf would turn an infinite product into nan)
-                const float r1 = (hi & 0x7f800000u) == 0x7f800000u ? 0.f : __uint_as_float(u[i]) - __uint_as_float(hi);
+                const float r1 = (hi & 0x7f800000u) == 0x7f800000u ? 0.f : __uint_as_float(v[i]) - __uint_as_float(hi);
                 const uint32_t mid = __float_as_uint(r1) & 0xffff0000u;
                 const float r2 = r1 - __uint_as_float(mid);
                 t[0][i] = hi, t[1][i] = mid, t[2][i] = __float_as_uint(r2) & 0xffff0000u;
@@ -169,62 +207,41 @@ __global__ __launch_bounds__(256) void dense_gemm_bf16_kernel(const void* __rest
                                                                (t[j][4] >> 16) | t[j][5], (t[j][6] >> 16) | t[j][7]));
         }
     };
-    const uint4* wp[2];
+    f32x16_t acc;
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const uint32_t wr = n0 + 32u * t + l32 < n ? n0 + 32u * t + l32 : n - 1u;
-        wp[t] = reinterpret_cast<const uint4*>(w + (size_t)wr * k) + lg;
-    }
-    f32x16_t acc[2];
+    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+    if (first < end) fetch(first);
+    for (uint32_t st = first; st < end; st += ST) {
+        store();
+        if (st + ST < end) fetch(st + ST);
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+        for (uint32_t u = 0; u < ST; ++u) {
+            if (st + u < end) {  // uniform
+                bf16x8_t b[XT];
+                x_frags(u, b);
+                const bf16x8_t wf = *reinterpret_cast<const bf16x8_t*>(lw + l32 * WP + 32u * u + 16u * lg);
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[t][v] = 0.f;
-    const uint32_t steps = k / 16u, per = (steps + 3u) / 4u;
-    uint32_t st = wave * per;
-    const uint32_t end = st + per < steps ? st + per : steps;
-    constexpr uint32_t UN = X_BF16 ? 8u : 4u;  // k-steps of loads in flight
-    for (; st + UN <= end; st += UN) {
-        uint4 a0[UN], a1[UN];
-        bf16x8_t b[UN][XT];
-#pragma unroll
-        for (uint32_t u = 0; u < UN; ++u) a0[u] = wp[0][2u * (st + u)], a1[u] = wp[1][2u * (st + u)], x_frags(st + u, b[u]);
-#pragma unroll
-        for (uint32_t u = 0; u < UN; ++u)
-#pragma unroll
-            for (int j = XT - 1; j >= 0; --j) {  // the smallest term first
-                acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a0[u]), b[u][j], acc[0], 0, 0, 0);
-                acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a1[u]), b[u][j], acc[1], 0, 0, 0);
+                for (int j = XT - 1; j >= 0; --j) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, b[j], acc, 0, 0, 0);  // the smallest term first
             }
-    }
-    for (; st < end; ++st) {
-        bf16x8_t b[XT];
-        x_frags(st, b);
-#pragma unroll
-        for (int j = XT - 1; j >= 0; --j) {
-            acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, wp[0][2u * st]), b[j], acc[0], 0, 0, 0);
-            acc[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, wp[1][2u * st]), b[j], acc[1], 0, 0, 0);
         }
+        asm volatile("" ::: "memory");
     }
+    __syncthreads();  // every wave is done with its share
+    auto part = reinterpret_cast<float (*)[16][64]>(smem);
     if (wave) {
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) part[wave - 1][t][v][lane] = acc[t][v];
+        for (int v = 0; v < 16; ++v) part[wave - 1][v][lane] = acc[v];
     }
     __syncthreads();
     if (wave || m0 + l32 >= m) return;
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int v = 0; v < 16; ++v) acc[v] = ((acc[v] + part[0][v][lane]) + part[1][v][lane]) + part[2][v][lane];
+    float* yp = y + (size_t)(m0 + l32) * n + n0 + 4u * lg;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[t][v] = ((acc[t][v] + part[0][t][v][lane]) + part[1][t][v][lane]) + part[2][t][v][lane];
-        float* yp = y + (size_t)(m0 + l32) * n + n0 + 32u * t + 4u * lg;
+    for (int g = 0; g < 4; ++g)
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (n0 + 32u * t + 4u * lg + 8u * g + i < n) yp[8 * g + i] = acc[t][4 * g + i];
-    }
+        for (int i = 0; i < 4; ++i)
+            if (n0 + 4u * lg + 8u * g + i < n) yp[8 * g + i] = acc[4 * g + i];
 }
 
 }  // namespace
@@ -237,7 +254,7 @@ int launch_dense_gemv_bf16_pair(hipStream_t s, const void* x, hq_act_dtype xdt, 
     // tokens x 256 experts x 2048: one wave per (token, expert) over the whole row took 175 us); a second matrix of a few
     // rows (the shared expert's gate) keeps the one-wave-per-output form in a launch of its own.
     if (m >= 32 && n_a >= 32 && k % 16 == 0) {
-        const uint32_t tiles_a = ((m + 31u) / 32u) * ((n_a + 63u) / 64u);
+        const uint32_t tiles_a = ((m + 255u) / 256u * 8u) * ((n_a + 31u) / 32u);
         if (xdt == HQ_BF16)
             hipLaunchKernelGGL(dense_gemm_bf16_kernel<true>, dim3(tiles_a), dim3(256), 0, s, x, wa, y_a, m, n_a, k);
         else
