@@ -1437,7 +1437,7 @@ int launch_flat_passes(hipStream_t s, const void* x, const uint8_t* w0, const ui
 // rows of eleven super-blocks badly and whose many workgroups each stage the activations again; 7.0 us here (bf16: 8.8 -> 6.9).  In
 // that kernel / here, us at one and two rows: Q8_0 f32 12.8 / 7.6 and 15.4 / 10.8, Q4_0 bf16 8.7 / 5.6 and 13.1 / 7.5, Q6_K bf16 9.0 / 6.7 and
 // 11.4 / 9.1; x 4096: Q4_K f32 10.5 / 6.2 and 14.7 / 8.3, bf16 7.4 / 7.4 and 9.6 / 9.7, Q8_0 11.6 / 9.9 and 15.9 / 14.0.  Eight entries,
-// a row each: three rows of three products stay with that kernel.
+// a row each; more rows: gemv_flat_jobs_rows_kernel.
 constexpr uint32_t MAX_FLAT_JOBS = 8;
 struct FJobs {
     FArgs j[MAX_FLAT_JOBS];
@@ -1512,6 +1512,101 @@ int launch_flat_jobs(hipStream_t s, const GemvArgs* jobs, uint32_t n_jobs, uint3
     if (int rc = ensure_lds_limit(reinterpret_cast<const void*>(kern), lds, "hipFuncSetAttribute(gemv flat jobs LDS)")) return rc;
     hipLaunchKernelGGL(kern, dim3(fj.first[fj.count]), dim3(64 * W), lds, s, fj);
     return check_launch("gemv flat jobs kernel launch");
+}
+
+// The same of two rows and more: an entry is a product's rows, or as many of them as a pass takes, walked together as
+// gemv_flat_rows_kernel walks them; bound by the LDS reads of the activations, where an entry per row or gemv_jobs_kernel fetched and
+// converted the weights for every row.  q / k / v and the output projection (a launch of its own, the same before and after) of
+// 4096 + 1024 + 1024 rows x 2816, us per layer at 3 / 5 / 8 rows, before and here: Q4_K f32 27.2 / 34.6 / 38.9 and 14.7 / 19.9 / 27.8,
+// bf16 20.5 / 20.5 / 24.6 and 15.0 / 17.6 / 21.7; Q8_0 f32 31.9 / 43.0 / 49.8 and 21.1 / 26.9 / 32.9; Q6_K f32 25.0 / 31.9 / 51.9 and 18.6 / 27.0 /
+// 37.0; Q4_0 f32 22.9 / 30.4 / 40.0 and 18.4 / 25.0 / 31.6.  At two rows Q6_K 16.7 and 15.6, Q8_0 19.0 and 18.6, Q5_K 15.2 and 14.0, but Q4_0 14.6
+// and 15.7, Q4_K 13.6 and 13.8: those two from three rows on.  Q4_0 under bf16 rows stays with gemv_jobs_kernel, whose products there are
+// exact (6e-7 of the result between the two).
+struct FJobsRows {
+    FJobs f;
+    uint32_t rows[MAX_FLAT_JOBS];
+};
+template <int TYPE, bool X_BF16, int NR>
+__global__ __launch_bounds__(64 * kFlatRowsWaves<TYPE>) void gemv_flat_jobs_rows_kernel(FJobsRows js) {
+    constexpr uint32_t W = kFlatRowsWaves<TYPE>;
+    using X = FlatX<TYPE, X_BF16>;
+    extern __shared__ uint4 smem[];
+    uint32_t i = 0;
+    while (i + 1u < js.f.count && blockIdx.x >= js.f.first[i + 1u]) ++i;  // uniform
+    const FArgs& a = js.f.j[i];
+    const uint32_t wg = blockIdx.x - js.f.first[i], wgs = js.f.first[i + 1u] - js.f.first[i], rows = js.rows[i];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t x_pitch = (uint32_t)(X::value_bytes(a.k) / 16u), s_pitch = a.k / 16u;
+    float* lds_s = reinterpret_cast<float*>(smem + NR * x_pitch);
+#pragma unroll
+    for (uint32_t r = 0; r < (uint32_t)NR; ++r)  // (past the entry's rows: its last one, whose sums are not stored again)
+        X::stage(static_cast<const uint8_t*>(a.x) + (size_t)(r < rows ? r : rows - 1u) * a.k * (X_BF16 ? 2 : 4), a.k, smem + r * x_pitch, lds_s + r * s_pitch,
+                 tid, 64u * W);
+    FlatWalk<TYPE, X_BF16> wk;
+    wk.init(a.w0, a.w0, a.n, 1u, a.g, wv * wgs + wg, W * wgs);
+    wk.prime();
+    __syncthreads();
+    wk.load_masks(a.m4, a.m2, a.magic);
+    wk.template run_rows<NR>(smem, lds_s, x_pitch, s_pitch, [&](uint32_t cnt, const float* k0, const float*, uint32_t row) {
+        if (lane < cnt && row < a.n) {
+#pragma unroll
+            for (uint32_t r = 0; r < (uint32_t)NR; ++r)
+                if (r < rows) a.y0[(size_t)r * a.n + row] = k0[r];
+        }
+    });
+}
+
+// Rows per entry, 0 where the form does not take the products: dense ones of sizes the flat form takes, all of the same rows.
+template <int TYPE, bool X_BF16>
+uint32_t flat_jobs_rows_take(const GemvArgs* jobs, uint32_t n_jobs, uint32_t cus) {
+    const uint32_t m = jobs[0].pairs;
+    if (m < (TYPE == HQ_Q4_K || TYPE == HQ_Q4_0 ? 3u : 2u) || m > 8u || (TYPE == HQ_Q4_0 && X_BF16)) return 0;
+    uint32_t most = m;
+    for (uint32_t i = 0; i < n_jobs; ++i) {
+        const GemvArgs& j = jobs[i];
+        if (j.x2 || j.ids || j.route_logits || j.pairs != m) return 0;
+        if (kBlock32<TYPE> && j.k < 1024) return 0;
+        const size_t lds = FlatX<TYPE, X_BF16>::lds_bytes(j.k);
+        if (!flat_takes<TYPE>(j.n, j.k, cus, lds) && !flat_takes_small<TYPE, X_BF16>(j.n, j.k, cus, lds)) return 0;
+        const uint32_t fit = flat_rows_per_pass<TYPE, X_BF16>(j.k);
+        most = fit < most ? fit : most;
+    }
+    const uint32_t groups = (m + most - 1u) / most;
+    return n_jobs * groups <= MAX_FLAT_JOBS && most >= 2u ? (m + groups - 1u) / groups : 0u;
+}
+template <int TYPE, bool X_BF16, int NR = kFlatMaxRows<TYPE, X_BF16>>
+int launch_flat_jobs_rows(hipStream_t s, const GemvArgs* jobs, uint32_t n_jobs, uint32_t per, uint32_t cus) {
+    if constexpr (NR > 2)
+        if (per < (uint32_t)NR) return launch_flat_jobs_rows<TYPE, X_BF16, NR - 1>(s, jobs, n_jobs, per, cus);
+    constexpr uint32_t W = kFlatRowsWaves<TYPE>, UE = kUnitElems<TYPE>;
+    FJobsRows js{};
+    FJobs& fj = js.f;
+    size_t lds = 81 * 1024;  // more than half a CU's LDS: one workgroup per CU
+    const uint32_t groups = (jobs[0].pairs + per - 1u) / per;
+    uint64_t total = 0, sofar = 0;
+    for (uint32_t i = 0; i < n_jobs; ++i) total += (uint64_t)groups * jobs[i].n * (jobs[i].k / UE);
+    for (uint32_t i = 0; i < n_jobs; ++i) {
+        const GemvArgs& j = jobs[i];
+        const size_t l = (size_t)NR * FlatX<TYPE, X_BF16>::lds_bytes(j.k);
+        lds = l > lds ? l : lds;
+        for (uint32_t r = 0; r < j.pairs; r += per) {
+            const uint32_t q = fj.count++;
+            sofar += (uint64_t)j.n * (j.k / UE);
+            uint32_t end = (uint32_t)((sofar * cus + total / 2) / total);
+            if (end <= fj.first[q]) end = fj.first[q] + 1u;
+            fj.first[q + 1u] = end;
+            js.rows[q] = j.pairs - r < per ? j.pairs - r : per;
+            float* y = j.y + (size_t)r * j.n;
+            fj.j[q] = FArgs{static_cast<const uint8_t*>(j.x) + (size_t)r * j.k * (X_BF16 ? 2 : 4), j.w, j.w, y, y, j.n, j.k, 1u, 0u,
+                            flat_geom(j.k, UE, kUnitsPerWindow<TYPE>, j.n, 1, (end - fj.first[q]) * W), TYPE == HQ_Q6_K ? N4 : M4,
+                            TYPE == HQ_Q5_K ? M1 : TYPE == HQ_Q6_K ? N2 : M2, MAGIC};
+        }
+    }
+    auto kern = gemv_flat_jobs_rows_kernel<TYPE, X_BF16, NR>;
+    if (int rc = ensure_lds_limit(reinterpret_cast<const void*>(kern), lds, "hipFuncSetAttribute(gemv flat jobs rows LDS)")) return rc;
+    hipLaunchKernelGGL(kern, dim3(fj.first[fj.count]), dim3(64 * W), lds, s, js);
+    return check_launch("gemv flat jobs rows kernel launch");
 }
 
 template <typename K>
@@ -1731,6 +1826,7 @@ int launch_jobs_t(hipStream_t s, const GemvArgs* jobs, uint32_t n_jobs) {
             flat_takes<TYPE>((uint64_t)j0.n * 2, j0.k, cus, FlatX<TYPE, X_BF16>::lds_bytes(j0.k)))
             return launch_flat_passes<TYPE, X_BF16>(s, j0.x, j0.w, j1.w, j0.y, j1.y, j0.pairs, j0.n, j0.k, 2, cus);
     }
+    if (const uint32_t per = flat_jobs_rows_take<TYPE, X_BF16>(jobs, n_jobs, cus)) return launch_flat_jobs_rows<TYPE, X_BF16>(s, jobs, n_jobs, per, cus);
     if (flat_jobs_take<TYPE, X_BF16>(jobs, n_jobs, cus)) return launch_flat_jobs<TYPE, X_BF16>(s, jobs, n_jobs, cus);
     const uint64_t per_simd = slots / (4ull * cus);
     if (per_simd >= 8) return launch_j<TYPE, X_BF16, PAIR, 4, 4>(s, js, n_jobs, lds);

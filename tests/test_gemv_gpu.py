@@ -151,6 +151,20 @@ def test_batch_of_dense_products_matches_oracle(oracle, dev, t, xdt, shapes):
         assert_matmul_close(j.output.cpu().numpy(), ref, f"batched dense t={t} {xdt} {j.rows}x{j.n}x{j.k}")
 
 
+@pytest.mark.parametrize("t", ALL_TYPES)
+@pytest.mark.parametrize("xdt", ["bf16", "f32"])
+@pytest.mark.parametrize("m,shapes", [
+    (2, [(1100, 1280), (515, 2816)]),
+    (3, [(1100, 1280), (515, 1280), (70, 1280)]),
+    (7, [(600, 2816), (2050, 1280)]),             # f32 K-quants: passes of four and three
+    (8, [(1024, 7424), (600, 2816), (33, 1280)]),  # two passes where LDS holds fewer of the long rows
+    (8, [(600, 12288), (600, 2816), (600, 1280)]),  # three passes of three products: more than the form takes
+])
+def test_batch_of_dense_products_of_the_same_rows_matches_oracle(oracle, dev, t, xdt, m, shapes):
+    """Two to eight rows of every product: walked together, several rows to a fetch of the weights."""
+    test_batch_of_dense_products_matches_oracle(oracle, dev, t, xdt, [(n, k, m) for n, k in shapes])
+
+
 ID_CASES = [  # (E, n, k, T, K); k = 768, 2816, 1280: rows whose pieces no sixteen lanes divide (a ragged last step under bf16 rows)
     (8, 64, 512, 1, 2), (16, 512, 2048, 1, 8), (16, 2048, 512, 8, 1), (256, 128, 256, 8, 8), (4, 33, 768, 5, 3),
     (8, 48, 2816, 3, 2), (4, 40, 1280, 2, 4),
