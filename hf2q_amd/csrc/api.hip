@@ -259,7 +259,7 @@ int qmatmul_routes(hipStream_t stream, const void* x, hq_act_dtype xdt, const vo
             }
             continue;
         }
-        if (gemv_rows32_supported(t, rows, k)) {
+        if (gemv_rows32_supported(t, rows, k) && !(t == HQ_Q8_0 && gemv_q80_rows_walked(xdt, rows, n, k))) {
             if (int rc = launch_gemv_rows32(stream, static_cast<const uint8_t*>(x) + (size_t)r0 * xrow_bytes, xdt, w_blocks,
                                             y + (size_t)r0 * n, rows, n, k, t))
                 return rc;

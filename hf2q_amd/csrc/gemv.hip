@@ -1929,6 +1929,23 @@ bool gemv_flat_rows_preferred(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint
     return false;
 }
 
+// Rows of Q8_0 over a matrix of ordinary size in one pass of the flat walk, where the kernel of small batches (gemvr32.hip) stages k in
+// chunks and meets its barriers once per 2048 of them; both have exact products.  us per layer of q / k / v and the output projection,
+// that kernel / the walk: n 2816 x k 8192 at 2 / 4 f32 rows 26.5 / 20.3 and 33.6 / 27.1, bf16 at 3 / 6 30.6 / 22.7 and 43.6 / 37.9; 2048 x 4096 at
+// 4 / 8 16.2 / 14.2 and 22.8 / 21.4; two passes of 5120 x 6144 at 8 rows 50.9 / 54.9.  Against matrices of sixteen weight rows per CU and
+// more the walk loses from four rows on (4096 x 4096 at 2 / 4 / 8 rows 19.7 / 18.8, 24.1 / 24.3, 34.4 / 35.6).
+bool gemv_q80_rows_walked(hq_act_dtype xdt, uint32_t m, uint32_t n, uint32_t k) {
+    uint32_t cus = 0;
+    if (m < 2 || n >= 8192 || cu_count(&cus)) return false;
+    auto go = [&](auto bf) {
+        constexpr bool BF = decltype(bf)::value;
+        const size_t lds = FlatX<HQ_Q8_0, BF>::lds_bytes(k);
+        return m <= flat_rows_per_pass<HQ_Q8_0, BF>(k) && (m <= 3u || n < 16u * cus) &&
+               (flat_takes<HQ_Q8_0>(n, k, cus, lds) || flat_takes_small<HQ_Q8_0, BF>(n, k, cus, lds));
+    };
+    return xdt == HQ_BF16 ? go(std::true_type{}) : go(std::false_type{});
+}
+
 int launch_gemv(hipStream_t s, const GemvArgs& a, hq_act_dtype xdt, hq_ggml_type t) {
     const bool bf = xdt == HQ_BF16;
     switch (t) {
