@@ -1213,12 +1213,13 @@ int launch_flat(hipStream_t s, const void* x, const uint8_t* w0, const uint8_t* 
 // 107; Q4_K 12288 x 4096 bf16: 23 / 34 / 56 / 88 -> 17 / 21 / 27 / 38; Q8_0 37 / 55 / 91 / 145 -> 21 / 24 / 32 / 44.  One matrix,
 // Q6_K 5120 x 6144 f32: 15 / 22 -> 10 / 12 at 2 / 3 rows.
 //
-// PAIRED (K-quants): two pieces meet every activation read from LDS (run_rows_paired), by twelve waves per CU.
-template <int TYPE, bool PAIRED = false>
+// PAIRED (K-quants): two pieces meet every activation read from LDS (run_rows_paired), by twelve waves per CU; the number of matrices
+// they are of.
+template <int TYPE, int PAIRED = 0>
 constexpr int kFlatRowsWaves = PAIRED || kBaseType<TYPE> == HQ_Q6_K || kBlock32<kBaseType<TYPE>> ? 12 : 16;
 template <int TYPE>
 constexpr bool kFlatPairs = !kIsX2<TYPE> && !kBlock32<TYPE>;
-template <int TYPE, bool X_BF16, int NR, bool PAIRED>
+template <int TYPE, bool X_BF16, int NR, int PAIRED>
 __global__ __launch_bounds__((64 * kFlatRowsWaves<TYPE, PAIRED>)) void gemv_flat_rows_kernel(FArgs a) {
     constexpr uint32_t W = kFlatRowsWaves<TYPE, PAIRED>;
     using X = FlatX<TYPE, X_BF16>;
@@ -1233,8 +1234,15 @@ __global__ __launch_bounds__((64 * kFlatRowsWaves<TYPE, PAIRED>)) void gemv_flat
         X::stage(static_cast<const uint8_t*>(a.x) + (size_t)r * a.k * (X_BF16 ? 2 : 4), a.k, smem + r * x_pitch, lds_s + r * s_pitch, tid, 64u * W);
     FlatWalk<TYPE, X_BF16> wk;
     wk.init(a.w0, a.w1, a.n, a.nm, a.g, wv * gridDim.x + blockIdx.x, W * gridDim.x);
+    [[maybe_unused]] Piece<TYPE> pair[2];
+    // (the first fetch ahead of the barrier hides its round trip; bf16 rows whose waves all have a task only get their activations
+    // staged later by it: gate + up of 3072 x 4096 Q6_K at five rows 12.1 and 12.8 us without and with, 2048 x 2048 10.2 and 9.7)
+    const bool ahead = !X_BF16 || (a.n >> a.g.log_r) < 8u * gridDim.x;
     if constexpr (!PAIRED) wk.prime();
+    else if (ahead) wk.prime_pair(pair);
     __syncthreads();
+    if constexpr (PAIRED)
+        if (!ahead) wk.prime_pair(pair);
     wk.load_masks(a.m4, a.m2, a.magic);
     auto out = [&](uint32_t cnt, const float* k0, const float* k1, uint32_t row) {
         if (lane < cnt && row < a.n) {
@@ -1245,12 +1253,12 @@ __global__ __launch_bounds__((64 * kFlatRowsWaves<TYPE, PAIRED>)) void gemv_flat
                 } else {
                     a.y0[(size_t)r * a.n + row] = k0[r];
                     if (a.nm == 2u) a.y1[(size_t)r * a.n + row] = k1[r];
-                    if (PAIRED && a.nm == 1u && row + wk.pair_rows() < a.n) a.y0[(size_t)r * a.n + row + wk.pair_rows()] = k1[r];
+                    if (PAIRED == 1 && row + wk.pair_rows() < a.n) a.y0[(size_t)r * a.n + row + wk.pair_rows()] = k1[r];
                 }
             }
         }
     };
-    if constexpr (PAIRED) wk.template run_rows_paired<NR>(smem, lds_s, x_pitch, s_pitch, out);
+    if constexpr (PAIRED) wk.template run_rows_paired<NR, PAIRED == 1>(pair, smem, lds_s, x_pitch, s_pitch, out);
     else wk.template run_rows<NR>(smem, lds_s, x_pitch, s_pitch, out);
 }
 
@@ -1279,7 +1287,9 @@ __global__ __launch_bounds__((64 * kFlatRowsWaves<TYPE, PAIRED>)) void gemv_flat
     FlatWalk<TYPE, false, 1, false, false, false, true> wk;
     wk.init(a.w0, a.w0, a.n, 1u, a.g, wv * gridDim.x + blockIdx.x, W * gridDim.x);
     wk.pitch_u = s.k_row / kUnitElems<TYPE>;
-    if constexpr (!PAIRED) wk.prime();
+    [[maybe_unused]] Piece<TYPE> pair[2];
+    if constexpr (PAIRED) wk.prime_pair(pair);
+    else wk.prime();
     __syncthreads();
     wk.load_masks(a.m4, a.m2, a.magic);
     auto out = [&](uint32_t cnt, const float* k0, const float* k1, uint32_t row) {
@@ -1295,19 +1305,24 @@ __global__ __launch_bounds__((64 * kFlatRowsWaves<TYPE, PAIRED>)) void gemv_flat
             }
         }
     };
-    if constexpr (PAIRED) wk.template run_rows_paired<NR>(smem, lds_s, x_pitch, s_pitch, out);
+    if constexpr (PAIRED) wk.template run_rows_paired<NR, true>(pair, smem, lds_s, x_pitch, s_pitch, out);
     else wk.template run_rows<NR>(smem, lds_s, x_pitch, s_pitch, out);
 }
 
 // Two pieces at a time: both matrices' where there are two, else (three rows or more) where every wave has two super-tasks to
-// pair.  Gate + up at five f32 rows, Q5_K: 17408 x 5120 62 -> 48 us, 12288 x 4096 32 -> 28, 4101 x 2816 15.6 -> 12.6, at two 36 -> 32,
-// 19.5 -> 18.9, 9.4 -> 8.7; bf16 55 -> 48, 29 -> 27, 14.4 -> 12.9.  One matrix, Q6_K f32 28000 x 5120: 31 -> 32 at two rows, 47 -> 45 at five.
+// pair.  Gate + up at five f32 rows, Q5_K: 17408 x 5120 62 -> 51 us, 12288 x 4096 35 -> 31, 4101 x 2816 16.0 -> 13.3, at two 35 -> 32,
+// 21.2 -> 20.5, 9.1 -> 8.5; bf16 57 -> 50, 30 -> 27, 14.7 -> 13.5.  One matrix, Q6_K f32 28000 x 5120: 31 -> 32 at two rows, 48 -> 43 at five;
+// 9216 x 4096 (three super-tasks a wave) 16.8 -> 16.1.  Q4_K / Q5_K at three rows, which unpaired have sixteen waves, from four
+// super-tasks a wave on: 9216 x 4096 Q4_K 10.9 and 11.7, 17408 x 2048 Q5_K 12.1 and 13.1, 12300 x 3584 13.1 and 12.2.
 // Q6_K under bf16 rows from four to six: 20 -> 23 us at two rows of 14336 x 4096, 31 -> 30 at five, and the registers of seven
 // rows and eight no longer fit (41 -> 45 at eight, 12288 x 4096).
 template <int TYPE, bool X_BF16, int NR>
-inline bool flat_paired(const FArgs& fa, uint32_t cus) {
-    if (TYPE == HQ_Q6_K && X_BF16 && (NR < 4 || NR > 6)) return false;
-    return fa.nm == 2u || (NR >= 3 && (fa.n >> fa.g.log_r) >= 2u * 12u * cus);
+constexpr bool kPairsTwo = kFlatPairs<TYPE> && !(TYPE == HQ_Q6_K && X_BF16 && (NR < 4 || NR > 6));
+template <int TYPE, bool X_BF16, int NR>
+constexpr bool kPairsOne = kPairsTwo<TYPE, X_BF16, NR> && NR >= 3;
+template <int TYPE, int NR>
+inline bool flat_pairs_one(const FArgs& fa, uint32_t cus) {
+    return (fa.n >> fa.g.log_r) >= (TYPE == HQ_Q6_K || NR > 3 ? 2u : 4u) * 12u * cus;
 }
 
 // Rows per pass at most: eight; six of f32 K-quant rows, which keep the sums of two halves each.
@@ -1317,13 +1332,12 @@ template <int TYPE, bool X_BF16, int NR = kFlatMaxRows<TYPE, X_BF16>>
 int launch_flat_rows(hipStream_t s, const FArgs& fa, uint32_t rows, size_t lds, uint32_t cus) {
     if constexpr (NR > 2)
         if (rows < (uint32_t)NR) return launch_flat_rows<TYPE, X_BF16, NR - 1>(s, fa, rows, lds, cus);
-    auto kern = gemv_flat_rows_kernel<TYPE, X_BF16, NR, false>;
+    auto kern = gemv_flat_rows_kernel<TYPE, X_BF16, NR, 0>;
     uint32_t waves = kFlatRowsWaves<TYPE>;
-    if constexpr (kFlatPairs<TYPE>)
-        if (flat_paired<TYPE, X_BF16, NR>(fa, cus)) {
-            kern = gemv_flat_rows_kernel<TYPE, X_BF16, NR, true>;
-            waves = kFlatRowsWaves<TYPE, true>;
-        }
+    if constexpr (kPairsTwo<TYPE, X_BF16, NR>)
+        if (fa.nm == 2u) kern = gemv_flat_rows_kernel<TYPE, X_BF16, NR, 2>, waves = kFlatRowsWaves<TYPE, 2>;
+    if constexpr (kPairsOne<TYPE, X_BF16, NR>)
+        if (fa.nm == 1u && flat_pairs_one<TYPE, NR>(fa, cus)) kern = gemv_flat_rows_kernel<TYPE, X_BF16, NR, 1>, waves = kFlatRowsWaves<TYPE, 1>;
     if (int rc = ensure_lds_limit(reinterpret_cast<const void*>(kern), lds, "hipFuncSetAttribute(gemv flat rows LDS)")) return rc;
     hipLaunchKernelGGL(kern, dim3(cus), dim3(64 * waves), lds, s, fa);
     return check_launch("gemv flat rows kernel launch");
@@ -1355,12 +1369,13 @@ FlatSlices flat_slices(uint32_t m, uint32_t k) {
 }
 template <int TYPE, int NR = kFlatMaxRows<TYPE, false>>
 int launch_flat_slice(hipStream_t s, const FSliceArgs& fa, uint32_t rows, size_t lds, uint32_t cus) {
-    if constexpr (NR > 1)
+    if constexpr (NR > 3)  // (flat_slices_take: three rows or more, and passes of three or more)
         if (rows < (uint32_t)NR) return launch_flat_slice<TYPE, NR - 1>(s, fa, rows, lds, cus);
-    const bool paired = flat_paired<TYPE, false, NR>(fa.f, cus);
+    if (rows != (uint32_t)NR) return fail(HQ_ERR_UNSUPPORTED, "gemv flat slices: %u rows", rows);
+    const bool paired = flat_pairs_one<TYPE, NR>(fa.f, cus);
     auto kern = paired ? gemv_flat_slice_kernel<TYPE, NR, true> : gemv_flat_slice_kernel<TYPE, NR, false>;
     if (int rc = ensure_lds_limit(reinterpret_cast<const void*>(kern), lds, "hipFuncSetAttribute(gemv flat slice LDS)")) return rc;
-    hipLaunchKernelGGL(kern, dim3(cus), dim3(64 * (paired ? kFlatRowsWaves<TYPE, true> : kFlatRowsWaves<TYPE>)), lds, s, fa);
+    hipLaunchKernelGGL(kern, dim3(cus), dim3(64 * (paired ? kFlatRowsWaves<TYPE, 1> : kFlatRowsWaves<TYPE>)), lds, s, fa);
     return check_launch("gemv flat slice kernel launch");
 }
 template <int TYPE>

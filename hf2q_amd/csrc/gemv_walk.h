@@ -648,10 +648,11 @@ struct FlatWalk {
         if (done & 63u) out(done & 63u, keep0, keep1, keep_row);
     }
 
-    // run_rows over two pieces at a time that meet the same activations: the same window of both matrices (nm == 2), or of two
+    // run_rows over two pieces at a time that meet the same activations: the same window of both matrices (nm == 2), or (ONE) of two
     // super-tasks one after the other in the wave's sequence (nm == 1), so that an activation read from LDS serves twice the
     // weights.  K-quants.  The operations and their order per row are those of run_rows: the same bits.  out's keep1: the second
-    // matrix's sums, or those of the rows pair_rows() further on (past the matrix's end where the sequence has none left).
+    // matrix's sums, or those of the rows pair_rows() further on (past the matrix's end for a super-task by itself).  The caller
+    // has fetched the first two pieces (prime_pair).
     __device__ __forceinline__ uint32_t pair_rows() const { return nm == 2u ? 0u : seq_stride << g.log_r; }
     __device__ __forceinline__ void fetch_pair(Piece<TYPE>& pa, Piece<TYPE>& pb) {
         const uint32_t sid = seq_first + f_q * seq_stride;
@@ -671,16 +672,18 @@ struct FlatWalk {
             f_q += 3u - nm;
         }
     }
-    template <int NR, typename OUT>
-    __device__ __forceinline__ void run_rows_paired(const uint4* lds_x, const float* lds_s, uint32_t x_pitch, uint32_t s_pitch, OUT&& out) {
+    __device__ __forceinline__ void prime_pair(Piece<TYPE> (&p)[2]) {
+        if (q_cur < count) fetch_pair(p[0], p[1]);
+    }
+    template <int NR, bool ONE, typename OUT>
+    __device__ __forceinline__ void run_rows_paired(Piece<TYPE> (&p)[2], const uint4* lds_x, const float* lds_s, uint32_t x_pitch, uint32_t s_pitch, OUT&& out) {
         static_assert(D == 1 && !DYN && !COPY && !kLaneUnit<TYPE> && !kIsX2<TYPE>, "the plain walk of a K-quant");
         uint32_t c_w = 0, done = 0, keep_row = 0;
         float keep0[NR] = {}, keep1[NR] = {}, acc0[NR] = {}, acc1[NR] = {};
         const int last_lane = (int)(g.uwe * LPU - 1u);
         const bool one_row = g.log_r == 0u;
-        Piece<TYPE> pa, pb;
-        if (q_cur < count) fetch_pair(pa, pb);
-        while (q_cur < count) {
+        Piece<TYPE>&pa = p[0], &pb = p[1];  // (prime_pair's)
+        while (q_cur + (ONE ? 1u : 0u) < count) {
             const uint32_t lu_raw = g.uwe * c_w + lv, su = g.bu << g.log_r;
             const bool in_task = lu_raw < su;
             const uint32_t lu = in_task ? lu_raw : su - 1u;
@@ -773,6 +776,11 @@ struct FlatWalk {
             }
         }
         if (done & 63u) out(done & 63u, keep0, keep1, keep_row);
+        if constexpr (ONE)
+            if (q_cur < count) {  // the last super-task of an odd number, by itself: its first window is in pa
+                buf[0] = pa;
+                run_rows<NR>(lds_x, lds_s, x_pitch, s_pitch, out);
+            }
     }
 };
 

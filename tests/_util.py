@@ -68,3 +68,37 @@ def weights(seed, n, k, sigma=0.02):
 
 def acts(seed, m, k):
     return np.random.default_rng(seed).standard_normal((m, k), dtype=np.float32)
+
+
+def launched_kernels(call):
+    """Names (mangled) of the kernels that call() launches on the current device, in order.  It is captured into a graph that is
+    never run, so the call itself must have run once before."""
+    import ctypes
+
+    import torch
+
+    class Dim3(ctypes.Structure):
+        _fields_ = [("x", ctypes.c_uint32), ("y", ctypes.c_uint32), ("z", ctypes.c_uint32)]
+
+    class KernelNodeParams(ctypes.Structure):
+        _fields_ = [("block", Dim3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", Dim3), ("params", ctypes.c_void_p),
+                    ("shared", ctypes.c_uint32)]
+
+    hip = ctypes.CDLL("libamdhip64.so.7")  # (the one torch has loaded)
+    hip.hipKernelNameRefByPtr.restype = ctypes.c_char_p
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        call()
+    graph, n = ctypes.c_void_p(int(g.raw_cuda_graph())), ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(graph, nodes, ctypes.byref(n)) == 0
+    names = []
+    for node in nodes:
+        kind, p = ctypes.c_int(), KernelNodeParams()
+        assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0
+        if kind.value == 0:  # a kernel
+            assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
+            names.append(hip.hipKernelNameRefByPtr(ctypes.c_void_p(p.func), ctypes.c_void_p(0)).decode())
+    return names

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from _util import acts, assert_matmul_close, weights
-from _util import assert_matmul_close_f16_tile
+from _util import assert_matmul_close_f16_tile, launched_kernels
 from hf2q_amd import ops
 from hf2q_amd.ops import (HQ_Q4_0, HQ_Q4_K, HQ_Q5_K, HQ_Q6_K, HQ_Q8_0, GgmlQuantizedMatmulIdParams,
                           GgmlQuantizedMatmulParams)
@@ -163,6 +163,35 @@ def test_batch_of_dense_products_matches_oracle(oracle, dev, t, xdt, shapes):
 def test_batch_of_dense_products_of_the_same_rows_matches_oracle(oracle, dev, t, xdt, m, shapes):
     """Two to eight rows of every product: walked together, several rows to a fetch of the weights."""
     test_batch_of_dense_products_matches_oracle(oracle, dev, t, xdt, [(n, k, m) for n, k in shapes])
+
+
+@pytest.mark.parametrize("t,n,k,m", [
+    # super-tasks of four rows, two or three to a wave: pairs, a last one by itself, and a ragged end
+    (HQ_Q6_K, 28001, 2816, 3), (HQ_Q6_K, 28001, 2816, 6), (HQ_Q6_K, 28003, 5120, 5), (HQ_Q5_K, 28003, 5120, 5), (HQ_Q4_K, 28003, 5120, 6),
+    (HQ_Q6_K, 9001, 3584, 3), (HQ_Q6_K, 9001, 3584, 5),  # of one row, two or three to a wave
+    (HQ_Q4_K, 12300, 3584, 3), (HQ_Q5_K, 12300, 3584, 3),  # four or five
+    (HQ_Q6_K, 17411, 2048, 4),  # of two rows
+    (HQ_Q6_K, 8195, 14336, 3), (HQ_Q5_K, 8195, 14336, 4),  # slices of k, two or three to a wave
+])
+def test_rows_over_pairs_of_super_tasks(dev, t, n, k, m):
+    """Several f32 rows over one K-quant matrix whose super-tasks a wave takes two at a time: every output against float64 products
+    of the dequantised weights (which are tested bit for bit), and the bits of the two-row walk, which takes them one by one."""
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(n + m)
+    w = ops.quantize_ggml(torch.randn(n * k, generator=gen, device=dev).mul_(0.02), k, t)
+    x = torch.randn(m, k, generator=gen, device=dev)
+    y, y2 = torch.full((m, n), float("nan"), device=dev), torch.full((2, n), float("nan"), device=dev)
+    call = lambda: ops.quantized_matmul_ggml(x, w, y, GgmlQuantizedMatmulParams(m, n, k, t))  # noqa: E731
+    call()
+    ref = x.double() @ ops.dequantize_ggml(w, n * k, t).view(n, k).double().T
+    assert_matmul_close(y.cpu().numpy(), ref.cpu().numpy(), f"paired super-tasks t={t} {m}x{n}x{k}")
+    names = launched_kernels(call)
+    sliced = k == 14336
+    assert all(f"gemv_flat_slice_kernelILi{t}ELi{m}ELb1E" in s or f"gemv_flat_rows_kernelILi{t}ELb0ELi{m}ELi1E" in s for s in names), names
+    assert len(names) > 1 if sliced else len(names) == 1
+    if not sliced:
+        ops.quantized_matmul_ggml(x[:2].contiguous(), w, y2, GgmlQuantizedMatmulParams(2, n, k, t))
+        assert torch.equal(y[:2], y2)
 
 
 ID_CASES = [  # (E, n, k, T, K); k = 768, 2816, 1280: rows whose pieces no sixteen lanes divide (a ragged last step under bf16 rows)
