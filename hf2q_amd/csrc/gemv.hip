@@ -1529,17 +1529,18 @@ int launch_flat_jobs(hipStream_t s, const GemvArgs* jobs, uint32_t n_jobs, uint3
     return check_launch("gemv flat jobs kernel launch");
 }
 
-// The same of two rows and more: an entry is a product's rows, or as many of them as a pass takes, walked together as
-// gemv_flat_rows_kernel walks them; bound by the LDS reads of the activations, where an entry per row or gemv_jobs_kernel fetched and
-// converted the weights for every row.  q / k / v and the output projection (a launch of its own, the same before and after) of
-// 4096 + 1024 + 1024 rows x 2816, us per layer at 3 / 5 / 8 rows, before and here: Q4_K f32 27.2 / 34.6 / 38.9 and 14.7 / 19.9 / 27.8,
-// bf16 20.5 / 20.5 / 24.6 and 15.0 / 17.6 / 21.7; Q8_0 f32 31.9 / 43.0 / 49.8 and 21.1 / 26.9 / 32.9; Q6_K f32 25.0 / 31.9 / 51.9 and 18.6 / 27.0 /
-// 37.0; Q4_0 f32 22.9 / 30.4 / 40.0 and 18.4 / 25.0 / 31.6.  At two rows Q6_K 16.7 and 15.6, Q8_0 19.0 and 18.6, Q5_K 15.2 and 14.0, but Q4_0 14.6
-// and 15.7, Q4_K 13.6 and 13.8: those two from three rows on.  Q4_0 under bf16 rows stays with gemv_jobs_kernel, whose products there are
-// exact (6e-7 of the result between the two).
-struct FJobsRows {
-    FJobs f;
-    uint32_t rows[MAX_FLAT_JOBS];
+// The same of two rows and more: an entry is some of a product's rows, walked together as gemv_flat_rows_kernel walks them; bound by
+// the LDS reads of the activations, where an entry per row or gemv_jobs_kernel fetch and convert the weights for every row.
+// q / k / v of 4096 + 1024 + 1024 rows, us at 3 / 5 / 8 rows, in gemv_jobs_kernel and here: x 2816 Q4_K f32 20.9 / 26.5 / 26.1 and 9.2 /
+// 12.6 / 16.4, bf16 13.1 / 13.2 / 17.1 and 8.4 / 10.7 / 14.7, Q8_0 f32 21.0 / 27.2 / 33.0 and 10.4 / 13.6 / 18.4, Q6_K f32 17.0 / 19.9 / 28.6 and
+// 10.6 / 15.8 / 19.4, Q4_0 f32 14.7 / 18.1 / 24.6 and 10.0 / 13.6 / 19.2; x 4096 Q4_K f32 19.5 / 27.4 / 38.5 and 9.6 / 13.1 / 17.1, Q8_0 f32
+// 16.1 / 23.3 / 32.6 and 10.7 / 13.7 / 18.3.  At two rows Q4_K and Q4_0 are the same as an entry per row, the other types 1 us faster.  Q4_0
+// under bf16 rows stays with gemv_jobs_kernel, whose products there are exact (6e-7 of the result between the two).
+struct FJobsRows {  // (what an entry is found by: one cache line)
+    uint32_t count, m, per;                     // products; rows in all and to an entry
+    uint32_t first[HQ_QMATMUL_BATCH_MAX_JOBS];  // product i's entries run on share[i] workgroups each, from first[i] on
+    uint32_t share[HQ_QMATMUL_BATCH_MAX_JOBS];
+    FArgs j[HQ_QMATMUL_BATCH_MAX_JOBS];
 };
 template <int TYPE, bool X_BF16, int NR>
 __global__ __launch_bounds__(64 * kFlatRowsWaves<TYPE>) void gemv_flat_jobs_rows_kernel(FJobsRows js) {
@@ -1547,16 +1548,21 @@ __global__ __launch_bounds__(64 * kFlatRowsWaves<TYPE>) void gemv_flat_jobs_rows
     using X = FlatX<TYPE, X_BF16>;
     extern __shared__ uint4 smem[];
     uint32_t i = 0;
-    while (i + 1u < js.f.count && blockIdx.x >= js.f.first[i + 1u]) ++i;  // uniform
-    const FArgs& a = js.f.j[i];
-    const uint32_t wg = blockIdx.x - js.f.first[i], wgs = js.f.first[i + 1u] - js.f.first[i], rows = js.rows[i];
+    while (i + 1u < js.count && blockIdx.x >= js.first[i + 1u]) ++i;  // uniform
+    const FArgs& a = js.j[i];
+    const uint32_t wgs = js.share[i];
+    uint32_t wg = blockIdx.x - js.first[i], row0 = 0;
+    for (; wg >= wgs; wg -= wgs) row0 += js.per;  // (uniform)
+    const uint32_t rows = js.m - row0 < js.per ? js.m - row0 : js.per;
+    const uint8_t* x = static_cast<const uint8_t*>(a.x) + (size_t)row0 * a.k * (X_BF16 ? 2 : 4);
+    float* y = a.y0 + (size_t)row0 * a.n;
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t x_pitch = (uint32_t)(X::value_bytes(a.k) / 16u), s_pitch = a.k / 16u;
     float* lds_s = reinterpret_cast<float*>(smem + NR * x_pitch);
 #pragma unroll
     for (uint32_t r = 0; r < (uint32_t)NR; ++r)  // (past the entry's rows: its last one, whose sums are not stored again)
-        X::stage(static_cast<const uint8_t*>(a.x) + (size_t)(r < rows ? r : rows - 1u) * a.k * (X_BF16 ? 2 : 4), a.k, smem + r * x_pitch, lds_s + r * s_pitch,
+        X::stage(x + (size_t)(r < rows ? r : rows - 1u) * a.k * (X_BF16 ? 2 : 4), a.k, smem + r * x_pitch, lds_s + r * s_pitch,
                  tid, 64u * W);
     FlatWalk<TYPE, X_BF16> wk;
     wk.init(a.w0, a.w0, a.n, 1u, a.g, wv * wgs + wg, W * wgs);
@@ -1567,17 +1573,29 @@ __global__ __launch_bounds__(64 * kFlatRowsWaves<TYPE>) void gemv_flat_jobs_rows
         if (lane < cnt && row < a.n) {
 #pragma unroll
             for (uint32_t r = 0; r < (uint32_t)NR; ++r)
-                if (r < rows) a.y0[(size_t)r * a.n + row] = k0[r];
+                if (r < rows) y[(size_t)r * a.n + row] = k0[r];
         }
     });
 }
 
-// Rows per entry, 0 where the form does not take the products: dense ones of sizes the flat form takes, all of the same rows.
+// Rows per entry, 0 where the form does not take the products: dense ones of sizes the flat form takes, all of the same rows.  Each
+// line from batches of two and three products of 256 .. 4096 rows x 512 .. 5120 (7800 of them with types and rows), both sides:
+// * Where an entry per row fits gemv_flat_jobs_kernel and the windows of all rows give less than half a window per wave (1.5 of 32-weight
+//   blocks), that: 384 + 384 x 3072 Q6_K f32 at two rows 4.5 us and 4.7 here, 512 + 256 x 5120 Q8_0 at two 5.5 and 5.9.
+// * Little work in gemv_jobs_kernel (its lane steps per SIMD and per row): 768 + 192 + 192 x 768 Q4_K bf16 at seven rows 4.8 us there and 7.4
+//   here, 384 + 192 + 192 Q5_K 4.2 and 7.3.  f32 rows of K-quants: always here (256 + 64 + 64 x 2816 Q4_K at three 11.4 and 5.3).
+// * Q4_0 rows shorter than a window that lie across two: every row's masked sums cost more than the fetch (4096 + 2048 x 1280 at eight
+//   rows 10.4 us there, 14.5 here).
+// * As many rows to an entry as a pass takes, but fewer while the entries' windows leave waves without two (one under bf16 rows of
+//   K-quants): three products of 512 x 1024 Q8_0 at eight rows 7.1 us as one entry each, 6.1 as four of two rows; 512 + 512 x 3072 Q4_K at
+//   five 6.9 and 5.8, Q6_K at six 7.7 and 7.2.  No entry mostly of repeated rows, and not three rows where four were: the entries' fixed cost is 0.1 us each.
 template <int TYPE, bool X_BF16>
-uint32_t flat_jobs_rows_take(const GemvArgs* jobs, uint32_t n_jobs, uint32_t cus) {
+uint32_t flat_jobs_rows_take(const GemvArgs* jobs, uint32_t n_jobs, uint32_t cus, uint64_t lane_steps, uint32_t row_steps) {
     const uint32_t m = jobs[0].pairs;
     if (m < (TYPE == HQ_Q4_K || TYPE == HQ_Q4_0 ? 3u : 2u) || m > 8u || (TYPE == HQ_Q4_0 && X_BF16)) return 0;
     uint32_t most = m;
+    uint64_t windows = 0;
+    bool ragged = false;  // short rows that lie across windows
     for (uint32_t i = 0; i < n_jobs; ++i) {
         const GemvArgs& j = jobs[i];
         if (j.x2 || j.ids || j.route_logits || j.pairs != m) return 0;
@@ -1586,9 +1604,21 @@ uint32_t flat_jobs_rows_take(const GemvArgs* jobs, uint32_t n_jobs, uint32_t cus
         if (!flat_takes<TYPE>(j.n, j.k, cus, lds) && !flat_takes_small<TYPE, X_BF16>(j.n, j.k, cus, lds)) return 0;
         const uint32_t fit = flat_rows_per_pass<TYPE, X_BF16>(j.k);
         most = fit < most ? fit : most;
+        ragged = ragged || (kUnitsPerWindow<TYPE> % (j.k / kUnitElems<TYPE>) != 0 && j.k / kUnitElems<TYPE> < kUnitsPerWindow<TYPE>);
+        windows += ((uint64_t)j.n * (j.k / kUnitElems<TYPE>) + kUnitsPerWindow<TYPE> - 1) / kUnitsPerWindow<TYPE>;
     }
-    const uint32_t groups = (m + most - 1u) / most;
-    return n_jobs * groups <= MAX_FLAT_JOBS && most >= 2u ? (m + groups - 1u) / groups : 0u;
+    const uint32_t groups = (m + most - 1u) / most, per = (m + groups - 1u) / groups;
+    if (n_jobs * groups > MAX_FLAT_JOBS || most < 2u) return 0;
+    if (n_jobs * m <= MAX_FLAT_JOBS && windows * m < (kBlock32<TYPE> ? 24u : 8u) * cus) return 0;
+    if (TYPE == HQ_Q4_0 && ragged && windows >= 10u * cus) return 0;
+    if (kBlock32<TYPE> ? lane_steps + row_steps < 4u : X_BF16 && 2u * (lane_steps + row_steps) < 2u + m) return 0;
+    const uint64_t fill = (X_BF16 && !kBlock32<TYPE> ? 1u : 2u) * (uint64_t)cus * kFlatRowsWaves<TYPE> / windows;
+    const uint32_t by_two = m == 7u ? 4u : m / 2u;  // (three rows or five as two and one: 0.95 .. 1.02 of the time, up to 1.2)
+    for (uint32_t g = fill < by_two ? (uint32_t)fill : by_two; g > groups; --g) {
+        const uint32_t fewer = (m + g - 1u) / g;
+        if (g * fewer <= m + 1u && 3u * fewer <= 2u * per) return fewer;
+    }
+    return per;
 }
 template <int TYPE, bool X_BF16, int NR = kFlatMaxRows<TYPE, X_BF16>>
 int launch_flat_jobs_rows(hipStream_t s, const GemvArgs* jobs, uint32_t n_jobs, uint32_t per, uint32_t cus) {
@@ -1596,31 +1626,30 @@ int launch_flat_jobs_rows(hipStream_t s, const GemvArgs* jobs, uint32_t n_jobs, 
         if (per < (uint32_t)NR) return launch_flat_jobs_rows<TYPE, X_BF16, NR - 1>(s, jobs, n_jobs, per, cus);
     constexpr uint32_t W = kFlatRowsWaves<TYPE>, UE = kUnitElems<TYPE>;
     FJobsRows js{};
-    FJobs& fj = js.f;
+    js.count = n_jobs;
+    js.m = jobs[0].pairs;
+    js.per = per;
     size_t lds = 81 * 1024;  // more than half a CU's LDS: one workgroup per CU
-    const uint32_t groups = (jobs[0].pairs + per - 1u) / per;
+    const uint32_t groups = (js.m + per - 1u) / per;
     uint64_t total = 0, sofar = 0;
-    for (uint32_t i = 0; i < n_jobs; ++i) total += (uint64_t)groups * jobs[i].n * (jobs[i].k / UE);
+    for (uint32_t i = 0; i < n_jobs; ++i) total += (uint64_t)jobs[i].n * (jobs[i].k / UE);
+    uint32_t at = 0, end = 0;
     for (uint32_t i = 0; i < n_jobs; ++i) {
         const GemvArgs& j = jobs[i];
         const size_t l = (size_t)NR * FlatX<TYPE, X_BF16>::lds_bytes(j.k);
         lds = l > lds ? l : lds;
-        for (uint32_t r = 0; r < j.pairs; r += per) {
-            const uint32_t q = fj.count++;
-            sofar += (uint64_t)j.n * (j.k / UE);
-            uint32_t end = (uint32_t)((sofar * cus + total / 2) / total);
-            if (end <= fj.first[q]) end = fj.first[q] + 1u;
-            fj.first[q + 1u] = end;
-            js.rows[q] = j.pairs - r < per ? j.pairs - r : per;
-            float* y = j.y + (size_t)r * j.n;
-            fj.j[q] = FArgs{static_cast<const uint8_t*>(j.x) + (size_t)r * j.k * (X_BF16 ? 2 : 4), j.w, j.w, y, y, j.n, j.k, 1u, 0u,
-                            flat_geom(j.k, UE, kUnitsPerWindow<TYPE>, j.n, 1, (end - fj.first[q]) * W), TYPE == HQ_Q6_K ? N4 : M4,
-                            TYPE == HQ_Q5_K ? M1 : TYPE == HQ_Q6_K ? N2 : M2, MAGIC};
-        }
+        sofar += (uint64_t)j.n * (j.k / UE);
+        const uint32_t upto = (uint32_t)((sofar * (cus / groups) + total / 2) / total);
+        js.share[i] = upto > end ? upto - end : 1u;
+        end += js.share[i];
+        js.first[i] = at;
+        at += groups * js.share[i];
+        js.j[i] = FArgs{j.x, j.w, j.w, j.y, j.y, j.n, j.k, 1u, 0u, flat_geom(j.k, UE, kUnitsPerWindow<TYPE>, j.n, 1, js.share[i] * W),
+                        TYPE == HQ_Q6_K ? N4 : M4, TYPE == HQ_Q5_K ? M1 : TYPE == HQ_Q6_K ? N2 : M2, MAGIC};
     }
     auto kern = gemv_flat_jobs_rows_kernel<TYPE, X_BF16, NR>;
     if (int rc = ensure_lds_limit(reinterpret_cast<const void*>(kern), lds, "hipFuncSetAttribute(gemv flat jobs rows LDS)")) return rc;
-    hipLaunchKernelGGL(kern, dim3(fj.first[fj.count]), dim3(64 * W), lds, s, js);
+    hipLaunchKernelGGL(kern, dim3(at), dim3(64 * W), lds, s, js);
     return check_launch("gemv flat jobs rows kernel launch");
 }
 
@@ -1815,13 +1844,17 @@ int launch_jobs_t(hipStream_t s, const GemvArgs* jobs, uint32_t n_jobs) {
     constexpr bool PAIR = X_BF16 && !kBlock32<TYPE>;
     KJobs js{};
     size_t lds = 0;
-    uint64_t slots = 0;
+    uint64_t slots = 0, lane_steps = 0;  // of gemv_jobs_kernel; the steps that a lane takes over a row
+    uint32_t row_steps = 0;
     for (uint32_t i = 0; i < n_jobs; ++i) {
         size_t l;
         uint64_t sl;
         if (int rc = plan_job<TYPE, X_BF16>(jobs[i], &js.j[i], &l, &sl)) return rc;
         lds = l > lds ? l : lds;
         slots += sl;
+        const uint32_t steps = (jobs[i].k / Lane<TYPE>::kElems + (1u << js.j[i].log_l) - 1u) >> js.j[i].log_l;
+        lane_steps += sl * steps;
+        row_steps = steps > row_steps ? steps : row_steps;
     }
     uint32_t cus = 0;
     if (int rc = cu_count(&cus)) return rc;
@@ -1841,7 +1874,7 @@ int launch_jobs_t(hipStream_t s, const GemvArgs* jobs, uint32_t n_jobs) {
             flat_takes<TYPE>((uint64_t)j0.n * 2, j0.k, cus, FlatX<TYPE, X_BF16>::lds_bytes(j0.k)))
             return launch_flat_passes<TYPE, X_BF16>(s, j0.x, j0.w, j1.w, j0.y, j1.y, j0.pairs, j0.n, j0.k, 2, cus);
     }
-    if (const uint32_t per = flat_jobs_rows_take<TYPE, X_BF16>(jobs, n_jobs, cus)) return launch_flat_jobs_rows<TYPE, X_BF16>(s, jobs, n_jobs, per, cus);
+    if (const uint32_t per = flat_jobs_rows_take<TYPE, X_BF16>(jobs, n_jobs, cus, lane_steps / (4ull * cus), row_steps)) return launch_flat_jobs_rows<TYPE, X_BF16>(s, jobs, n_jobs, per, cus);
     if (flat_jobs_take<TYPE, X_BF16>(jobs, n_jobs, cus)) return launch_flat_jobs<TYPE, X_BF16>(s, jobs, n_jobs, cus);
     const uint64_t per_simd = slots / (4ull * cus);
     if (per_simd >= 8) return launch_j<TYPE, X_BF16, PAIR, 4, 4>(s, js, n_jobs, lds);

@@ -165,6 +165,34 @@ def test_batch_of_dense_products_of_the_same_rows_matches_oracle(oracle, dev, t,
     test_batch_of_dense_products_matches_oracle(oracle, dev, t, xdt, [(n, k, m) for n, k in shapes])
 
 
+@pytest.mark.parametrize("t,xdt,m,shapes,rows", [  # rows of an entry; 0: an entry per row; -1: not on shares of the flat walk
+    (HQ_Q8_0, "f32", 8, [(512, 1024)] * 3, 2), (HQ_Q6_K, "f32", 5, [(512, 1024)] * 3, 3), (HQ_Q4_K, "f32", 7, [(600, 2816), (2050, 1280)], 2),
+    (HQ_Q8_0, "bf16", 7, [(515, 2816), (130, 1280)], 2), (HQ_Q4_0, "f32", 7, [(1030, 2048), (520, 2048)], 4),
+    (HQ_Q5_K, "bf16", 8, [(1027, 2816), (260, 2816), (260, 2816)], 3), (HQ_Q4_K, "f32", 7, [(3072, 1280), (3072, 1280), (2050, 1280)], 4),
+    (HQ_Q8_0, "f32", 2, [(512, 1024)] * 3, 0), (HQ_Q6_K, "f32", 2, [(384, 3072), (385, 2048)], 0),
+    (HQ_Q4_K, "bf16", 7, [(768, 768), (300, 768)], -1), (HQ_Q4_0, "f32", 8, [(4096, 1280), (2050, 1280)], -1),
+])
+def test_entries_of_a_batch_of_several_rows(oracle, dev, t, xdt, m, shapes, rows):
+    """A batch whose entries hold fewer rows than a pass takes, the last one of each product fewer still; and the batches that go to
+    the kernels beside it."""
+    jobs, refs = [], []
+    for i, (n, k) in enumerate(shapes):
+        blocks, x = oracle.quantize(weights(n + k + i, n, k), k, t, threads=8), acts(m + k + i, m, k)
+        xd = torch.from_numpy(x).to(dev)
+        if xdt == "bf16":
+            xd, x = xd.to(torch.bfloat16), oracle.f32_to_bf16_bits(x)
+        refs.append(oracle.qmatmul_f64(x, blocks, m, n, k, t))
+        jobs.append(ops.QmatmulJob(xd, torch.from_numpy(blocks).to(dev), torch.full((m, n), float("nan"), device=dev), m, n, k))
+    call = lambda: ops.quantized_matmul_batch_ggml(jobs, t)  # noqa: E731
+    call()
+    for j, ref in zip(jobs, refs):
+        assert_matmul_close(j.output.cpu().numpy(), ref, f"batch entries t={t} {xdt} {m}x{j.n}x{j.k}")
+    (name,) = launched_kernels(call)
+    form = f"ILi{t}ELb{int(xdt == 'bf16')}E"
+    want = {0: f"gemv_flat_jobs_kernel{form}", -1: f"gemv_jobs_kernel{form}"}.get(rows, f"gemv_flat_jobs_rows_kernel{form}Li{rows}E")
+    assert want in name, name
+
+
 @pytest.mark.parametrize("t,n,k,m", [
     # super-tasks of four rows, two or three to a wave: pairs, a last one by itself, and a ragged end
     (HQ_Q6_K, 28001, 2816, 3), (HQ_Q6_K, 28001, 2816, 6), (HQ_Q6_K, 28003, 5120, 5), (HQ_Q5_K, 28003, 5120, 5), (HQ_Q4_K, 28003, 5120, 6),
