@@ -1978,17 +1978,21 @@ bool gemv_flat_rows_preferred(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint
 }
 
 // Rows of Q8_0 over a matrix of ordinary size in one pass of the flat walk, where the kernel of small batches (gemvr32.hip) stages k in
-// chunks and meets its barriers once per 2048 of them; both have exact products.  us per layer of q / k / v and the output projection,
-// that kernel / the walk: n 2816 x k 8192 at 2 / 4 f32 rows 26.5 / 20.3 and 33.6 / 27.1, bf16 at 3 / 6 30.6 / 22.7 and 43.6 / 37.9; 2048 x 4096 at
-// 4 / 8 16.2 / 14.2 and 22.8 / 21.4; two passes of 5120 x 6144 at 8 rows 50.9 / 54.9.  Against matrices of sixteen weight rows per CU and
-// more the walk loses from four rows on (4096 x 4096 at 2 / 4 / 8 rows 19.7 / 18.8, 24.1 / 24.3, 34.4 / 35.6).
+// chunks and meets its barriers once per 2048 of them; both have exact products.  us, that kernel / the walk, f32 rows (bf16 the same):
+// 2816 x 8192 at 2 / 4 15.7 / 8.4 and 18.3 / 11.0; 2048 x 4096 at 4 / 8 8.9 / 7.3 and 12.1 / 10.8; 5120 x 6144 at 3 14.3 / 11.3; two passes of it at 8
+// 21.3 / 23.  Against matrices of sixteen weight rows per CU and more the walk loses from four rows on (4096 x 4096 at 2 / 4 / 8 7.8 / 7.1,
+// 9.3 / 9.4, 13.0 / 14.1), of twelve at eight rows (4064 x 3072 12.7 / 13.7, 3072 x 3072 11.8 / 11.4).  One chunk: 2048 x 2048 at 2 / 5 / 7
+// rows 4.8 / 4.6, 7.1 / 6.4, 7.1 / 7.9; 1024 x 2048 at 7 / 8 7.0 / 6.6, 7.0 / 7.3; 3072 x 2048 at 2 / 4 4.9 / 5.2, 5.7 / 6.5; 4096 x 2048 at 2 / 3
+// 5.0 / 5.7, 5.7 / 6.5; 3072 x 1024 at 3 / 4 5.3 / 5.0, 5.3 / 5.6, 8160 x 1024 at 2 / 3 5.5 / 5.8, 7.0 / 6.5.
 bool gemv_q80_rows_walked(hq_act_dtype xdt, uint32_t m, uint32_t n, uint32_t k) {
     uint32_t cus = 0;
     if (m < 2 || n >= 8192 || cu_count(&cus)) return false;
     auto go = [&](auto bf) {
         constexpr bool BF = decltype(bf)::value;
         const size_t lds = FlatX<HQ_Q8_0, BF>::lds_bytes(k);
-        return m <= flat_rows_per_pass<HQ_Q8_0, BF>(k) && (m <= 3u || n < 16u * cus) &&
+        const bool ahead = k > 2048u ? m <= 3u || n <= (m < 8u ? 16u * cus - 1u : 12u * cus)
+                                     : m <= 3u ? (uint64_t)n * k <= (1u << 22) || (m == 3u && k <= 1024u) : m <= 7u && n <= (m < 7u ? 8u : 4u) * cus;
+        return m <= flat_rows_per_pass<HQ_Q8_0, BF>(k) && ahead &&
                (flat_takes<HQ_Q8_0>(n, k, cus, lds) || flat_takes_small<HQ_Q8_0, BF>(n, k, cus, lds));
     };
     return xdt == HQ_BF16 ? go(std::true_type{}) : go(std::false_type{});

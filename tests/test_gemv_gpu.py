@@ -193,6 +193,24 @@ def test_entries_of_a_batch_of_several_rows(oracle, dev, t, xdt, m, shapes, rows
     assert want in name, name
 
 
+@pytest.mark.parametrize("n,k,m,walk", [(2048, 2048, 3, True), (2080, 2048, 3, False), (4064, 1024, 2, True), (2048, 2048, 6, True), (2050, 1536, 6, False),
+                                        (1024, 2048, 7, True), (1030, 2048, 7, False), (512, 1024, 8, False), (4095, 2304, 7, True),
+                                        (4096, 2304, 4, False), (4096, 2304, 3, True), (3072, 2560, 8, True), (3073, 2560, 8, False)])
+@pytest.mark.parametrize("xdt", ["bf16", "f32"])
+def test_q8_0_rows_on_either_side_of_the_walk(oracle, dev, xdt, n, k, m, walk):
+    """Several rows over Q8_0 matrices at the lines between the flat walk and the kernel of small batches."""
+    blocks, x = oracle.quantize(weights(n + m, n, k), k, HQ_Q8_0, threads=8), acts(k + m, m, k)
+    xd = torch.from_numpy(x).to(dev)
+    if xdt == "bf16":
+        xd, x = xd.to(torch.bfloat16), oracle.f32_to_bf16_bits(x)
+    w, y = torch.from_numpy(blocks).to(dev), torch.full((m, n), float("nan"), device=dev)
+    call = lambda: ops.quantized_matmul_ggml(xd, w, y, GgmlQuantizedMatmulParams(m, n, k, HQ_Q8_0))  # noqa: E731
+    call()
+    assert_matmul_close(y.cpu().numpy(), oracle.qmatmul_f64(x, blocks, m, n, k, HQ_Q8_0), f"q8_0 rows {xdt} {m}x{n}x{k}")
+    names = launched_kernels(call)
+    assert len(names) == 1 and ("gemv_flat_rows_kernel" in names[0]) == (walk and (xdt == "f32" or k >= 2048)), names
+
+
 @pytest.mark.parametrize("t,n,k,m", [
     # super-tasks of four rows, two or three to a wave: pairs, a last one by itself, and a ragged end
     (HQ_Q6_K, 28001, 2816, 3), (HQ_Q6_K, 28001, 2816, 6), (HQ_Q6_K, 28003, 5120, 5), (HQ_Q5_K, 28003, 5120, 5), (HQ_Q4_K, 28003, 5120, 6),
