@@ -592,6 +592,31 @@ def test_mul_mat_id_swiglu_grouped(oracle, dev, t, xdt, E, n, k, T, K):
     assert np.sqrt(np.mean((got - ref) ** 2)) <= 1.5e-3 * np.sqrt(np.mean(ref * ref))
 
 
+@pytest.mark.parametrize("t", [HQ_Q8_0, HQ_Q4_0])
+@pytest.mark.parametrize("E,n,k,T,own", [(16, 2050, 32, 1800, 1), (16, 2050, 96, 1800, 1), (24, 2050, 736, 1501, 1), (16, 2050, 736, 500, 0),
+                                         (40, 2050, 1056, 1100, 1), (60, 2050, 1056, 1700, 0)])
+def test_mul_mat_id_exact_tiles_of_own_blocks(dev, t, E, n, k, T, own):
+    """The exact grouped form over f32 rows in tiles of 64 where a lane fetches its own blocks (one block, an odd number of them, whole
+    stages) and on the other side of the lines: against float64 products of the dequantised weights."""
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(E + k)
+    w = ops.quantize_ggml(torch.randn(E * n * k, generator=gen, device=dev).mul_(0.02), k, t)
+    x = torch.randn(T, k, generator=gen, device=dev)
+    ids = torch.randint(0, E, (T,), generator=gen, device=dev, dtype=torch.int32)
+    p = GgmlQuantizedMatmulIdParams(T, 1, n, k, E, n * ops.ggml_row_bytes(t, k), t)
+    scratch = torch.empty(ops.quantized_matmul_id_workspace_bytes(p), dtype=torch.uint8, device=dev)
+    y = torch.full((T, n), float("nan"), device=dev)
+    call = lambda: ops.quantized_matmul_id_ggml(x, w, ids, y, p, scratch=scratch)  # noqa: E731
+    call()
+    ref, deq = torch.empty(T, n, dtype=torch.float64, device=dev), ops.dequantize_ggml(w, E * n * k, t).view(E, n, k)
+    for e in range(E):
+        ref[ids == e] = x[ids == e].double() @ deq[e].double().T
+    assert_matmul_close(y.cpu().numpy(), ref.cpu().numpy(), f"exact tiles t={t} E={E} {T}x{n}x{k}")
+    assert float((y.double() - ref).norm() / ref.norm()) <= 3e-7  # f32 products and sums (1e-7 observed)
+    names = launched_kernels(call)
+    assert any(f"grouped_exact_kernelILi{t}ELi2ELi3ELb{1 - own}E" in s for s in names), names
+
+
 @pytest.mark.parametrize("t", [HQ_Q4_K, HQ_Q5_K])
 @pytest.mark.parametrize("rows", [(95, 96, 97, 1, 33), (193, 0, 64, 32, 3)])
 def test_mul_mat_id_swiglu_grouped_at_tile_edges(oracle, dev, t, rows):
