@@ -637,6 +637,30 @@ def test_mul_mat_id_swiglu_grouped_at_tile_edges(oracle, dev, t, rows):
     assert torch.equal(y, sep)
 
 
+@pytest.mark.parametrize("t", [HQ_Q4_K, HQ_Q5_K])
+@pytest.mark.parametrize("rows,n,mt", [((97, 96, 95, 1, 33), 5128, 3), ((193, 0, 64, 32, 3), 5128, 3), ((129, 128, 20, 65, 1), 5128, 3),
+                                       ((160, 66, 40, 30, 31), 5128, 3), ((97, 64, 96, 66, 20), 136, 2)])
+def test_mul_mat_id_swiglu_grouped_rows_dealt_out(oracle, dev, t, rows, n, mt):
+    """Tiles of 96 that an expert's rows are dealt out to evenly, run as 64 rows where they hold no more, and the tiles of 64 that few
+    workgroups keep: the bits of two grouped calls followed by silu_mul."""
+    E, k, T = len(rows), 256, sum(rows)
+    gate, _, _, xd, p = _grouped_setup(oracle, dev, t, E, n, k, T, 1, "f32", seed=13)
+    up, _, _, _, _ = _grouped_setup(oracle, dev, t, E, n, k, T, 1, "f32", seed=14)
+    ids = np.random.default_rng(15).permutation(np.repeat(np.arange(E, dtype=np.int32), rows))
+    gd, ud, idd = torch.from_numpy(gate).to(dev), torch.from_numpy(up).to(dev), torch.from_numpy(ids).to(dev)
+    scratch = torch.empty(ops.quantized_matmul_id_swiglu_workspace_bytes(p), dtype=torch.uint8, device=dev)
+    yg, yu = torch.empty(T, n, device=dev), torch.empty(T, n, device=dev)
+    ops.quantized_matmul_id_ggml(xd, gd, idd, yg, p, scratch=scratch)
+    ops.quantized_matmul_id_ggml(xd, ud, idd, yu, p, scratch=scratch)
+    sep, y = torch.empty_like(yg), torch.full((T, n), float("nan"), device=dev)
+    ops.dispatch_silu_mul(yg, yu, sep)
+    call = lambda: ops.quantized_matmul_id_swiglu_ggml(xd, gd, ud, idd, y, p, scratch)  # noqa: E731
+    call()
+    assert torch.equal(y, sep)
+    names = launched_kernels(call)
+    assert any(f"grouped_gemm_kernelILi{t}ELi{mt}ELb1E" in s for s in names), names
+
+
 def test_mul_mat_id_swiglu_has_no_form_for_other_types_and_small_calls(dev):
     p = GgmlQuantizedMatmulIdParams(64, 4, 128, 512, 8, 128 * ops.ggml_row_bytes(HQ_Q6_K, 512), HQ_Q6_K)
     assert ops.quantized_matmul_id_workspace_bytes(p) > 0 and ops.quantized_matmul_id_swiglu_workspace_bytes(p) == 0
