@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 import torch
 
-from _util import acts, assert_matmul_close, weights
+from _util import acts, assert_matmul_close, launched_kernels, weights
 from hf2q_amd import ops
 from hf2q_amd.ops import HQ_Q4_0, HQ_Q4_K, HQ_Q5_K, HQ_Q6_K, HQ_Q8_0, GgmlQuantizedMatmulParams
 
@@ -779,6 +779,38 @@ def test_moe_block_as_one_library_call_equals_the_dispatches_made_by_hand(oracle
     # too small a scratch is refused before anything runs
     with pytest.raises(ops.HqError):
         ops.moe_ffn_prefill(x, w, got2, scratch[:need - 256], residual=res)
+
+
+@pytest.mark.parametrize("t,td,E,K,T,SI,mt,mt_down", [
+    (HQ_Q4_K, HQ_Q6_K, 64, 4, 300, 256, 2, 2),  # tiles of 64 routed rows in both products; 44 shared rows in their last one
+    (HQ_Q4_K, HQ_Q4_K, 32, 4, 400, 256, 3, 4),  # of 96, and of 128 with 16 shared rows in their last one, run as 64
+    (HQ_Q5_K, HQ_Q4_0, 8, 4, 100, 256, 3, 4),   # the shared run of 100 as two tiles of 64 and 36
+    (HQ_Q5_K, HQ_Q8_0, 8, 4, 136, 256, 2, 4),   # eight shared rows in the last tiles
+    (HQ_Q4_K, HQ_Q5_K, 4, 2, 700, 256, 4, 8),   # of 128 and of 256
+    (HQ_Q6_K, HQ_Q6_K, 8, 4, 96, 256, 0, 0),    # a type without the gate + up + SwiGLU form: by itself
+    (HQ_Q4_K, HQ_Q4_K, 8, 4, 96, 512, 0, 0),    # wider than the routed experts: by itself
+])
+def test_shared_expert_inside_the_grouped_products(oracle, dev, t, td, E, K, T, SI, mt, mt_down):
+    """With kept row scales the shared expert's rows are tiles of the grouped products (no launch of a dense product), of every
+    height that those have; the bits are those of the block that runs it by itself."""
+    H, I = 512, 256
+    w = _moe_weights_mixed(oracle, dev, t, td, H, E, K, I, SI, seed=T)
+    x, res = torch.from_numpy(acts(31 + T, T, H)).to(dev), torch.from_numpy(acts(32, T, H)).to(dev)
+    scratch = torch.full((ops.moe_ffn_prefill_scratch_bytes(w, T, x.dtype),), 0xA5, dtype=torch.uint8, device=dev)
+    want, got = (torch.full((T, H), float("nan"), device=dev) for _ in range(2))
+    dense = lambda names: [s for s in names if "mid_gemm" in s or "tile_gemm" in s or "tile_prep" in s]  # noqa: E731
+    by_itself = lambda: ops.moe_ffn_prefill(x, w, want, scratch, residual=res)  # noqa: E731
+    by_itself()
+    assert dense(launched_kernels(by_itself))
+    w.prepare_prefill()
+    call = lambda: ops.moe_ffn_prefill(x, w, got, scratch, residual=res)  # noqa: E731
+    call()
+    assert torch.isfinite(got).all() and torch.equal(got, want)
+    names = launched_kernels(call)
+    assert bool(dense(names)) == (mt == 0), names
+    if mt:
+        assert any(f"grouped_gemm_kernelILi{t}ELi{mt}ELb1E" in s for s in names), names
+        assert any(f"grouped_gemm_kernelILi{td}ELi{mt_down}ELb0E" in s for s in names), names
 
 
 def test_moe_block_mixed_types_match_cpu_spec(oracle, dev):
