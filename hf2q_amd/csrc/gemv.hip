@@ -1209,8 +1209,8 @@ int launch_flat(hipStream_t s, const void* x, const uint8_t* w0, const uint8_t* 
 
 // NR activation rows in one pass of the flat walk: the weights are fetched and converted once for all of them (a pass per row
 // did both again), then bound by the LDS reads of the activations, four bytes per weight and row (two for bf16 pairs).
-// Gate + up + SwiGLU of 17408 x 5120 Q5_K, f32: 56 / 84 / 138 / 220 us at 2 / 3 / 5 / 8 rows as a pass per row -> 38 / 47 / 64 /
-// 107; Q4_K 12288 x 4096 bf16: 23 / 34 / 56 / 88 -> 17 / 21 / 27 / 38; Q8_0 37 / 55 / 91 / 145 -> 21 / 24 / 32 / 44.  One matrix,
+// Gate + up + SwiGLU of 17408 x 5120 Q5_K, f32: 56 / 84 / 138 / 220 us at 2 / 3 / 5 / 8 rows as a pass per row -> 39 / 42 / 55 /
+// 90; Q4_K 12288 x 4096 bf16: 23 / 34 / 56 / 88 -> 17 / 20 / 27 / 36; Q8_0 37 / 55 / 91 / 145 -> 23 / 27 / 34 / 46.  One matrix,
 // Q6_K 5120 x 6144 f32: 15 / 22 -> 10 / 12 at 2 / 3 rows.
 //
 // PAIRED (K-quants): two pieces meet every activation read from LDS (run_rows_paired), by twelve waves per CU; the number of matrices
@@ -1310,8 +1310,8 @@ __global__ __launch_bounds__((64 * kFlatRowsWaves<TYPE, PAIRED>)) void gemv_flat
 }
 
 // Two pieces at a time: both matrices' where there are two, else (three rows or more) where every wave has two super-tasks to
-// pair.  Gate + up at five f32 rows, Q5_K: 17408 x 5120 62 -> 51 us, 12288 x 4096 35 -> 31, 4101 x 2816 16.0 -> 13.3, at two 35 -> 32,
-// 21.2 -> 20.5, 9.1 -> 8.5; bf16 57 -> 50, 30 -> 27, 14.7 -> 13.5.  One matrix, Q6_K f32 28000 x 5120: 31 -> 32 at two rows, 48 -> 43 at five;
+// pair.  Gate + up at five f32 rows, Q5_K: 17408 x 5120 67 -> 55 us, 12288 x 4096 35.3 -> 31.6, 4101 x 2816 16.5 -> 13.3, at two 42 -> 39,
+// 21.4 -> 21.0, 9.8 -> 8.8; bf16 at five 57 -> 50, 30 -> 27, 14.7 -> 13.5.  One matrix, Q6_K f32 28000 x 5120: 31 -> 32 at two rows, 52 -> 48 at five;
 // 9216 x 4096 (three super-tasks a wave) 16.8 -> 16.1.  Q4_K / Q5_K at three rows, which unpaired have sixteen waves, from four
 // super-tasks a wave on: 9216 x 4096 Q4_K 10.9 and 11.7, 17408 x 2048 Q5_K 12.1 and 13.1, 12300 x 3584 13.1 and 12.2.
 // Q6_K under bf16 rows from four to six: 20 -> 23 us at two rows of 14336 x 4096, 31 -> 30 at five, and the registers of seven

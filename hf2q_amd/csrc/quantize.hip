@@ -92,9 +92,9 @@ __device__ __forceinline__ float code_of(float f) {
 // Bound by VALU instructions: a candidate costs eight per element for the sums (sub, mul, rndne, med3, mul, three fma)
 // and four for the error, over codes that stay in registers as floats.  The codes themselves are not kept: the best
 // candidate is remembered by its scale and minimum (`best`), from which qkx2_codes() works them out for the rare
-// super-block that needs them.  12288 x 4096, Q4_K 498 -> 397 us, Q5_K 406 -> 316, with an importance matrix 953 -> 741 and
-// 986 -> 732 (seventeen instructions and packed codes before; keeping x - min as well, for a round of 32 subtractions less,
-// leaves room for two waves per SIMD instead of three: 408 us).
+// super-block that needs them.  12288 x 4096, Q4_K 443 -> 334 us, Q5_K 353 -> 269, with an importance matrix 874 -> 632 and
+// 920 -> 637 (seventeen instructions and packed codes before; keeping x - min as well, for a round of 32 subtractions less,
+// leaves room for two waves per SIMD instead of three: 3 % slower).
 struct Candidate {
     float iscale, mn;
     bool flat;  // all values alike: every code is zero
@@ -490,7 +490,7 @@ __global__ __launch_bounds__(256) void quantize_q4_0_kernel(const float* __restr
 // common.rs:61-167 make_qx_quants with rmse_type = 1: n = 16, nmax = 32 for Q6_K (q6_k.rs:58; W: the sub-block's slice
 // of the importance matrix as the weights, else x^2), n = 32, nmax = 8 with weights for Q4_0's importance-matrix path
 // (q4_0.rs:75).  Six VALU instructions per element and candidate (mul, rndne, med3, mul, two fma; w and w * x are kept);
-// the best candidate is remembered by its scale, `best_iscale` (qx_codes() makes codes of it).  Q6_K 12288 x 4096: 272 -> 203 us
+// the best candidate is remembered by its scale, `best_iscale` (qx_codes() makes codes of it).  Q6_K 12288 x 4096: 241 -> 185 us
 // (eleven instructions and packed codes before).
 template <int N, int nmax, bool W, bool FAST>
 __device__ float qx_search_n(const float (&x)[N], const float* qw, float& best_iscale, bool& flat, bool& ok) {

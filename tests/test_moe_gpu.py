@@ -79,7 +79,7 @@ def test_dense_gemv_bf16(oracle, dev):
 @pytest.mark.parametrize("m,n,k", [(2048, 256, 2048), (100, 70, 528), (33, 1, 2048), (32, 33, 16)])
 def test_dense_bf16_product_of_many_rows(oracle, dev, m, n, k):
     """The router of a prefill chunk: many bf16 activation rows take the matrix-core form (exact products, f32 sums),
-    edges in every dimension; the pair form gives the same bits as two calls; f32 activations keep the GEMV form."""
+    edges in every dimension; the pair form gives the same bits as two calls; f32 activations take it as three bf16 terms."""
     w = oracle.bf16_bits_to_f32(oracle.f32_to_bf16_bits(weights(3 + n, n, k, 0.05)))
     xb = oracle.bf16_bits_to_f32(oracle.f32_to_bf16_bits(acts(4 + m, m, k)))
     wd = torch.from_numpy(w).to(dev).to(torch.bfloat16)
