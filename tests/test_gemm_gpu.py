@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 import torch
 
-from _util import acts, assert_matmul_close, assert_matmul_close_f16_tile, weights
+from _util import acts, assert_matmul_close, assert_matmul_close_f16_tile, launched_kernels, weights
 from hf2q_amd import ops
 from hf2q_amd.ops import HQ_Q4_0, HQ_Q4_K, HQ_Q5_K, HQ_Q6_K, HQ_Q8_0, GgmlQuantizedMatmulParams
 
@@ -73,6 +73,41 @@ def test_small_tiles_and_k_slices_match_f64_oracle(oracle, dev, t, m, n, k):
     assert_matmul_close_f16_tile(y, ref, f"small tiles t={t} {m}x{n}x{k}")
     y2, _ = _run(oracle, dev, t, "bf16", m, n, k)
     assert np.array_equal(y, y2)
+
+
+@pytest.mark.parametrize("t,m,n,k,at,own", [
+    (HQ_Q8_0, 9, 33003, 384, 0, True), (HQ_Q8_0, 32, 33003, 384, 2, True), (HQ_Q8_0, 33, 33003, 384, 0, False),
+    (HQ_Q4_0, 9, 33003, 384, 2, True), (HQ_Q4_0, 64, 33003, 896, 0, True), (HQ_Q4_0, 9, 33003, 256, 0, True),
+    (HQ_Q8_0, 17, 17000, 2560, 2, True), (HQ_Q4_0, 64, 17000, 2560, 0, True),  # two slices of k
+    (HQ_Q4_0, 17, 33003, 1024, 0, False),  # rows of whole half lines
+    (HQ_Q8_0, 17, 65537, 384, 0, False),  # three workgroups on a CU
+])
+def test_small_tiles_whose_lanes_fetch_their_own_blocks(dev, t, m, n, k, at, own):
+    """Two workgroups on some CUs: the lanes' own blocks or the hand-over through LDS, the bits of the same rows in matrices of at
+    most a workgroup per CU, which hand over; matrices on 4n and 4n + 2."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(n + k + m)
+    q = ops.quantize_ggml(torch.randn(n * k, generator=g, device=dev).mul_(0.05), k, t)
+    w = torch.zeros(q.numel() + 16, dtype=torch.uint8, device=dev)[at:at + q.numel()].copy_(q)
+    x = torch.randn(m, k, generator=g, device=dev)
+    rb = ops.ggml_row_bytes(t, k)
+
+    def product(rows, wr):
+        p = GgmlQuantizedMatmulParams(m, rows, k, t)
+        y = torch.full((m, rows), float("nan"), device=dev)
+        ws = torch.empty(ops.quantized_matmul_workspace_bytes(p, x.dtype), dtype=torch.uint8, device=dev)
+        call = lambda: ops.quantized_matmul_ggml(x, wr, y, p, ws)  # noqa: E731
+        call()
+        return y, [s for s in launched_kernels(call) if "mid_gemm_small_kernel" in s]
+
+    y, names = product(n, w)
+    assert names and f"mid_gemm_small_kernelILi{t}ELi2ELb{0 if own else 1}E" in names[0], names
+    at_most = 16384 if n < 32768 else 32768
+    for r0 in range(0, n, at_most):
+        rows = min(at_most, n - r0)
+        part, names = product(rows, w[r0 * rb:(r0 + rows) * rb])
+        assert f"mid_gemm_small_kernelILi{t}ELi2ELb1E" in names[0], names
+        assert torch.isfinite(part).all() and torch.equal(y[:, r0:r0 + rows], part)
 
 
 @pytest.mark.parametrize("t,k", [(HQ_Q6_K, 256), (HQ_Q6_K, 768), (HQ_Q8_0, 128), (HQ_Q8_0, 384), (HQ_Q4_0, 128), (HQ_Q4_0, 384)])
