@@ -19,6 +19,10 @@ const SOURCES: &[&str] = &[
     "gemm.hip",
     "gemm_f16.hip",
     "gemv.hip",
+    "gemvk.hip",
+    "gemvk_32.hip",
+    "gemvk_q45.hip",
+    "gemvk_q6.hip",
     "gemvm.hip",
     "gemvr32.hip",
     "gguf.hip",

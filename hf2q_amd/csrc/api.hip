@@ -240,6 +240,11 @@ int qmatmul_routes(hipStream_t stream, const void* x, hq_act_dtype xdt, const vo
     const size_t xrow_bytes = (size_t)k * (xdt == HQ_BF16 ? 2 : 4);
     for (uint32_t r0 = 0; r0 < m; r0 += kGemvMaxRows) {
         const uint32_t rows = m - r0 < kGemvMaxRows ? m - r0 : kGemvMaxRows;
+        if (gemv_krows_takes(t, xdt, rows, n, k, w_blocks)) {
+            const KRowsSeg seg{w_blocks, y + (size_t)r0 * n, n};
+            if (int rc = launch_gemv_krows(stream, static_cast<const uint8_t*>(x) + (size_t)r0 * xrow_bytes, xdt, rows, k, t, &seg, 1, false)) return rc;
+            continue;
+        }
         if ((gemv_rows_supported(t, rows, k) || gemv_rows_stream_fast(t, xdt, rows, n, k) || gemv_rows_stream_takes(t, xdt, rows, n, k)) &&
             !gemv_stream_passes_preferred(t, xdt, rows, n, k) && !gemv_flat_rows_preferred(t, xdt, rows, n, k)) {
             if (int rc = launch_gemv_rows(stream, static_cast<const uint8_t*>(x) + (size_t)r0 * xrow_bytes, xdt, w_blocks,
@@ -417,6 +422,23 @@ int hq_qmatmul_swiglu_ggml_ws(void* stream, const void* x, hq_act_dtype xdt, con
         return fail(HQ_ERR_INVALID_ARGUMENT, "%s: workspace of %zu bytes, %zu needed", fn, workspace ? workspace_bytes : (size_t)0, need);
     if (reinterpret_cast<uintptr_t>(workspace) % 256) return fail(HQ_ERR_INVALID_ARGUMENT, "%s: workspace must be 256-byte aligned", fn);
     return launch_gemm_f16_swiglu((hipStream_t)stream, x, xdt, w_gate, w_up, y, m, n, k, t, workspace, gate_row_scales, up_row_scales);
+}
+
+int hq_qmatmul_swiglu_rows_supported(uint32_t m, uint32_t n, uint32_t k, hq_ggml_type t, hq_act_dtype xdt, const void* w_gate, const void* w_up) {
+    if (!known_type(t) || (xdt != HQ_F32 && xdt != HQ_BF16) || !w_gate || !w_up) return 0;
+    return gemv_krows_swiglu_takes(t, xdt, m, n, k, w_gate, w_up) ? 1 : 0;
+}
+
+int hq_qmatmul_swiglu_rows(void* stream, const void* x, hq_act_dtype xdt, const void* w_gate, const void* w_up, float* y, uint32_t m, uint32_t n,
+                           uint32_t k, hq_ggml_type t) {
+    const char* fn = "hq_qmatmul_swiglu_rows";
+    if (int rc = check_matmul_common(fn, x, xdt, w_gate, y, n, k, t)) return rc;
+    if (int rc = check_matmul_common(fn, x, xdt, w_up, y, n, k, t)) return rc;
+    if (m == 0) return HQ_OK;
+    if (!gemv_krows_swiglu_takes(t, xdt, m, n, k, w_gate, w_up))
+        return fail(HQ_ERR_UNSUPPORTED, "%s: %u rows, %u x %u of type %d (hq_qmatmul_swiglu_rows_supported)", fn, m, n, k, (int)t);
+    const KRowsSeg seg[2] = {{w_gate, y, n}, {w_up, y, n}};
+    return launch_gemv_krows((hipStream_t)stream, x, xdt, m, k, t, seg, 2, true);
 }
 
 int hq_qmatmul_swiglu_decode_supported(uint32_t n, uint32_t k, hq_ggml_type t, hq_act_dtype xdt) {
@@ -676,6 +698,21 @@ int hq_qmatmul_batch_ggml(void* stream, const hq_qmatmul_job* jobs, uint32_t n_j
         }
         if (a.pairs == 0) continue;
         ga[live++] = a;
+    }
+    // dense products of the same few rows as one walk (two matrices of one shape are gate and up, which have the bits of
+    // hq_qmatmul_swiglu_decode)
+    if (live >= 2 && live <= 4) {
+        KRowsSeg seg[4];
+        uint32_t n_all = 0;
+        bool same = live > 2 || ga[0].n != ga[1].n;
+        for (uint32_t i = 0; i < live; ++i) {
+            const GemvArgs& a = ga[i];
+            same = same && !a.x2 && !a.ids && !a.route_logits && a.x == ga[0].x && a.k == ga[0].k && a.pairs == ga[0].pairs && a.n % 16u == 0 && is_aligned(a.w, 16);
+            n_all += a.n;
+            seg[i] = KRowsSeg{a.w, a.y, a.n};
+        }
+        if (same && gemv_krows_batch_takes(t, xdt, ga[0].pairs, n_all, ga[0].k))
+            return launch_gemv_krows((hipStream_t)stream, ga[0].x, xdt, ga[0].pairs, ga[0].k, t, seg, live, false);
     }
     return launch_gemv_jobs((hipStream_t)stream, ga, live, xdt, t);
 }

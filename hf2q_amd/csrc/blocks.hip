@@ -58,7 +58,12 @@ int dense_ffn_steps(void* stream, const void* x, hq_act_dtype xdt, const void* w
                     uint32_t inter, const DenseBufs& b) {
     if (m <= kDecodeRows) {
         // decode: gate + up + SwiGLU as one launch where the streaming GEMV takes the pair, else gate and up as one
-        // batched launch; then down (with the SwiGLU folded into its staging where that pays)
+        // batched launch; then down (with the SwiGLU folded into its staging where that pays).  Several rows over matrices that are
+        // large enough: gate + up + SwiGLU on the matrix cores.
+        if (hq_qmatmul_swiglu_rows_supported(m, inter, hidden, tg, xdt, wg, wu)) {
+            if (int rc = hq_qmatmul_swiglu_rows(stream, x, xdt, wg, wu, b.act, m, inter, hidden, tg)) return rc;
+            return hq_qmatmul_ggml(stream, b.act, HQ_F32, wd, out, m, hidden, inter, td);
+        }
         if (hq_qmatmul_swiglu_decode_supported(inter, hidden, tg, xdt)) {
             if (int rc = hq_qmatmul_swiglu_decode(stream, x, xdt, wg, wu, b.act, m, inter, hidden, tg)) return rc;
             return hq_qmatmul_ggml(stream, b.act, HQ_F32, wd, out, m, hidden, inter, td);

@@ -97,6 +97,18 @@ bool gemv_rows32_supported(hq_ggml_type t, uint32_t m, uint32_t k);
 int launch_gemv_rows32(hipStream_t s, const void* x, hq_act_dtype xdt, const void* w, float* y, uint32_t m, uint32_t n,
                        uint32_t k, hq_ggml_type t);
 
+// The same with the activations as MFMA operands in registers (gemvk.hip): matrices of one k over the same rows in one launch.
+struct KRowsSeg {
+    const void* w;
+    float* y;
+    uint32_t n;
+};
+bool gemv_krows_takes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32_t n, uint32_t k, const void* w);
+bool gemv_krows_swiglu_takes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32_t n, uint32_t k, const void* wg, const void* wu);
+bool gemv_krows_batch_takes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32_t n_all, uint32_t k);
+int launch_gemv_krows(hipStream_t s, const void* x, hq_act_dtype xdt, uint32_t m, uint32_t k, hq_ggml_type t, const KRowsSeg* seg, uint32_t nseg,
+                      bool swiglu);
+
 // MFMA GEMM for m > 8 (prefill).  gemm_supported() says whether (type, k) has a tile kernel.
 bool gemm_supported(hq_ggml_type t, uint32_t k);
 int launch_gemm(hipStream_t s, const void* x, hq_act_dtype xdt, const void* w, float* y, uint32_t m, uint32_t n,

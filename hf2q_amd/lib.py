@@ -71,6 +71,8 @@ SIGNATURES = {
     "hq_qmatmul_swiglu_ggml_ws": (_i32, [_vp, _vp, _i32, _vp, _vp, _vp, _vp, _vp, _u32, _u32, _u32, _i32, _vp, _sz]),
     "hq_qmatmul_swiglu_decode_supported": (_i32, [_u32, _u32, _i32, _i32]),
     "hq_qmatmul_swiglu_decode": (_i32, [_vp, _vp, _i32, _vp, _vp, _vp, _u32, _u32, _u32, _i32]),
+    "hq_qmatmul_swiglu_rows_supported": (_i32, [_u32, _u32, _u32, _i32, _i32, _vp, _vp]),
+    "hq_qmatmul_swiglu_rows": (_i32, [_vp, _vp, _i32, _vp, _vp, _vp, _u32, _u32, _u32, _i32]),
     "hq_qmatmul_perm021_ggml_workspace_bytes": (_sz, [_u32, _u32, _u32, _i32, _i32]),
     "hq_qmatmul_perm021_ggml_ws": (_i32, [_vp, _vp, _i32, _vp, _vp, _u32, _u32, _u32, _u32, _i32, _vp, _sz]),
     "hq_qmatmul_id_ggml_workspace_bytes": (_sz, [_u32, _u32, _u32, _u32, _u32, _u64, _i32]),

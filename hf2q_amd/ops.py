@@ -170,6 +170,19 @@ def quantized_matmul_swiglu_ggml(input: torch.Tensor, gate: torch.Tensor, up: to
         params.k, params.ggml_type, _dev(workspace, "workspace"), workspace.numel() * workspace.element_size()))
 
 
+def quantized_matmul_swiglu_rows_supported(params: GgmlQuantizedMatmulParams, act_dtype: torch.dtype, gate: torch.Tensor, up: torch.Tensor) -> bool:
+    xdt = HQ_BF16 if act_dtype == torch.bfloat16 else HQ_F32
+    return bool(_l.load().hq_qmatmul_swiglu_rows_supported(params.m, params.n, params.k, params.ggml_type, xdt, gate.data_ptr(), up.data_ptr()))
+
+
+def quantized_matmul_swiglu_rows(input: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, dst: torch.Tensor,
+                                 params: GgmlQuantizedMatmulParams) -> None:
+    """dst[m, n] = silu(gate . x) * (up . x) for several rows of a decode step as one launch on the matrix cores, for the sizes that
+    quantized_matmul_swiglu_rows_supported names."""
+    _l.check(_l.load().hq_qmatmul_swiglu_rows(_stream(), _dev(input, "input"), _act_dtype(input), _dev(gate, "gate"), _dev(up, "up"),
+                                              _dev(dst, "dst"), params.m, params.n, params.k, params.ggml_type))
+
+
 def quantized_matmul_swiglu_decode_supported(params: GgmlQuantizedMatmulParams, act_dtype: torch.dtype) -> bool:
     xdt = HQ_BF16 if act_dtype == torch.bfloat16 else HQ_F32
     return bool(_l.load().hq_qmatmul_swiglu_decode_supported(params.n, params.k, params.ggml_type, xdt))
@@ -859,6 +872,11 @@ def build_dense_ffn_layer_gpu_q_into(x: torch.Tensor, w: DenseFfnWeightsGpuQ, ga
         if m > _BATCH_MAX_DENSE_ROWS:
             raise ValueError(f"batched dense FFN: {m} rows (limit {_BATCH_MAX_DENSE_ROWS})")
         pgu = GgmlQuantizedMatmulParams(m, I, H, t)
+        if act_buf is not None and quantized_matmul_swiglu_rows_supported(pgu, x.dtype, w.gate_q, w.up_q):
+            # several rows: gate, up and the SwiGLU as one launch on the matrix cores
+            quantized_matmul_swiglu_rows(x, w.gate_q, w.up_q, act_buf, pgu)
+            quantized_matmul_ggml(act_buf, w.down_q, out, GgmlQuantizedMatmulParams(m, H, I, td))
+            return
         if act_buf is not None and quantized_matmul_swiglu_decode_supported(pgu, x.dtype):
             # gate, up and the SwiGLU as one launch for as many rows as a CU's LDS holds, then down over the f32 activations
             quantized_matmul_swiglu_decode(x, w.gate_q, w.up_q, act_buf, pgu)

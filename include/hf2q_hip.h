@@ -195,6 +195,14 @@ HQ_API int hq_qmatmul_swiglu_decode_supported(uint32_t n, uint32_t k, hq_ggml_ty
 HQ_API int hq_qmatmul_swiglu_decode(void* stream, const void* x, hq_act_dtype xdt, const void* w_gate, const void* w_up, float* y,
                              uint32_t m, uint32_t n, uint32_t k, hq_ggml_type t);
 
+/* The same for three to eight rows on the matrix cores, in sums of its own order (as exact as the walk above, whose cost grows with
+ * the rows); whether a size is taken, and is ahead, hq_qmatmul_swiglu_rows_supported() says (n a multiple of 16, k of 256, both
+ * matrices 16-byte aligned).  What hq_dense_ffn runs for such sizes. */
+HQ_API int hq_qmatmul_swiglu_rows_supported(uint32_t m, uint32_t n, uint32_t k, hq_ggml_type t, hq_act_dtype xdt, const void* w_gate,
+                                            const void* w_up);
+HQ_API int hq_qmatmul_swiglu_rows(void* stream, const void* x, hq_act_dtype xdt, const void* w_gate, const void* w_up, float* y, uint32_t m,
+                           uint32_t n, uint32_t k, hq_ggml_type t);
+
 /* y[m, n] = sum_k x[m, k] * W[n, k] with the activations stored heads-outermost, [k / head_dim][m][head_dim]
  * (the attention output of a batched prefill): element (row, kk) sits at ((kk / head_dim) * m + row) * head_dim +
  * kk % head_dim.  Replaces quantized_matmul_mm_tensor_perm021(enc, reg, dev, input, weight, dst,
@@ -453,7 +461,7 @@ HQ_API int hq_moe_ffn_prefill(void* stream, const hq_moe_ffn_layer* layer, const
 
 /* The dense SwiGLU FFN at ANY row count: out[m, hidden] = W_down . (silu(W_gate . x) * (W_up . x)), the sequence of calls
  * that stands for build_dense_ffn_layer_gpu_q (gpu_ffn.rs:1017-1351) with its buffers carved out of one caller scratch:
- *   up to 8 rows   gate + up + SwiGLU as one streaming launch (hq_qmatmul_swiglu_decode) and the down GEMV; for
+ *   up to 8 rows   gate + up + SwiGLU as one launch (hq_qmatmul_swiglu_rows or hq_qmatmul_swiglu_decode) and the down GEMV; for
  *                  matrices too small for that, gate and up as one batched launch and the down GEMV with the SwiGLU
  *                  folded into its staging (inter <= 8192) or behind hq_silu_mul;
  *   more           gate, the up projection finishing the gating in its epilogue (hq_qmatmul_gated_ggml_ws; where the tile

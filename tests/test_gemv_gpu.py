@@ -240,6 +240,94 @@ def test_rows_over_pairs_of_super_tasks(dev, t, n, k, m):
         assert torch.equal(y[:2], y2)
 
 
+def _rows_ref(dev, t, n, k, x, seed):
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(seed)
+    w = ops.quantize_ggml(torch.randn(n * k, generator=gen, device=dev).mul_(0.02), k, t)
+    return w, x.double() @ ops.dequantize_ggml(w, n * k, t).view(n, k).double().T  # (dequantised bit-exactly: tested above)
+
+
+# Products of a few rows with the activations in registers.  Their sums are f32: one rounding per block of 32 (16) weights inside the matrix
+# instruction, one per block behind it, and 8 + 16 + 3 for the super-blocks, waves and slices, of values that grow like the square root
+# of the blocks: 2^-24 * sqrt(96 + 27) = 6.6e-7 of the result at most.
+@pytest.mark.parametrize("t,xdt,m,n,k", [
+    # super-blocks that fill the waves unevenly: 4, 9, 11, 14 (two groups side by side on 12 waves of three), 16, 20, 24, 32, 36
+    (HQ_Q4_K, "bf16", 3, 16, 1024), (HQ_Q5_K, "bf16", 5, 48, 2304), (HQ_Q6_K, "bf16", 8, 4112, 2816), (HQ_Q4_K, "bf16", 7, 16416, 3584),
+    (HQ_Q6_K, "bf16", 4, 80, 4096), (HQ_Q5_K, "f32", 5, 4128, 5120), (HQ_Q8_0, "f32", 5, 4096, 6144), (HQ_Q4_0, "f32", 3, 4112, 8192),
+    (HQ_Q6_K, "f32", 5, 8208, 9216), (HQ_Q4_0, "bf16", 2, 4096, 2048), (HQ_Q8_0, "bf16", 6, 4112, 2816),
+    # f32 rows of one operand (3 + 1, 4 + 1) and of two (3 + 3, 4 + 3, 4 + 4)
+    (HQ_Q4_K, "f32", 4, 8192, 2816), (HQ_Q8_0, "f32", 6, 4112, 4096), (HQ_Q6_K, "f32", 7, 2064, 2816), (HQ_Q6_K, "f32", 8, 48, 4096),
+    # slices of k, of unequal lengths
+    (HQ_Q6_K, "f32", 5, 4112, 17408), (HQ_Q4_0, "bf16", 3, 2064, 14336), (HQ_Q8_0, "f32", 8, 32768, 5120),
+])
+def test_rows_with_activations_in_registers(dev, t, xdt, m, n, k):
+    x = torch.randn(m, k, generator=torch.Generator(device=dev).manual_seed(n + m), device=dev)
+    x = x.to(torch.bfloat16) if xdt == "bf16" else x
+    w, ref = _rows_ref(dev, t, n, k, x, k + m)
+    y = torch.full((m + 1, n), float("nan"), device=dev)
+    call = lambda: ops.quantized_matmul_ggml(x, w, y, GgmlQuantizedMatmulParams(m, n, k, t))  # noqa: E731
+    for _ in range(2):  # (a first slice overwrites what an earlier call left)
+        call()
+    assert torch.isfinite(y[:m]).all() and torch.isnan(y[m]).all()
+    assert ((y[:m] - ref).norm() / ref.norm()).item() <= 6.6e-7
+    assert all(f"krows_kernelILi{t}ELb{int(xdt == 'f32')}E" in s for s in launched_kernels(call))
+
+
+@pytest.mark.parametrize("t", ALL_TYPES)
+@pytest.mark.parametrize("xdt", ["bf16", "f32"])
+@pytest.mark.parametrize("m", [5, 8])
+def test_rows_in_registers_as_batches_and_pairs(dev, t, xdt, m):
+    """Three matrices of their own heights over the same rows, and gate + up + SwiGLU, against float64."""
+    ns, k = (4112, 528, 16), 2816
+    x = torch.randn(m, k, generator=torch.Generator(device=dev).manual_seed(m), device=dev)
+    x = x.to(torch.bfloat16) if xdt == "bf16" else x
+    mats = [_rows_ref(dev, t, n, k, x, n + m) for n in ns]
+    jobs = [ops.QmatmulJob(x, w, torch.full((m, n), float("nan"), device=dev), m, n, k) for n, (w, _) in zip(ns, mats)]
+    call = lambda: ops.quantized_matmul_batch_ggml(jobs, t)  # noqa: E731
+    call()
+    for j, (_, ref) in zip(jobs, mats):
+        assert ((j.output - ref).norm() / ref.norm()).item() <= 6.6e-7
+    if xdt == "bf16" or m == 5 or t != HQ_Q5_K:
+        (name,) = launched_kernels(call)
+        assert f"krows_kernelILi{t}E" in name, name
+    n = 4112
+    (wg, g), (wu, u) = mats[0], _rows_ref(dev, t, n, k, x, 7)
+    y, p = torch.full((m + 1, n), float("nan"), device=dev), GgmlQuantizedMatmulParams(m, n, k, t)
+    if t == HQ_Q4_K:
+        assert not ops.quantized_matmul_swiglu_rows_supported(GgmlQuantizedMatmulParams(m, n + 8, k, t), x.dtype, wg, wu)
+    assert ops.quantized_matmul_swiglu_rows_supported(p, x.dtype, wg, wu)
+    ops.quantized_matmul_swiglu_rows(x, wg, wu, y, p)
+    want = g / (1 + torch.exp(-g)) * u
+    # (the gating: silu has a derivative of 1.1 at most, and its own roundings are four of 2^-24)
+    assert ((y[:m] - want).norm() / want.norm()).item() <= 2 * 1.1 * 6.6e-7 + 4 * 2 ** -24 and torch.isnan(y[m]).all()
+
+
+@pytest.mark.parametrize("t,m", [(HQ_Q4_K, 5), (HQ_Q6_K, 5), (HQ_Q8_0, 5), (HQ_Q8_0, 8), (HQ_Q4_0, 8)])
+def test_rows_in_registers_keep_large_small_and_non_finite_values(dev, t, m):
+    """f32 rows are cut into three bf16 parts: rows beside one with an infinity or a NaN keep their bits, that one is not finite where it meets
+    it, and a power of two scales the result exactly."""
+    n, k = 4096, 4096
+    x = torch.randn(m, k, generator=torch.Generator(device=dev).manual_seed(t), device=dev)
+    w, _ = _rows_ref(dev, t, n, k, x, 3)
+    p = GgmlQuantizedMatmulParams(m, n, k, t)
+
+    def run(v):
+        y = torch.full((m, n), float("nan"), device=dev)
+        ops.quantized_matmul_ggml(v, w, y, p)
+        return y
+
+    y, z = run(x), torch.empty(m, n, device=dev)
+    assert "krows_kernel" in launched_kernels(lambda: ops.quantized_matmul_ggml(x, w, z, p))[0]
+    assert torch.equal(run(x * 2.0 ** 20), y * 2.0 ** 20) and torch.equal(run(x * 2.0 ** -40), y * 2.0 ** -40)
+    met = ops.dequantize_ggml(w, n * k, t).view(n, k)[:, 1000] != 0
+    keep = [i for i in range(m) if i != 2]
+    for bad in (float("inf"), float("-inf"), float("nan")):
+        xb = x.clone()
+        xb[2, 1000] = bad
+        yb = run(xb)
+        assert torch.equal(yb[keep], y[keep]) and not torch.isfinite(yb[2][met]).any()
+
+
 ID_CASES = [  # (E, n, k, T, K); k = 768, 2816, 1280: rows whose pieces no sixteen lanes divide (a ragged last step under bf16 rows)
     (8, 64, 512, 1, 2), (16, 512, 2048, 1, 8), (16, 2048, 512, 8, 1), (256, 128, 256, 8, 8), (4, 33, 768, 5, 3),
     (8, 48, 2816, 3, 2), (4, 40, 1280, 2, 4),
