@@ -590,6 +590,36 @@ def test_mul_mat_id_grouped_sparse_experts_skewed(oracle, dev, t):
     assert_matmul_close_f16_tile(y.cpu().numpy(), ref, f"grouped, sparse + skewed, t={t}")
 
 
+@pytest.mark.parametrize("t", [HQ_Q4_K, HQ_Q5_K, HQ_Q6_K, HQ_Q8_0, HQ_Q4_0])
+@pytest.mark.parametrize("rows,k,n,mt", [
+    ((1, 31, 32, 0, 33, 0, 0, 64, 0, 0), 256, 161, 2),      # tiles of 32 and 64 rows; one super-block; weight rows that end inside a wave
+    ((33, 65, 2, 0, 0, 32, 0, 0, 0), 768, 33, 2),           # an odd number of super-blocks: rows start at either half of a word
+    ((40, 1, 0, 0, 3), 1280, 97, 2),
+    ((64, 65, 128, 129, 32, 0, 1), 768, 130, 4),            # tiles of 128 rows, and of 64 at an expert's end
+])
+def test_mul_mat_id_grouped_at_tile_edges(oracle, dev, t, rows, k, n, mt):
+    """Rows per expert at the edges of the tiles that the grouped product picks, weights that start two bytes into a word of memory: the
+    products of the oracle, and the same bits from a stack that starts at a word."""
+    E, rng = len(rows), np.random.default_rng(k + n)
+    ids = rng.permutation(np.repeat(np.arange(E, dtype=np.uint32), rows))
+    T = ids.size
+    assert (2 if T <= E * (24 if t in (HQ_Q8_0, HQ_Q4_0) else 40) else 4 if T < 160 * E else 8) == mt
+    stack, _, xv, xd, p = _grouped_setup(oracle, dev, t, E, n, k, T, 1, "f32", seed=k)
+    scratch = torch.empty(ops.quantized_matmul_id_workspace_bytes(p), dtype=torch.uint8, device=dev)
+    sd, idd = torch.from_numpy(stack).to(dev), torch.from_numpy(ids.view(np.int32)).to(dev)
+    ys = []
+    for at in (0, 2):
+        if at and t in (HQ_Q4_K, HQ_Q5_K):
+            continue  # (their blocks are whole 16-byte pieces, and so is their alignment)
+        holder = torch.zeros(sd.numel() + 16, dtype=torch.uint8, device=dev)
+        holder[at:at + sd.numel()] = sd.flatten()
+        ys.append(torch.full((T, n), float("nan"), device=dev))
+        ops.quantized_matmul_id_ggml(xd, holder[at:at + sd.numel()], idd, ys[-1], p, scratch=scratch)
+    ref = oracle.qmatmul_id_f64(xv, stack, ids, T, 1, n, k, E, p.expert_stride, t)
+    assert_matmul_close_f16_tile(ys[0].cpu().numpy(), ref, f"grouped at tile edges t={t}")
+    assert all(torch.equal(y, ys[0]) for y in ys)
+
+
 @pytest.mark.parametrize("t", [HQ_Q4_K, HQ_Q6_K, HQ_Q8_0])
 @pytest.mark.parametrize("E,n,k,T,K", [(8, 128, 512, 64, 4), (4, 160, 256, 400, 3), (16, 64, 1024, 300, 1)])
 def test_mul_mat_id_grouped_with_prepared_weight_row_scales(oracle, dev, t, E, n, k, T, K):
