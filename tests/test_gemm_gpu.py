@@ -75,6 +75,31 @@ def test_small_tiles_and_k_slices_match_f64_oracle(oracle, dev, t, m, n, k):
     assert np.array_equal(y, y2)
 
 
+@pytest.mark.parametrize("t", [HQ_Q4_K, HQ_Q5_K, HQ_Q6_K, HQ_Q8_0, HQ_Q4_0])
+@pytest.mark.parametrize("m,n,k,height", [(257, 130, 256, 2), (321, 4097, 768, 2), (1000, 2300, 256, 4), (1025, 2049, 512, 4), (500, 12290, 256, 8)])
+def test_tile_height_above_256_rows(dev, t, m, n, k, height):
+    """Tiles of 64, 128 or 256 rows by the workgroups they make, ragged at both ends: the bits of the same rows 256 at a time, which are
+    one tile each."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(m + n)
+    w = ops.quantize_ggml(torch.randn(n * k, generator=g, device=dev).mul_(0.05), k, t)
+    x = torch.randn(m, k, generator=g, device=dev)
+
+    def product(xr):
+        y = torch.full((xr.shape[0], n), float("nan"), device=dev)
+        call = lambda: ops.quantized_matmul_ggml(xr, w, y, GgmlQuantizedMatmulParams(xr.shape[0], n, k, t))  # noqa: E731
+        call()
+        return y, call
+
+    y, call = product(x)
+    kind = "q4k" if t in (HQ_Q4_K, HQ_Q5_K) else "mid"
+    names = [s for s in launched_kernels(call) if "gemm" in s]
+    assert any(f"{kind}_gemm_small_kernelILi{t}ELi{height}E" in s for s in names) == (height < 8), names
+    for r0 in [*range(0, m - 255, 256), m - 256]:
+        assert torch.equal(y[r0:r0 + 256], product(x[r0:r0 + 256].contiguous())[0]), r0
+    assert torch.isfinite(y).all()
+
+
 @pytest.mark.parametrize("t,m,n,k,at,own", [
     (HQ_Q8_0, 9, 33003, 384, 0, True), (HQ_Q8_0, 32, 33003, 384, 2, True), (HQ_Q8_0, 33, 33003, 384, 0, False),
     (HQ_Q4_0, 9, 33003, 384, 2, True), (HQ_Q4_0, 64, 33003, 896, 0, True), (HQ_Q4_0, 9, 33003, 256, 0, True),
