@@ -596,10 +596,13 @@ def test_mul_mat_id_grouped_sparse_experts_skewed(oracle, dev, t):
     ((33, 65, 2, 0, 0, 32, 0, 0, 0), 768, 33, 2),           # an odd number of super-blocks: rows start at either half of a word
     ((40, 1, 0, 0, 3), 1280, 97, 2),
     ((64, 65, 128, 129, 32, 0, 1), 768, 130, 4),            # tiles of 128 rows, and of 64 at an expert's end
+    ((33, 20, 0, 0, 0), 128, 65, 2), ((40, 30, 0, 0, 0), 384, 130, 2), ((100, 60, 20), 640, 97, 4),  # Q8_0 / Q4_0: rows that end inside a fetch
 ])
 def test_mul_mat_id_grouped_at_tile_edges(oracle, dev, t, rows, k, n, mt):
     """Rows per expert at the edges of the tiles that the grouped product picks, weights that start two bytes into a word of memory: the
     products of the oracle, and the same bits from a stack that starts at a word."""
+    if k % oracle.BLOCK_ELEMS[t]:
+        pytest.skip("k is not a multiple of the block size")
     E, rng = len(rows), np.random.default_rng(k + n)
     ids = rng.permutation(np.repeat(np.arange(E, dtype=np.uint32), rows))
     T = ids.size
