@@ -233,6 +233,7 @@ bool f16_tile_route(uint32_t m, uint32_t k, hq_ggml_type t) {
 // All routes of the dense product; `workspace` is only read on the f16 tile route.
 int qmatmul_routes(hipStream_t stream, const void* x, hq_act_dtype xdt, const void* w_blocks, float* y, uint32_t m,
                    uint32_t n, uint32_t k, hq_ggml_type t, void* workspace, const float* w_scales = nullptr) {
+    if (gemv_krows_passes(t, xdt, m, n, k, w_blocks)) return launch_gemv_krows_passes(stream, x, xdt, w_blocks, y, m, n, k, t, nullptr);
     if (f16_tile_route(m, k, t)) return launch_gemm_f16_tile(stream, x, xdt, w_blocks, y, m, n, k, t, workspace, 0, w_scales);
     if (m > chunked_rows_limit(k, t) && gemm_supported(t, k)) return launch_gemm(stream, x, xdt, w_blocks, y, m, n, k, t);
     // kGemvMaxRows activation rows per launch: the small-batch kernel where it exists for the chunk, else one GEMV
@@ -392,6 +393,7 @@ int hq_qmatmul_gated_ggml_ws(void* stream, const void* x, hq_act_dtype xdt, cons
     if (!workspace || workspace_bytes < need)
         return fail(HQ_ERR_INVALID_ARGUMENT, "%s: workspace of %zu bytes, %zu needed", fn, workspace ? workspace_bytes : (size_t)0, need);
     if (reinterpret_cast<uintptr_t>(workspace) % 256) return fail(HQ_ERR_INVALID_ARGUMENT, "%s: workspace must be 256-byte aligned", fn);
+    if (gemv_krows_passes(t, xdt, m, n, k, w_blocks)) return launch_gemv_krows_passes((hipStream_t)stream, x, xdt, w_blocks, y, m, n, k, t, gate);
     return launch_gemm_f16_tile((hipStream_t)stream, x, xdt, w_blocks, y, m, n, k, t, workspace, 0, w_row_scales, gate);
 }
 

@@ -44,6 +44,7 @@ struct KRowsArgs {
     uint32_t kp, rg, ring;   // waves that share a group's k, groups side by side in a workgroup, slots of a wave's ring
     uint32_t base, extra;    // super-blocks per wave: nsb / kp, and the first nsb % kp waves one more
     uint32_t units, full, rem;  // groups of sixteen rows, all segments (swiglu: of one matrix); units over gridDim * rg, and the rest
+    const float* gate;       // may be null, laid out as y[0]: silu(gate) * product is stored
     uint32_t add, swiglu;    // add: products are added to y; swiglu: seg 0 = gate, seg 1 = up, y[0] = silu(gate) * up
     uint32_t nseg;
     const uint8_t* w[kKMaxSegs];
@@ -598,8 +599,12 @@ __global__ __launch_bounds__(64 * W) void krows_kernel(KRowsArgs a) {
                 uint32_t seg = 0, from = 0;
                 if (!a.swiglu)
                     while (seg + 1u < a.nseg && u >= a.end[seg]) from = a.end[seg++];
-                float* y = a.y[seg] + (size_t)row * a.n[seg] + (size_t)(u - from) * 16u + j;
-                *y = a.swiglu ? silu_mul_f32(held[i], v) : a.add ? *y + v : v;
+                const size_t at = (size_t)row * a.n[seg] + (size_t)(u - from) * 16u + j;
+                float* y = a.y[seg] + at;
+                if (a.swiglu || a.gate)
+                    *y = silu_mul_f32(a.swiglu ? held[i] : a.gate[at], v);
+                else
+                    *y = a.add ? *y + v : v;
             }
         }
     }

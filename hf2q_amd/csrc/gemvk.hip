@@ -86,7 +86,7 @@ bool gemv_krows_batch_takes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32
 }
 
 int launch_gemv_krows(hipStream_t s, const void* x, hq_act_dtype xdt, uint32_t m, uint32_t k, hq_ggml_type t, const KRowsSeg* seg, uint32_t nseg,
-                      bool swiglu) {
+                      bool swiglu, const float* gate) {
     uint32_t cus = 0;
     if (int rc = cu_count(&cus)) return rc;
     if (nseg == 0 || nseg > kKMaxSegs || (swiglu && nseg != 2)) return fail(HQ_ERR_INVALID_ARGUMENT, "k rows: %u matrices", nseg);
@@ -98,6 +98,7 @@ int launch_gemv_krows(hipStream_t s, const void* x, hq_act_dtype xdt, uint32_t m
     a.rowb = k / hq_block_elems(t) * hq_block_bytes(t);
     a.nseg = nseg;
     a.swiglu = swiglu;
+    a.gate = gate;
     for (uint32_t i = 0; i < nseg; ++i) {
         a.w[i] = static_cast<const uint8_t*>(seg[i].w);
         a.y[i] = seg[i].y;
@@ -106,7 +107,7 @@ int launch_gemv_krows(hipStream_t s, const void* x, hq_act_dtype xdt, uint32_t m
     }
     const bool f32 = xdt != HQ_BF16;
     const uint32_t per = krows_per_slice(nsb, f32, m);
-    if (swiglu && per < nsb) return fail(HQ_ERR_INVALID_ARGUMENT, "k rows: gate and up in slices of k");
+    if ((swiglu || gate) && per < nsb) return fail(HQ_ERR_INVALID_ARGUMENT, "k rows: gating in slices of k");
     for (uint32_t sb = 0; sb < nsb; sb += per) {
         a.sb0 = sb;
         a.nsb = nsb - sb < per ? nsb - sb : per;
@@ -120,6 +121,34 @@ int launch_gemv_krows(hipStream_t s, const void* x, hq_act_dtype xdt, uint32_t m
             case HQ_Q4_0: rc = launch_krows_q40(s, a, f32, cus); break;
         }
         if (rc) return rc;
+    }
+    return HQ_OK;
+}
+
+// Nine to sixteen rows of Q8_0 / Q4_0 / Q6_K (Q4_K and Q5_K take passes of eight anyway) as two passes of half of them: both find the weights in the
+// device's caches, and no tile of 64 rows is filled with 16.  us, a tile / two passes, as the calls follow each other (about 24 us is what the
+// host takes for a call): bf16 Q8_0 at 12 rows 4096 x 4096 27.3 / 23.9, 17408 x 5120 60.6 / 45.2, 151936 x 4096 325 / 234, Q4_0 5120 x 5120 30.3 / 24.0, 17408 x 5120 47.6 /
+// 42.3 (14336 x 5120 36.4 / 39.5), Q6_K 4096 x 4096 30.0 / 24.9 (14336 x 5120 37.8 / 45.4, 18944 x 3584 37.3 / 43.8); f32 at 9 / 16 Q8_0 4096 x 4096 27.9 / 25.5, 29.3 / 25.4,
+// 151936 x 4096 327 / 235, 327 / 257 (12288 x 4096 38.4 / 42.3), Q4_0 4096 x 4096 29.7 / 22.5, 29.5 / 26.3 (12288 x 4096 32 / 40), Q6_K 4096 x 4096 29.8 / 24.2, 27.8 / 29.7.
+// No less exact: these kernels' error is 2e-7 of the result at most, a tile rounds its weights to f16.
+bool gemv_krows_passes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32_t n, uint32_t k, const void* w) {
+    if (m <= 8 || m > 16 || (t != HQ_Q8_0 && t != HQ_Q4_0 && t != HQ_Q6_K)) return false;
+    const uint32_t half = (m + 1u) / 2u;
+    if (!gemv_krows_takes(t, xdt, half, n, k, w) || !gemv_krows_takes(t, xdt, m - half, n, k, w)) return false;
+    if (krows_per_slice(k / 256u, xdt != HQ_BF16, half) < k / 256u) return false;
+    const uint64_t weights = (uint64_t)n * k, M = 1u << 20;
+    if (xdt == HQ_BF16) return t == HQ_Q8_0 || (t == HQ_Q4_0 ? n <= 12288 || n > 16384 : weights <= 25 * M);
+    if (t == HQ_Q8_0) return n >= 32768 || (n >= 4096 && weights <= 16 * M);
+    return weights <= (t == HQ_Q4_0 && m <= 10 ? 25 : 16) * M && (t == HQ_Q4_0 || m <= 12);
+}
+
+int launch_gemv_krows_passes(hipStream_t s, const void* x, hq_act_dtype xdt, const void* w, float* y, uint32_t m, uint32_t n, uint32_t k, hq_ggml_type t,
+                             const float* gate) {
+    const uint32_t half = (m + 1u) / 2u;
+    for (uint32_t r0 = 0; r0 < m; r0 += half) {
+        const KRowsSeg seg{w, y + (size_t)r0 * n, n};
+        const uint8_t* xr = static_cast<const uint8_t*>(x) + (size_t)r0 * k * (xdt == HQ_BF16 ? 2 : 4);
+        if (int rc = launch_gemv_krows(s, xr, xdt, m - r0 < half ? m - r0 : half, k, t, &seg, 1, false, gate ? gate + (size_t)r0 * n : nullptr)) return rc;
     }
     return HQ_OK;
 }

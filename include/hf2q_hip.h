@@ -156,7 +156,7 @@ HQ_API int hq_qmatmul_ggml_ws(void* stream, const void* x, hq_act_dtype xdt, con
  * with `gate` the f32 output of the gate projection computed before it.  Replaces the second quantized_matmul_ggml
  * and the silu_mul of the dense FFN at prefill (gpu_ffn.rs:1236-1306): the stand-alone SwiGLU pass reads both
  * products and writes the activations (300 MB at 2048 x 12288, about 50 us); here the gate values are read while the
- * tiles are stored and the up product never goes to memory.  The bits of the separate calls.  Every weight type of
+ * products are stored and the up product never goes to memory.  The bits of the separate calls.  Every weight type of
  * the tile route, any token count above the small-batch kernels' -- except where the product is cut into slices of k
  * (up to 256 rows over few weight rows): hq_qmatmul_gated_ggml_workspace_bytes() is 0 there and the call returns
  * HQ_ERR_UNSUPPORTED.  y may be the gate buffer itself (every element is read before it is written, by the same lane).

@@ -273,6 +273,47 @@ def test_rows_with_activations_in_registers(dev, t, xdt, m, n, k):
     assert all(f"krows_kernelILi{t}ELb{int(xdt == 'f32')}E" in s for s in launched_kernels(call))
 
 
+@pytest.mark.parametrize("t,xdt,m,n,k,takes", [
+    (HQ_Q8_0, "bf16", 9, 4112, 2816, True), (HQ_Q8_0, "f32", 16, 4096, 4096, True), (HQ_Q4_0, "bf16", 15, 2064, 4096, True), (HQ_Q4_0, "f32", 10, 5120, 4096, True),
+    (HQ_Q6_K, "bf16", 16, 4096, 4096, True), (HQ_Q6_K, "f32", 9, 4096, 4096, True), (HQ_Q8_0, "bf16", 12, 12288, 1024, True), (HQ_Q4_0, "f32", 9, 8192, 1024, True),
+    (HQ_Q8_0, "bf16", 17, 4112, 2816, False), (HQ_Q4_0, "f32", 16, 12288, 4096, False), (HQ_Q6_K, "bf16", 12, 14336, 5120, False), (HQ_Q6_K, "f32", 13, 4096, 4096, False),
+])
+def test_rows_in_registers_in_two_passes(dev, t, xdt, m, n, k, takes):
+    """Nine to sixteen rows: the bits of the two halves' own calls within the bound above, one matrix row past or short of whole groups
+    and the sizes beyond the rule on the tiles; where the tile has a gated form, the bits of product and silu_mul, also in place."""
+    x = torch.randn(m, k, generator=torch.Generator(device=dev).manual_seed(n + m), device=dev)
+    x = x.to(torch.bfloat16) if xdt == "bf16" else x
+    w, ref = _rows_ref(dev, t, n, k, x, k + m)
+
+    def product(xr):
+        y = torch.full((xr.shape[0] + 1, n), float("nan"), device=dev)
+        call = lambda: ops.quantized_matmul_ggml(xr, w, y, GgmlQuantizedMatmulParams(xr.shape[0], n, k, t))  # noqa: E731
+        call()
+        assert torch.isnan(y[-1]).all()
+        return y[:-1], call
+
+    y, call = product(x)
+    names = launched_kernels(call)
+    assert all("krows_kernel" in s for s in names) == takes, names
+    if not takes:
+        return
+    half = (m + 1) // 2
+    assert torch.equal(y[:half], product(x[:half])[0]) and torch.equal(y[half:], product(x[half:].contiguous())[0])
+    assert ((y - ref).norm() / ref.norm()).item() <= 6.6e-7
+    p, adt = GgmlQuantizedMatmulParams(m, n, k, t), x.dtype
+    need = ops.quantized_matmul_gated_workspace_bytes(p, adt)
+    assert (need > 0) == (k == 1024)
+    if need:
+        ws = torch.empty(need, dtype=torch.uint8, device=dev)
+        gate = torch.randn(m, n, generator=torch.Generator(device=dev).manual_seed(m), device=dev)
+        sep, got = torch.empty_like(y), torch.full_like(y, float("nan"))
+        ops.dispatch_silu_mul(gate, y, sep)
+        ops.quantized_matmul_gated_ggml(x, w, gate, got, p, ws)
+        assert torch.equal(got, sep)
+        ops.quantized_matmul_gated_ggml(x, w, gate, gate, p, ws)
+        assert torch.equal(gate, sep)
+
+
 @pytest.mark.parametrize("t", ALL_TYPES)
 @pytest.mark.parametrize("xdt", ["bf16", "f32"])
 @pytest.mark.parametrize("m", [5, 8])
