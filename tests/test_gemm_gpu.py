@@ -75,6 +75,14 @@ def test_small_tiles_and_k_slices_match_f64_oracle(oracle, dev, t, m, n, k):
     assert np.array_equal(y, y2)
 
 
+@pytest.mark.parametrize("xdt", ["bf16", "f32"])
+@pytest.mark.parametrize("k", [4096, 4352, 16384, 16640])
+def test_activation_rows_of_the_pre_pass_by_length(oracle, dev, xdt, k):
+    """Rows that a workgroup holds in registers in two ways, and a longer one that it reads twice."""
+    y, ref = _run(oracle, dev, HQ_Q4_K, xdt, 18, 64, k)
+    assert_matmul_close_f16_tile(y, ref, f"pre-pass {xdt} k={k}")
+
+
 @pytest.mark.parametrize("t", [HQ_Q4_K, HQ_Q5_K, HQ_Q6_K, HQ_Q8_0, HQ_Q4_0])
 @pytest.mark.parametrize("m,n,k,height", [(257, 130, 256, 2), (321, 4097, 768, 2), (1000, 2300, 256, 4), (1025, 2049, 512, 4), (500, 12290, 256, 8)])
 def test_tile_height_above_256_rows(dev, t, m, n, k, height):
