@@ -108,6 +108,25 @@ def test_tile_height_above_256_rows(dev, t, m, n, k, height):
     assert torch.isfinite(y).all()
 
 
+@pytest.mark.parametrize("m,k", [(17, 16384), (100, 16384)])
+def test_tiles_over_a_matrix_of_more_than_4_gib(dev, m, k):
+    """Q6_K rows of 13440 bytes, 512 of them repeated over 4.3 GB: the offsets inside a wave's rows stay those of 32 rows wherever they lie in
+    the matrix, so that every repetition has the bits of the first, and the first is the float64 product of its rows."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(k + m)
+    rows, times = 512, 626
+    few = ops.quantize_ggml(torch.randn(rows * k, generator=g, device=dev).mul_(0.05), k, HQ_Q6_K).flatten()
+    w = few.repeat(times)
+    assert w.numel() > 2 ** 32
+    x = torch.randn(m, k, generator=g, device=dev).to(torch.bfloat16)
+    y = torch.full((m, rows * times), float("nan"), device=dev)
+    ops.quantized_matmul_ggml(x, w, y, GgmlQuantizedMatmulParams(m, rows * times, k, HQ_Q6_K))
+    first = y[:, -rows:]
+    ref = x.double() @ ops.dequantize_ggml(few, rows * k, HQ_Q6_K).view(rows, k).double().T
+    assert_matmul_close_f16_tile(first.cpu().numpy(), ref.cpu().numpy(), f"m={m}")
+    assert all(torch.equal(part, first) for part in y.split(rows, dim=1))
+
+
 @pytest.mark.parametrize("t,m,n,k,at,own", [
     (HQ_Q8_0, 9, 33003, 384, 0, True), (HQ_Q8_0, 32, 33003, 384, 2, True), (HQ_Q8_0, 33, 33003, 384, 0, False),
     (HQ_Q4_0, 9, 33003, 384, 2, True), (HQ_Q4_0, 64, 33003, 896, 0, True), (HQ_Q4_0, 9, 33003, 256, 0, True),
