@@ -493,9 +493,10 @@ __global__ __launch_bounds__(64 * W) void krows_kernel(KRowsArgs a) {
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             const uint32_t v = (T::BYTES % 16u ? (f_row[i] + off) & ~15u : f_row[i] + off) + f_off[i];
-            // (inline assembly: the compiler would wait for every fetch into LDS ahead of any read from it)
+            // (inline assembly: the compiler would wait for every fetch into LDS ahead of any read from it; one wait state between a scalar write
+            // of M0 and the load that reads it, which it does not put there)
             if (64u * (i + 1) <= PIECES || 64u * i + lane < PIECES)
-                asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(v), "s"(f_base), "s"(dst + 1024u * i) : "memory", "m0");
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(v), "s"(f_base), "s"(dst + 1024u * i) : "memory", "m0");
         }
         --f_left;
         if (++f_slot == a.ring) f_slot = 0;

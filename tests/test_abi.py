@@ -38,6 +38,22 @@ def test_block_geometry():
     assert L.hq_block_elems(3) == 0 and L.hq_block_bytes(10) == 0  # Q4_1, Q2_K: not built
 
 
+def test_loads_into_lds_wait_a_state_behind_m0():
+    """A scalar write of M0 and a load into LDS that reads it are one wait state apart; the compiler does not look into inline assembly."""
+    csrc, met = os.path.join(ROOT, "hf2q_amd", "csrc"), 0
+    for f in sorted(os.listdir(csrc)):
+        if not f.endswith((".h", ".hip")):
+            continue
+        for text in re.findall(r'asm volatile\(\s*"([^"]*)"', open(os.path.join(csrc, f)).read()):
+            ops = text.split("\\n\\t")
+            for op, behind in zip(ops, ops[1:]):
+                if re.match(r"s_\w+ m0\b", op):
+                    met += 1
+                    assert behind.startswith("s_nop"), f"{f}: {text}"
+            assert not re.match(r"s_\w+ m0\b", ops[-1]), f"{f}: {text}"
+    assert met >= 2
+
+
 def test_workspace_queries_follow_the_routing():
     """Pure host arithmetic (no GPU call): which shapes take a tile kernel and how much scratch that needs."""
     L = lib.load()
