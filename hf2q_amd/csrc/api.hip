@@ -477,6 +477,9 @@ int hq_qmatmul_perm021_ggml_ws(void* stream, const void* x_perm, hq_act_dtype xd
     if (!workspace || workspace_bytes < need)
         return fail(HQ_ERR_INVALID_ARGUMENT, "%s: workspace of %zu bytes, %zu needed", fn, workspace ? workspace_bytes : (size_t)0, need);
     if (reinterpret_cast<uintptr_t>(workspace) % 256) return fail(HQ_ERR_INVALID_ARGUMENT, "%s: workspace must be 256-byte aligned", fn);
+    // (what the plain product does, which may be no tile)
+    if (gemv_krows_passes(t, xdt, m, n, k, w_blocks))
+        return launch_gemv_krows_passes((hipStream_t)stream, x_perm, xdt, w_blocks, y, m, n, k, t, nullptr, head_dim);
     if (f16_tile_route(m, k, t))
         return launch_gemm_f16_tile((hipStream_t)stream, x_perm, xdt, w_blocks, y, m, n, k, t, workspace, head_dim);
     if (int rc = launch_unpermute021((hipStream_t)stream, x_perm, workspace, m, k, head_dim, xdt == HQ_BF16 ? 2 : 4)) return rc;

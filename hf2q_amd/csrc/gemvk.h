@@ -38,7 +38,8 @@ typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
 constexpr uint32_t kKMaxSegs = 4;
 struct KRowsArgs {
-    const void* x;           // [m][k]
+    const void* x;           // row r, element e at r * xstride + e; heads outermost (hd != 0): at (e / hd) * xplane + r * xstride + e % hd
+    uint32_t xstride, hd, xplane;
     uint32_t m, k, rowb;     // rowb: bytes of a weight row
     uint32_t sb0, nsb;       // the launch covers super-blocks sb0 .. sb0 + nsb - 1 of every row
     uint32_t kp, rg, ring;   // waves that share a group's k, groups side by side in a workgroup, slots of a wave's ring
@@ -326,13 +327,14 @@ struct XRows {
     static constexpr int N = F32 ? NV + 1 : 8;  // rows of an operand
     uint4 r[NF][F32 ? N : N / 2];               // (bf16: two rows to a uint4)
     __device__ __forceinline__ void load(const KRowsArgs& a, uint32_t k0, uint32_t lane) {
-        const uint32_t per = krows_per(a.m, NF);
+        const uint32_t per = krows_per(a.m, NF), kk = k0 + 4u * lane;
+        const size_t at = a.hd ? (size_t)(kk / a.hd) * a.xplane + kk % a.hd : kk;
 #pragma unroll
         for (int f = 0; f < NF; ++f)
 #pragma unroll
             for (int i = 0; i < N; ++i)
                 if ((uint32_t)i < per && f * per + i < a.m) {
-                    const size_t e = (size_t)(f * per + i) * a.k + k0 + 4u * lane;
+                    const size_t e = (size_t)(f * per + i) * a.xstride + at;
                     if constexpr (F32) {
                         r[f][i] = *reinterpret_cast<const uint4*>(static_cast<const float*>(a.x) + e);
                     } else {

@@ -86,12 +86,15 @@ bool gemv_krows_batch_takes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32
 }
 
 int launch_gemv_krows(hipStream_t s, const void* x, hq_act_dtype xdt, uint32_t m, uint32_t k, hq_ggml_type t, const KRowsSeg* seg, uint32_t nseg,
-                      bool swiglu, const float* gate) {
+                      bool swiglu, const float* gate, uint32_t perm_hd, uint32_t perm_rows) {
     uint32_t cus = 0;
     if (int rc = cu_count(&cus)) return rc;
     if (nseg == 0 || nseg > kKMaxSegs || (swiglu && nseg != 2)) return fail(HQ_ERR_INVALID_ARGUMENT, "k rows: %u matrices", nseg);
     KRowsArgs a{};
     a.x = x;
+    a.xstride = perm_hd ? perm_hd : k;
+    a.hd = perm_hd;
+    a.xplane = perm_rows * perm_hd;
     a.m = m;
     a.k = k;
     const uint32_t nsb = k / 256u;
@@ -143,12 +146,12 @@ bool gemv_krows_passes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32_t n,
 }
 
 int launch_gemv_krows_passes(hipStream_t s, const void* x, hq_act_dtype xdt, const void* w, float* y, uint32_t m, uint32_t n, uint32_t k, hq_ggml_type t,
-                             const float* gate) {
+                             const float* gate, uint32_t perm_hd) {
     const uint32_t half = (m + 1u) / 2u;
     for (uint32_t r0 = 0; r0 < m; r0 += half) {
         const KRowsSeg seg{w, y + (size_t)r0 * n, n};
-        const uint8_t* xr = static_cast<const uint8_t*>(x) + (size_t)r0 * k * (xdt == HQ_BF16 ? 2 : 4);
-        if (int rc = launch_gemv_krows(s, xr, xdt, m - r0 < half ? m - r0 : half, k, t, &seg, 1, false, gate ? gate + (size_t)r0 * n : nullptr)) return rc;
+        const uint8_t* xr = static_cast<const uint8_t*>(x) + (size_t)r0 * (perm_hd ? perm_hd : k) * (xdt == HQ_BF16 ? 2 : 4);
+        if (int rc = launch_gemv_krows(s, xr, xdt, m - r0 < half ? m - r0 : half, k, t, &seg, 1, false, gate ? gate + (size_t)r0 * n : nullptr, perm_hd, m)) return rc;
     }
     return HQ_OK;
 }

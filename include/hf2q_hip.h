@@ -208,8 +208,9 @@ HQ_API int hq_qmatmul_swiglu_rows(void* stream, const void* x, hq_act_dtype xdt,
  * kk % head_dim.  Replaces quantized_matmul_mm_tensor_perm021(enc, reg, dev, input, weight, dst,
  * GgmlQuantizedMatmulPerm021Params{m, n, k, head_dim, ggml_type}) (forward_prefill_batched.rs:2219-2257), which
  * saves the transpose between attention and the output projection.  The tile GEMM (m > 8) gathers in its
- * activation pre-pass at no extra cost; other shapes copy the activations into row-major order in `workspace`
- * first.  head_dim: a multiple of 8 that divides k. */
+ * activation pre-pass at no extra cost, and so do the kernels that take nine to sixteen rows in two passes; other shapes copy
+ * the activations into row-major order in `workspace` first.  The bits of hq_qmatmul_ggml over the row-major activations.
+ * head_dim: a multiple of 8 that divides k. */
 HQ_API size_t hq_qmatmul_perm021_ggml_workspace_bytes(uint32_t m, uint32_t n, uint32_t k, hq_act_dtype xdt, hq_ggml_type t);
 HQ_API int hq_qmatmul_perm021_ggml_ws(void* stream, const void* x_perm, hq_act_dtype xdt, const void* w_blocks, float* y,
                                uint32_t m, uint32_t n, uint32_t k, uint32_t head_dim, hq_ggml_type t, void* workspace,

@@ -454,6 +454,24 @@ def test_perm021_matches_oracle_and_the_plain_product(oracle, dev, t, m, heads, 
         ops.quantized_matmul_mm_tensor_perm021(x_perm, wd, y, ops.GgmlQuantizedMatmulPerm021Params(m, n, k, hd + 8, t))
 
 
+@pytest.mark.parametrize("t", [HQ_Q4_K, HQ_Q6_K, HQ_Q8_0, HQ_Q4_0])
+@pytest.mark.parametrize("xdt", ["bf16", "f32"])
+@pytest.mark.parametrize("m,heads,hd,n", [(9, 16, 256, 4096), (12, 44, 64, 4112), (16, 4, 1024, 4096), (10, 512, 8, 4096), (13, 16, 256, 4099)])
+def test_perm021_has_the_bits_of_the_plain_product_at_nine_to_sixteen_rows(dev, t, xdt, m, heads, hd, n):
+    """Heads that are parts of a super-block, several of them and of eight values, products of a few rows in two passes and as tiles."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(m + hd)
+    k = heads * hd
+    w = ops.quantize_ggml(torch.randn(n * k, generator=g, device=dev).mul_(0.05), k, t)
+    x = torch.randn(m, k, generator=g, device=dev)
+    x = x.to(torch.bfloat16) if xdt == "bf16" else x
+    x_perm = x.view(m, heads, hd).permute(1, 0, 2).contiguous()
+    y, y2 = torch.full((m, n), float("nan"), device=dev), torch.full((m, n), float("nan"), device=dev)
+    ops.quantized_matmul_mm_tensor_perm021(x_perm, w, y, ops.GgmlQuantizedMatmulPerm021Params(m, n, k, hd, t))
+    ops.quantized_matmul_ggml(x, w, y2, GgmlQuantizedMatmulParams(m, n, k, t))
+    assert torch.isfinite(y).all() and torch.equal(y, y2)
+
+
 @pytest.mark.parametrize("k", [1024, 4096])
 def test_tile_gemm_with_caller_workspace_replays_from_a_hip_graph(oracle, dev, k):
     """hq_qmatmul_ggml_ws on the f16 tile route allocates nothing, so a prefill step can record it into a HIP graph:
