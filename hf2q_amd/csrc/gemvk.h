@@ -27,10 +27,10 @@
 
 #include <type_traits>
 
+#include "gemvk_plan.h"
 #include "hq_internal.h"
 
 namespace hq {
-
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4_t;
@@ -615,31 +615,11 @@ __global__ __launch_bounds__(64 * W) void krows_kernel(KRowsArgs a) {
 
 constexpr size_t kKLds = 160 * 1024 - 512;
 
-// How nsb super-blocks are dealt out: kp waves to a group of sixteen rows, rg groups side by side, at most S super-blocks to a wave and W
-// waves.  What counts is the work of the busiest SIMD (wave i runs on SIMD i % 4) per group, then the waves that hide the latencies.
-struct KSplit {
-    uint32_t s, kp, rg, load;  // load: super-blocks of the busiest SIMD
-};
-inline KSplit krows_split(uint32_t nsb, uint32_t units, uint32_t m, uint32_t cus, uint32_t s, uint32_t w) {
-    KSplit best{s, 0, 0, 0};
-    for (uint32_t kp = (nsb + s - 1u) / s; kp <= w && kp <= nsb; ++kp) {
-        if (m > 2u * kp) continue;  // (a wave adds up the parts of at most two rows of a group)
-        const uint32_t base = nsb / kp, extra = nsb % kp;
-        for (uint32_t rg = 1; rg <= 4u && rg * kp <= w && (rg == 1u || units >= 2u * rg * cus); ++rg) {
-            uint32_t simd[4] = {0, 0, 0, 0}, load = 0;
-            for (uint32_t i = 0; i < rg * kp; ++i) simd[i % 4u] += base + (i % kp < extra ? 1u : 0u);
-            for (uint32_t i = 0; i < 4u; ++i) load = simd[i] > load ? simd[i] : load;
-            const uint32_t mine = load * (best.kp ? best.rg : 1u), theirs = best.load * rg;
-            if (!best.kp || mine < theirs || (mine == theirs && rg * kp > best.rg * best.kp)) best = KSplit{s, kp, rg, load};
-        }
-    }
-    return best;
-}
-
 template <int TYPE, bool F32, int NV, int NF, int S, int W>
 int launch_krows(hipStream_t s, KRowsArgs& a, const KSplit& p, uint32_t cus) {
     using T = KWeights<TYPE>;
     constexpr size_t SLOT = 256u * T::PITCH;
+    if (!p.kp) return fail(HQ_ERR_UNSUPPORTED, "k rows: %u rows over %u super-blocks", a.m, a.nsb);
     a.kp = p.kp;
     a.rg = p.rg;
     const uint32_t waves = a.kp * a.rg, wgs = (a.units + a.rg - 1u) / a.rg, grid = wgs < cus ? wgs : cus;
@@ -659,24 +639,21 @@ int launch_krows(hipStream_t s, KRowsArgs& a, const KSplit& p, uint32_t cus) {
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * waves), ask, s, a);
     return check_launch("k rows kernel launch");
 }
-// The forms by super-blocks per wave and the waves that the registers then allow (512 per SIMD lane; 32 to 34 per super-block and operand and
-// about sixty others; Q6_K has no room for sixteen waves of two).  Sixteen waves of two only where twelve would all have two: k = 5120 over
-// 17408 rows 21.2 us with sixteen, 19.8 with twelve, slices of 24 super-blocks of 4096 x 12288 21.0 and 23.2.
 template <int TYPE, bool F32, int NV>
 int launch_krows_s(hipStream_t s, KRowsArgs& a, uint32_t cus) {
-    const KSplit one = krows_split(a.nsb, a.units, a.m, cus, 1, 16), two = krows_split(a.nsb, a.units, a.m, cus, 2, 12), three = krows_split(a.nsb, a.units, a.m, cus, 3, 12);
-    if (one.kp && one.load * two.rg <= two.load * one.rg && one.load * three.rg <= three.load * one.rg) return launch_krows<TYPE, F32, NV, 1, 1, 16>(s, a, one, cus);
+    const KSplit p = krows_form(TYPE == HQ_Q6_K, F32, a.m, a.nsb, a.units, cus);
+    if (p.s == 1u) return launch_krows<TYPE, F32, NV, 1, 1, 16>(s, a, p, cus);
     if constexpr (TYPE != HQ_Q6_K)
-        if (a.nsb > 20u && a.nsb <= 24u) return launch_krows<TYPE, F32, NV, 1, 2, 16>(s, a, krows_split(a.nsb, a.units, a.m, cus, 2, 16), cus);
-    if (two.kp && two.load * three.rg <= three.load * two.rg) return launch_krows<TYPE, F32, NV, 1, 2, 12>(s, a, two, cus);
-    return launch_krows<TYPE, F32, NV, 1, 3, 12>(s, a, three, cus);
+        if (p.w == 16u) return launch_krows<TYPE, F32, NV, 1, 2, 16>(s, a, p, cus);
+    if (p.s == 2u) return launch_krows<TYPE, F32, NV, 1, 2, 12>(s, a, p, cus);
+    return launch_krows<TYPE, F32, NV, 1, 3, 12>(s, a, p, cus);
 }
 template <int TYPE>
 int launch_krows_t(hipStream_t s, KRowsArgs& a, bool f32, uint32_t cus) {
     if (!f32) return launch_krows_s<TYPE, false, 2>(s, a, cus);
     if (a.m <= 4u) return launch_krows_s<TYPE, true, 3>(s, a, cus);
     if (a.m == 5u) return launch_krows_s<TYPE, true, 4>(s, a, cus);
-    return launch_krows<TYPE, true, 3, 2, 1, 16>(s, a, krows_split(a.nsb, a.units, a.m, cus, 1, 16), cus);
+    return launch_krows<TYPE, true, 3, 2, 1, 16>(s, a, krows_form(TYPE == HQ_Q6_K, true, a.m, a.nsb, a.units, cus), cus);
 }
 
 }  // namespace

@@ -3,16 +3,6 @@
 
 namespace hq {
 
-namespace {
-
-// Slices of k: as many super-blocks of a launch as the registers hold (launch_krows_t).
-uint32_t krows_per_slice(uint32_t nsb, bool f32, uint32_t m) {
-    const uint32_t cap = f32 && m > 5u ? 16u : 36u, slices = (nsb + cap - 1u) / cap;
-    return (nsb + slices - 1u) / slices;
-}
-
-}  // namespace
-
 // Where it is ahead of the kernels that serve a few rows otherwise (and no less exact: 0.9 .. 2e-7 of the result, Q8_0 and Q4_0 rows in bf16 8e-8).
 // n of whole groups of sixteen rows, k of whole super-blocks; the rest of the rule is measured, us before / here:
 //   bf16 rows at 3, 5, 8: Q4_K 4096 x 2816 6.6 / 5.2, 9.7 / 5.7, 9.9 / 6.2, 17408 x 5120 20.9 / 16.4, 21.0 / 16.8, 20.9 / 17.8, 152064 x 5120 94 / 81, 96 / 85,
@@ -28,7 +18,7 @@ uint32_t krows_per_slice(uint32_t nsb, bool f32, uint32_t m) {
 //   22.1 / 18.9; behind for fewer rows over K-quants (Q6_K bf16 at four 17.6 / 21.3) and at six to eight f32 rows (Q4_K 28.8 / 37.6).
 bool gemv_krows_takes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32_t n, uint32_t k, const void* w) {
     if (m < 2 || m > 8 || n % 16u || k % 256u || k < 1024 || !is_aligned(w, 16)) return false;
-    const bool f32 = xdt != HQ_BF16, head = n >= 32768, sliced = krows_per_slice(k / 256u, f32, m) < k / 256u;
+    const bool f32 = xdt != HQ_BF16, head = n >= 32768, sliced = krows_slices(k / 256u, f32, m) > 1u;
     const bool b32 = t == HQ_Q8_0 || t == HQ_Q4_0;
     if (!b32 && t != HQ_Q4_K && t != HQ_Q5_K && t != HQ_Q6_K) return false;
     const bool odd_k = k % 1024u != 0;  // k for which the K-quants have no chunked small-batch kernel
@@ -64,7 +54,7 @@ bool gemv_krows_swiglu_takes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint3
     if (m < 3 || m > 8 || n % 16u || k % 256u || k < 1024 || !is_aligned(wg, 16) || !is_aligned(wu, 16) || (uint64_t)n * k < 6u << 20) return false;
     if (t != HQ_Q8_0 && t != HQ_Q4_0 && t != HQ_Q4_K && t != HQ_Q5_K && t != HQ_Q6_K) return false;
     const bool f32 = xdt != HQ_BF16, b32 = t == HQ_Q8_0 || t == HQ_Q4_0;
-    if (krows_per_slice(k / 256u, f32, m) < k / 256u) return false;
+    if (krows_slices(k / 256u, f32, m) > 1u) return false;
     if (!f32) return m >= 4;
     if (m >= 6) return m >= 7 || b32 || (t == HQ_Q4_K && n >= 8192 && k > 2048);
     if (t == HQ_Q4_0 && n >= 4096) return true;
@@ -79,7 +69,7 @@ bool gemv_krows_batch_takes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32
     const bool f32 = xdt != HQ_BF16, b32 = t == HQ_Q8_0 || t == HQ_Q4_0;
     if (m < 2 || m > 8 || k % 256u || k < 1024 || (uint64_t)N * k < (f32 ? 12u << 20 : 8u << 20)) return false;
     if (t != HQ_Q8_0 && t != HQ_Q4_0 && t != HQ_Q4_K && t != HQ_Q5_K && t != HQ_Q6_K) return false;
-    if (krows_per_slice(k / 256u, f32, m) < k / 256u) return false;
+    if (krows_slices(k / 256u, f32, m) > 1u) return false;
     if (!f32) return m >= (t == HQ_Q4_K ? 2u : t == HQ_Q8_0 && k <= 2048 ? 4u : 3u);
     if (m >= 6) return b32 || (k % 1024u != 0 && (m >= 7 || t != HQ_Q5_K)) || (m >= 7 && t == HQ_Q4_K);
     return m == 5 || (m == 4 && (b32 || t == HQ_Q4_K || k % 1024u != 0 || N >= 8192));
@@ -109,12 +99,13 @@ int launch_gemv_krows(hipStream_t s, const void* x, hq_act_dtype xdt, uint32_t m
         a.units = a.end[i] = (i && !swiglu ? a.end[i - 1] : 0u) + seg[i].n / 16u;
     }
     const bool f32 = xdt != HQ_BF16;
-    const uint32_t per = krows_per_slice(nsb, f32, m);
-    if ((swiglu || gate) && per < nsb) return fail(HQ_ERR_INVALID_ARGUMENT, "k rows: gating in slices of k");
-    for (uint32_t sb = 0; sb < nsb; sb += per) {
-        a.sb0 = sb;
-        a.nsb = nsb - sb < per ? nsb - sb : per;
-        a.add = sb != 0;
+    const uint32_t slices = krows_slices(nsb, f32, m);
+    if ((swiglu || gate) && slices > 1u) return fail(HQ_ERR_INVALID_ARGUMENT, "k rows: gating in slices of k");
+    a.nsb = 0;
+    for (uint32_t i = 0; i < slices; ++i) {
+        a.sb0 += a.nsb;
+        a.nsb = krows_slice_blocks(nsb, slices, i);
+        a.add = i != 0;
         int rc = HQ_ERR_UNSUPPORTED;
         switch (t) {
             case HQ_Q4_K: rc = launch_krows_q4k(s, a, f32, cus); break;
@@ -138,7 +129,7 @@ bool gemv_krows_passes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32_t n,
     if (m <= 8 || m > 16 || (t != HQ_Q8_0 && t != HQ_Q4_0 && t != HQ_Q6_K)) return false;
     const uint32_t half = (m + 1u) / 2u;
     if (!gemv_krows_takes(t, xdt, half, n, k, w) || !gemv_krows_takes(t, xdt, m - half, n, k, w)) return false;
-    if (krows_per_slice(k / 256u, xdt != HQ_BF16, half) < k / 256u) return false;
+    if (krows_slices(k / 256u, xdt != HQ_BF16, half) > 1u) return false;
     const uint64_t weights = (uint64_t)n * k, M = 1u << 20;
     if (xdt == HQ_BF16) return t == HQ_Q8_0 || (t == HQ_Q4_0 ? n <= 12288 || n > 16384 : weights <= 25 * M);
     if (t == HQ_Q8_0) return n >= 32768 || (n >= 4096 && weights <= 16 * M);
