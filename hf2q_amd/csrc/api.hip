@@ -362,7 +362,7 @@ int hq_qmatmul_ggml(void* stream, const void* x, hq_act_dtype xdt, const void* w
                     uint32_t m, uint32_t n, uint32_t k, hq_ggml_type t) {
     if (int rc = check_matmul_common("hq_qmatmul_ggml", x, xdt, w_blocks, y, n, k, t)) return rc;
     if (m == 0) return HQ_OK;
-    const size_t need = hq_qmatmul_ggml_workspace_bytes(m, n, k, xdt, t);
+    const size_t need = gemv_krows_passes(t, xdt, m, n, k, w_blocks) ? 0 : hq_qmatmul_ggml_workspace_bytes(m, n, k, xdt, t);
     if (!need) return qmatmul_routes((hipStream_t)stream, x, xdt, w_blocks, y, m, n, k, t, nullptr);
     void* ws = nullptr;
     if (int rc = check_hip(hipMallocAsync(&ws, need, (hipStream_t)stream), "hipMallocAsync(qmatmul workspace)"))

@@ -73,6 +73,11 @@ def acts(seed, m, k):
 def launched_kernels(call):
     """Names (mangled) of the kernels that call() launches on the current device, in order.  It is captured into a graph that is
     never run, so the call itself must have run once before."""
+    return [name for name in launched_nodes(call) if name]
+
+
+def launched_nodes(call):
+    """The same with an empty string for whatever else call() puts into the stream (allocations, copies)."""
     import ctypes
 
     import torch
@@ -98,7 +103,8 @@ def launched_kernels(call):
     for node in nodes:
         kind, p = ctypes.c_int(), KernelNodeParams()
         assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0
+        names.append("")
         if kind.value == 0:  # a kernel
             assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(p)) == 0
-            names.append(hip.hipKernelNameRefByPtr(ctypes.c_void_p(p.func), ctypes.c_void_p(0)).decode())
+            names[-1] = hip.hipKernelNameRefByPtr(ctypes.c_void_p(p.func), ctypes.c_void_p(0)).decode()
     return names

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from _util import acts, assert_matmul_close, weights
-from _util import assert_matmul_close_f16_tile, launched_kernels
+from _util import assert_matmul_close_f16_tile, launched_kernels, launched_nodes
 from hf2q_amd import ops
 from hf2q_amd.ops import (HQ_Q4_0, HQ_Q4_K, HQ_Q5_K, HQ_Q6_K, HQ_Q8_0, GgmlQuantizedMatmulIdParams,
                           GgmlQuantizedMatmulParams)
@@ -312,6 +312,18 @@ def test_rows_in_registers_in_two_passes(dev, t, xdt, m, n, k, takes):
         assert torch.equal(got, sep)
         ops.quantized_matmul_gated_ggml(x, w, gate, gate, p, ws)
         assert torch.equal(gate, sep)
+
+
+def test_two_passes_allocate_nothing(dev):
+    """hq_qmatmul_ggml without a workspace takes one from the stream's allocator for a tile, and none for two passes."""
+    n, k, t = 4096, 4096, HQ_Q8_0
+    w, _ = _rows_ref(dev, t, n, k, torch.zeros(1, k, device=dev), 1)
+    for m, kinds in ((9, 2), (16, 2), (8, 1)):
+        x, y = torch.randn(m, k, device=dev).to(torch.bfloat16), torch.empty(m, n, device=dev)
+        call = lambda: ops.quantized_matmul_ggml(x, w, y, GgmlQuantizedMatmulParams(m, n, k, t))  # noqa: E731,B023
+        call()
+        nodes = launched_nodes(call)
+        assert len(nodes) == kinds and all("krows_kernel" in s for s in nodes), nodes
 
 
 @pytest.mark.parametrize("t", ALL_TYPES)
