@@ -453,6 +453,59 @@ __device__ __forceinline__ void wait_behind(uint32_t tasks) {  // all but the ne
 }
 constexpr uint32_t kKMaxRing = 4;
 
+// Weight e (of 256) of a super-block.
+template <int TYPE>
+__device__ __forceinline__ float weight_at(const uint8_t* p, uint32_t e) {
+    if constexpr (TYPE == HQ_Q4_0) {
+        p += Q4_0_BYTES * (e >> 5);
+        const uint32_t q = p[2u + (e & 15u)];
+        return f16_bits_to_f32(ld2(p)) * ((float)(e & 16u ? q >> 4 : q & 15u) - 8.f);
+    } else if constexpr (TYPE == HQ_Q6_K) {
+        const uint32_t h = e >> 7, r = (e >> 5) & 3u, l = e & 31u, ql = p[64u * h + 32u * (r & 1u) + l], qh = p[128u + 32u * h + l];
+        const float q = (float)((r >= 2u ? ql >> 4 : ql & 15u) | ((qh >> (2u * r)) & 3u) << 4) - 32.f;
+        return f16_bits_to_f32(ld2(p + 208)) * (float)(int8_t)p[192u + (e >> 4)] * q;
+    } else {
+        constexpr bool Q5 = TYPE == HQ_Q5_K;
+        const uint32_t s = e >> 5, l = e & 31u, lo = s & 3u, a = p[4u + lo], b = p[8u + lo], c = p[12u + lo];
+        const uint32_t sc = s < 4u ? a & 63u : (c & 15u) | (a >> 6) << 4, mn = s < 4u ? b & 63u : c >> 4 | (b >> 6) << 4;
+        const uint32_t qs = p[(Q5 ? 48u : 16u) + 32u * (s >> 1) + l];
+        uint32_t q = s & 1u ? qs >> 4 : qs & 15u;
+        if constexpr (Q5) q |= ((p[16u + l] >> s) & 1u) << 4;
+        return f16_bits_to_f32(ld2(p)) * (float)sc * (float)q - f16_bits_to_f32(ld2(p + 2)) * (float)mn;
+    }
+}
+
+// A sum that came out infinite or NaN, once more with whole weights: row `row` of x and row j of the group u, lane group g a quarter of k.  The
+// MFMAs take a weight in parts (nibble and upper bits, the mins), whose products with an infinite activation are NaN even where the
+// weight is not zero, and multiply by the scales last, so that a large activation can overflow on the way.  Sums of all products, or
+// where activations are no finite numbers of the products with those (a few us a row, once in a great while).  The arguments are read here and not kept in registers.
+typedef const __attribute__((address_space(4))) KRowsArgs* KRowsArgsPtr;
+template <int TYPE, bool F32>
+__device__ __forceinline__ float sum_again(uint32_t row, uint32_t u, uint32_t j, uint32_t g, uint32_t matrix) {
+    uint64_t at = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(at), "+v"(j), "+v"(g));
+    const KRowsArgsPtr a = (KRowsArgsPtr)at;
+    uint32_t seg = matrix, from = 0;
+    if (!a->swiglu)
+        while (seg + 1u < a->nseg && u >= a->end[seg]) from = a->end[seg++];
+    const uint8_t* w = a->w[seg] + (size_t)((u - from) * 16u + j) * a->rowb + (size_t)a->sb0 * KWeights<TYPE>::BYTES;
+    const uint32_t k0 = a->sb0 * 256u, count = a->nsb * 256u, hd = a->hd;
+    auto x_at = [&](uint32_t e) {
+        const size_t i = (size_t)row * a->xstride + (hd ? (size_t)((k0 + e) / hd) * a->xplane + (k0 + e) % hd : k0 + e);
+        return F32 ? static_cast<const float*>(a->x)[i] : bf16_bits_to_f32(static_cast<const uint16_t*>(a->x)[i]);
+    };
+    float nan = 0.f, sum = 0.f;
+#pragma unroll 1
+    for (uint32_t e = 16u * g + j; e < count; e += 64u) nan = fmaf(x_at(e), 0.f, nan);
+    const bool odd = __any(nan != nan);
+#pragma unroll 1
+    for (uint32_t e = g; e < count; e += 4u) {
+        const float x = x_at(e);
+        if (!odd || !(fabsf(x) < __builtin_inff())) sum = fmaf(x, weight_at<TYPE>(w + (size_t)(e >> 8) * KWeights<TYPE>::BYTES, e & 255u), sum);
+    }
+    return xor32_add(xor16_add(sum));
+}
+
 template <int TYPE, bool F32, int NV, int NF, int S, int W>
 __global__ __launch_bounds__(64 * W) void krows_kernel(KRowsArgs a) {
     using T = KWeights<TYPE>;
@@ -595,7 +648,12 @@ __global__ __launch_bounds__(64 * W) void krows_kernel(KRowsArgs a) {
                 const float u4 = r[(4u * p + g < a.kp ? 4u * p + g : 0u) * part];
                 t[p] = 4u * p + g < a.kp ? u4 : 0.f;
             }
-            const float v = xor32_add(xor16_add((t[0] + t[1]) + (t[2] + t[3])));
+            float v = xor32_add(xor16_add((t[0] + t[1]) + (t[2] + t[3])));
+            if constexpr (TYPE != HQ_Q8_0)  // (whose weights are one number each)
+                if (__builtin_expect(__any(!(fabsf(v) < __builtin_inff())), 0)) {
+                    const float whole = sum_again<TYPE, F32>(row, u, j, g, a.swiglu ? round & 1u : 0u);
+                    if (!(fabsf(v) < __builtin_inff())) v = whole;
+                }
             if (a.swiglu && !(round & 1u)) {
                 held[i] = v;
             } else if (g == 0u) {
