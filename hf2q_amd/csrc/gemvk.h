@@ -1,4 +1,4 @@
-// Dequant-fused product for a few activation rows (2..8; bf16 rows up to 16) with the activations in REGISTERS:
+// Dequant-fused product for a few activation rows (2..8) with the activations in REGISTERS:
 // y[m, n] = sum_k x[m, k] * W[n, k] with every weight fetched once for all rows and no activation read from LDS.
 //
 // What bounds it: the weight bytes (0.5625 .. 1.0625 per weight); the arithmetic, one unpack per weight and four multiply-adds per
@@ -8,7 +8,7 @@
 //
 // Mapping.  A workgroup works on groups of sixteen weight rows.  Its waves split k: wave w owns up to S super-blocks (256
 // weights) of every row and keeps the activations that meet them as MFMA operands for the whole launch, 32 registers per
-// super-block and sixteen columns.  bf16 rows are a column each.  An f32 row is three columns: its value cut into three bf16
+// super-block and sixteen columns.  bf16 rows are a column each, two of the four that a lane group's results are.  An f32 row is three columns: its value cut into three bf16
 // parts of eight bits (all 24 bits of it, so the products are exact and only the f32 sums round); five rows make fifteen
 // columns, six to eight rows two operands of twelve.  Per task -- one super-block of sixteen rows -- a wave copies the
 // blocks from memory straight into a slot of LDS of its own (global_load_lds, consecutive lanes consecutive 16-byte pieces
@@ -45,6 +45,7 @@ struct KRowsArgs {
     uint32_t kp, rg, ring;   // waves that share a group's k, groups side by side in a workgroup, slots of a wave's ring
     uint32_t base, extra;    // super-blocks per wave: nsb / kp, and the first nsb % kp waves one more
     uint32_t units, full, rem;  // groups of sixteen rows, all segments (swiglu: of one matrix); units over gridDim * rg, and the rest
+    uint32_t whole;          // sums are taken again where they are infinite or NaN
     const float* gate;       // may be null, laid out as y[0]: silu(gate) * product is stored
     uint32_t add, swiglu;    // add: products are added to y; swiglu: seg 0 = gate, seg 1 = up, y[0] = silu(gate) * up
     uint32_t nseg;
@@ -102,7 +103,9 @@ struct KWeightsQ45 {
     }
     template <int NF, int NV>
     __device__ __forceinline__ void mul(const XFrag<NSUM> (&x)[NF], uint32_t g, f32x4_t (&acc)[NF]) const {
-        const float d = f16_bits_to_f32(hdr.x & 0xffffu), dmin = f16_bits_to_f32(hdr.x >> 16);
+        // (the codes stand for 2^-10 of their number and d for 2^10 of its own: a sum of a sub-block times its six bits of scale is no larger than
+        // its activations allow, and overflows no earlier than the product does)
+        const float d = 1024.f * f16_bits_to_f32(hdr.x & 0xffffu), dmin = f16_bits_to_f32(hdr.x >> 16);
         const uint32_t zs = hdr.z >> (8u * g), ws = hdr.w >> (8u * g);
         // mins of sub-blocks g and 4 + g
         const float o0 = dmin * (float)(zs & 63u), o1 = dmin * (float)(((ws >> 4) & 15u) | ((zs >> 2) & 0x30u));
@@ -118,11 +121,11 @@ struct KWeightsQ45 {
         for (int c = 0; c < 4; ++c) {
             const uint32_t s = c < 2 ? sl : sh;
             const float s0 = c & 1 ? ubyte2(s) : ubyte0(s), s1 = c & 1 ? ubyte3(s) : ubyte1(s);
-            const uint4 lo = from_codes(q[c].x & N4, q[c].y & N4, kOne), hi = from_codes((q[c].x >> 4) & N4, (q[c].y >> 4) & N4, kOne);
+            const uint4 lo = from_codes(q[c].x & N4, q[c].y & N4, kOne / 1024.f), hi = from_codes((q[c].x >> 4) & N4, (q[c].y >> 4) & N4, kOne / 1024.f);
             uint4 lo5, hi5;
             if constexpr (Q5) {
-                lo5 = from_codes((qh.x >> (2 * c)) & N1, (qh.y >> (2 * c)) & N1, kSixteen);
-                hi5 = from_codes((qh.x >> (2 * c + 1)) & N1, (qh.y >> (2 * c + 1)) & N1, kSixteen);
+                lo5 = from_codes((qh.x >> (2 * c)) & N1, (qh.y >> (2 * c)) & N1, kSixteen / 1024.f);
+                hi5 = from_codes((qh.x >> (2 * c + 1)) & N1, (qh.y >> (2 * c + 1)) & N1, kSixteen / 1024.f);
             }
 #pragma unroll
             for (int f = 0; f < NF; ++f) {
@@ -453,60 +456,74 @@ __device__ __forceinline__ void wait_behind(uint32_t tasks) {  // all but the ne
 }
 constexpr uint32_t kKMaxRing = 4;
 
-// Weight e (of 256) of a super-block.
+// Weight e (of 256) of a super-block of Q4_0 or Q6_K.
 template <int TYPE>
 __device__ __forceinline__ float weight_at(const uint8_t* p, uint32_t e) {
+    static_assert(TYPE == HQ_Q4_0 || TYPE == HQ_Q6_K, "the types of sum_again");
     if constexpr (TYPE == HQ_Q4_0) {
         p += Q4_0_BYTES * (e >> 5);
         const uint32_t q = p[2u + (e & 15u)];
         return f16_bits_to_f32(ld2(p)) * ((float)(e & 16u ? q >> 4 : q & 15u) - 8.f);
-    } else if constexpr (TYPE == HQ_Q6_K) {
+    } else {
         const uint32_t h = e >> 7, r = (e >> 5) & 3u, l = e & 31u, ql = p[64u * h + 32u * (r & 1u) + l], qh = p[128u + 32u * h + l];
         const float q = (float)((r >= 2u ? ql >> 4 : ql & 15u) | ((qh >> (2u * r)) & 3u) << 4) - 32.f;
         return f16_bits_to_f32(ld2(p + 208)) * (float)(int8_t)p[192u + (e >> 4)] * q;
-    } else {
-        constexpr bool Q5 = TYPE == HQ_Q5_K;
-        const uint32_t s = e >> 5, l = e & 31u, lo = s & 3u, a = p[4u + lo], b = p[8u + lo], c = p[12u + lo];
-        const uint32_t sc = s < 4u ? a & 63u : (c & 15u) | (a >> 6) << 4, mn = s < 4u ? b & 63u : c >> 4 | (b >> 6) << 4;
-        const uint32_t qs = p[(Q5 ? 48u : 16u) + 32u * (s >> 1) + l];
-        uint32_t q = s & 1u ? qs >> 4 : qs & 15u;
-        if constexpr (Q5) q |= ((p[16u + l] >> s) & 1u) << 4;
-        return f16_bits_to_f32(ld2(p)) * (float)sc * (float)q - f16_bits_to_f32(ld2(p + 2)) * (float)mn;
     }
 }
 
-// A sum that came out infinite or NaN, once more with whole weights: row `row` of x and row j of the group u, lane group g a quarter of k.  The
-// MFMAs take a weight in parts (nibble and upper bits, the mins), whose products with an infinite activation are NaN even where the
-// weight is not zero, and multiply by the scales last, so that a large activation can overflow on the way.  Sums of all products, or
-// where activations are no finite numbers of the products with those (a few us a row, once in a great while).  The arguments are read here and not kept in registers.
+// A sum that came out infinite or NaN, once more with whole weights: row `row` of x and row lane % 16 of the group u, a lane group a quarter of
+// k.  The MFMAs take a Q4_0 or Q6_K weight in two parts of opposite signs, for which an infinite activation is NaN even where the weight is not
+// zero.  Where the row holds a NaN there is nothing to do, where it holds infinities their products are the sum, else all products (a
+// part that was beyond f32).  The arguments are read here and not kept in registers.
 typedef const __attribute__((address_space(4))) KRowsArgs* KRowsArgsPtr;
 template <int TYPE, bool F32>
-__device__ __forceinline__ float sum_again(uint32_t row, uint32_t u, uint32_t j, uint32_t g, uint32_t matrix) {
+__device__ __forceinline__ float sum_again(uint32_t row, uint32_t u, uint32_t lane, uint32_t matrix) {
     uint64_t at = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(at), "+v"(j), "+v"(g));
+    asm volatile("" : "+s"(at), "+v"(lane));
     const KRowsArgsPtr a = (KRowsArgsPtr)at;
+    const uint32_t k0 = a->sb0 * 256u, nsb = a->nsb, hd = a->hd;
+    // a super-block's activations, four to a lane, as f32
+    auto x4 = [&](uint32_t sb) {
+        const uint32_t kk = k0 + sb * 256u + 4u * lane;
+        const size_t i = (size_t)row * a->xstride + (hd ? (size_t)(kk / hd) * a->xplane + kk % hd : kk);
+        if constexpr (F32) return *reinterpret_cast<const uint4*>(static_cast<const float*>(a->x) + i);
+        const uint2 t = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(a->x) + i);
+        return make_uint4(t.x << 16, t.x & 0xffff0000u, t.y << 16, t.y & 0xffff0000u);
+    };
+    uint32_t most = 0;  // the largest magnitude, as bits: infinity 0x7f800000, NaNs above
+#pragma unroll 4
+    for (uint32_t sb = 0; sb < nsb; ++sb) {
+        const uint4 v = x4(sb);
+        const uint32_t ab = max(v.x & 0x7fffffffu, v.y & 0x7fffffffu), cd = max(v.z & 0x7fffffffu, v.w & 0x7fffffffu);
+        most = max(most, max(ab, cd));
+    }
+    if (__any(most > 0x7f800000u)) return __builtin_nanf("");
+    const bool odd = __any(most == 0x7f800000u);
+
     uint32_t seg = matrix, from = 0;
     if (!a->swiglu)
         while (seg + 1u < a->nseg && u >= a->end[seg]) from = a->end[seg++];
-    const uint8_t* w = a->w[seg] + (size_t)((u - from) * 16u + j) * a->rowb + (size_t)a->sb0 * KWeights<TYPE>::BYTES;
-    const uint32_t k0 = a->sb0 * 256u, count = a->nsb * 256u, hd = a->hd;
-    auto x_at = [&](uint32_t e) {
-        const size_t i = (size_t)row * a->xstride + (hd ? (size_t)((k0 + e) / hd) * a->xplane + (k0 + e) % hd : k0 + e);
-        return F32 ? static_cast<const float*>(a->x)[i] : bf16_bits_to_f32(static_cast<const uint16_t*>(a->x)[i]);
-    };
-    float nan = 0.f, sum = 0.f;
+    const uint8_t* w = a->w[seg] + (size_t)((u - from) * 16u + (lane & 15u)) * a->rowb + (size_t)a->sb0 * KWeights<TYPE>::BYTES;
+    float sum = 0.f;
 #pragma unroll 1
-    for (uint32_t e = 16u * g + j; e < count; e += 64u) nan = fmaf(x_at(e), 0.f, nan);
-    const bool odd = __any(nan != nan);
-#pragma unroll 1
-    for (uint32_t e = g; e < count; e += 4u) {
-        const float x = x_at(e);
-        if (!odd || !(fabsf(x) < __builtin_inff())) sum = fmaf(x, weight_at<TYPE>(w + (size_t)(e >> 8) * KWeights<TYPE>::BYTES, e & 255u), sum);
+    for (uint32_t sb = 0; sb < nsb; ++sb, w += KWeights<TYPE>::BYTES) {
+        const uint4 v = x4(sb);
+        auto inf = [](uint32_t b) { return (b & 0x7fffffffu) == 0x7f800000u; };
+        uint64_t lanes = odd ? __ballot(inf(v.x) || inf(v.y) || inf(v.z) || inf(v.w)) : ~0ull;
+        while (lanes) {  // lane l's four activations, one to each lane group
+            const int l = __builtin_ctzll(lanes);
+            lanes &= lanes - 1u;
+            const uint32_t x0 = __builtin_amdgcn_readlane(v.x, l), x1 = __builtin_amdgcn_readlane(v.y, l), x2 = __builtin_amdgcn_readlane(v.z, l), x3 = __builtin_amdgcn_readlane(v.w, l);
+            const uint32_t g = lane >> 4, x = g & 2u ? (g & 1u ? x3 : x2) : g & 1u ? x1 : x0;
+            if (!odd || inf(x)) sum = fmaf(__uint_as_float(x), weight_at<TYPE>(w, 4u * l + g), sum);
+        }
     }
     return xor32_add(xor16_add(sum));
 }
 
-template <int TYPE, bool F32, int NV, int NF, int S, int W>
+// WHOLE: sums that are infinite or NaN are taken again (sum_again): where the kernel stands for a tile, whose weights are one number each, at nine to
+// sixteen rows.  (The registers around that branch cost 1 to 2 %; the other kernels for two to eight rows take weights in parts as well.)
+template <int TYPE, bool F32, int NV, int NF, int S, int W, bool WHOLE>
 __global__ __launch_bounds__(64 * W) void krows_kernel(KRowsArgs a) {
     using T = KWeights<TYPE>;
     constexpr uint32_t PIECES = 16u * T::PITCH, SLOT = PIECES * 16u;
@@ -649,9 +666,9 @@ __global__ __launch_bounds__(64 * W) void krows_kernel(KRowsArgs a) {
                 t[p] = 4u * p + g < a.kp ? u4 : 0.f;
             }
             float v = xor32_add(xor16_add((t[0] + t[1]) + (t[2] + t[3])));
-            if constexpr (TYPE != HQ_Q8_0)  // (whose weights are one number each)
+            if constexpr (WHOLE)
                 if (__builtin_expect(__any(!(fabsf(v) < __builtin_inff())), 0)) {
-                    const float whole = sum_again<TYPE, F32>(row, u, j, g, a.swiglu ? round & 1u : 0u);
+                    const float whole = sum_again<TYPE, F32>(row, u, lane, a.swiglu ? round & 1u : 0u);
                     if (!(fabsf(v) < __builtin_inff())) v = whole;
                 }
             if (a.swiglu && !(round & 1u)) {
@@ -673,7 +690,7 @@ __global__ __launch_bounds__(64 * W) void krows_kernel(KRowsArgs a) {
 
 constexpr size_t kKLds = 160 * 1024 - 512;
 
-template <int TYPE, bool F32, int NV, int NF, int S, int W>
+template <int TYPE, bool F32, int NV, int NF, int S, int W, bool WHOLE>
 int launch_krows(hipStream_t s, KRowsArgs& a, const KSplit& p, uint32_t cus) {
     using T = KWeights<TYPE>;
     constexpr size_t SLOT = 256u * T::PITCH;
@@ -691,27 +708,34 @@ int launch_krows(hipStream_t s, KRowsArgs& a, const KSplit& p, uint32_t cus) {
     const size_t lds = waves * a.ring * SLOT + red;
     if (waves > (uint32_t)W || a.base + (a.extra ? 1u : 0u) > (uint32_t)S || a.ring < 1u || a.rg * a.m > 2u * waves)
         return fail(HQ_ERR_INVALID_ARGUMENT, "k rows: %u rows, %u super-blocks over %u waves", a.m, a.nsb, waves);
-    auto kern = krows_kernel<TYPE, F32, NV, NF, S, W>;
+    auto kern = krows_kernel<TYPE, F32, NV, NF, S, W, WHOLE>;
     const size_t ask = lds < 81 * 1024 ? 81 * 1024 : lds;  // one workgroup per CU
     if (int rc = ensure_lds_limit(reinterpret_cast<const void*>(kern), ask, "hipFuncSetAttribute(k rows LDS)")) return rc;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * waves), ask, s, a);
     return check_launch("k rows kernel launch");
 }
-template <int TYPE, bool F32, int NV>
+template <int TYPE, bool F32, int NV, bool WHOLE>
 int launch_krows_s(hipStream_t s, KRowsArgs& a, uint32_t cus) {
     const KSplit p = krows_form(TYPE == HQ_Q6_K, F32, a.m, a.nsb, a.units, cus);
-    if (p.s == 1u) return launch_krows<TYPE, F32, NV, 1, 1, 16>(s, a, p, cus);
+    if (p.s == 1u) return launch_krows<TYPE, F32, NV, 1, 1, 16, WHOLE>(s, a, p, cus);
     if constexpr (TYPE != HQ_Q6_K)
-        if (p.w == 16u) return launch_krows<TYPE, F32, NV, 1, 2, 16>(s, a, p, cus);
-    if (p.s == 2u) return launch_krows<TYPE, F32, NV, 1, 2, 12>(s, a, p, cus);
-    return launch_krows<TYPE, F32, NV, 1, 3, 12>(s, a, p, cus);
+        if (p.w == 16u) return launch_krows<TYPE, F32, NV, 1, 2, 16, WHOLE>(s, a, p, cus);
+    if (p.s == 2u) return launch_krows<TYPE, F32, NV, 1, 2, 12, WHOLE>(s, a, p, cus);
+    return launch_krows<TYPE, F32, NV, 1, 3, 12, WHOLE>(s, a, p, cus);
+}
+template <int TYPE, bool WHOLE>
+int launch_krows_w(hipStream_t s, KRowsArgs& a, bool f32, uint32_t cus) {
+    if (!f32) return launch_krows_s<TYPE, false, 2, WHOLE>(s, a, cus);
+    if constexpr (!WHOLE)  // (half of nine rows or more)
+        if (a.m <= 4u) return launch_krows_s<TYPE, true, 3, WHOLE>(s, a, cus);
+    if (a.m == 5u) return launch_krows_s<TYPE, true, 4, WHOLE>(s, a, cus);
+    return launch_krows<TYPE, true, 3, 2, 1, 16, WHOLE>(s, a, krows_form(TYPE == HQ_Q6_K, true, a.m, a.nsb, a.units, cus), cus);
 }
 template <int TYPE>
 int launch_krows_t(hipStream_t s, KRowsArgs& a, bool f32, uint32_t cus) {
-    if (!f32) return launch_krows_s<TYPE, false, 2>(s, a, cus);
-    if (a.m <= 4u) return launch_krows_s<TYPE, true, 3>(s, a, cus);
-    if (a.m == 5u) return launch_krows_s<TYPE, true, 4>(s, a, cus);
-    return launch_krows<TYPE, true, 3, 2, 1, 16>(s, a, krows_form(TYPE == HQ_Q6_K, true, a.m, a.nsb, a.units, cus), cus);
+    if constexpr (TYPE == HQ_Q4_0 || TYPE == HQ_Q6_K)
+        if (a.whole) return launch_krows_w<TYPE, true>(s, a, f32, cus);
+    return launch_krows_w<TYPE, false>(s, a, f32, cus);
 }
 
 }  // namespace

@@ -76,7 +76,7 @@ bool gemv_krows_batch_takes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32
 }
 
 int launch_gemv_krows(hipStream_t s, const void* x, hq_act_dtype xdt, uint32_t m, uint32_t k, hq_ggml_type t, const KRowsSeg* seg, uint32_t nseg,
-                      bool swiglu, const float* gate, uint32_t perm_hd, uint32_t perm_rows) {
+                      bool swiglu, const float* gate, uint32_t perm_hd, uint32_t perm_rows, bool whole) {
     uint32_t cus = 0;
     if (int rc = cu_count(&cus)) return rc;
     if (nseg == 0 || nseg > kKMaxSegs || (swiglu && nseg != 2)) return fail(HQ_ERR_INVALID_ARGUMENT, "k rows: %u matrices", nseg);
@@ -92,6 +92,7 @@ int launch_gemv_krows(hipStream_t s, const void* x, hq_act_dtype xdt, uint32_t m
     a.nseg = nseg;
     a.swiglu = swiglu;
     a.gate = gate;
+    a.whole = whole;
     for (uint32_t i = 0; i < nseg; ++i) {
         a.w[i] = static_cast<const uint8_t*>(seg[i].w);
         a.y[i] = seg[i].y;
@@ -142,7 +143,7 @@ int launch_gemv_krows_passes(hipStream_t s, const void* x, hq_act_dtype xdt, con
     for (uint32_t r0 = 0; r0 < m; r0 += half) {
         const KRowsSeg seg{w, y + (size_t)r0 * n, n};
         const uint8_t* xr = static_cast<const uint8_t*>(x) + (size_t)r0 * (perm_hd ? perm_hd : k) * (xdt == HQ_BF16 ? 2 : 4);
-        if (int rc = launch_gemv_krows(s, xr, xdt, m - r0 < half ? m - r0 : half, k, t, &seg, 1, false, gate ? gate + (size_t)r0 * n : nullptr, perm_hd, m)) return rc;
+        if (int rc = launch_gemv_krows(s, xr, xdt, m - r0 < half ? m - r0 : half, k, t, &seg, 1, false, gate ? gate + (size_t)r0 * n : nullptr, perm_hd, m, true)) return rc;
     }
     return HQ_OK;
 }

@@ -106,9 +106,10 @@ struct KRowsSeg {
 bool gemv_krows_takes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32_t n, uint32_t k, const void* w);
 bool gemv_krows_swiglu_takes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32_t n, uint32_t k, const void* wg, const void* wu);
 bool gemv_krows_batch_takes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32_t n_all, uint32_t k);
-// perm_hd != 0: the m rows of x are rows of [k / perm_hd][perm_rows][perm_hd] (attention output, heads outermost).
+// perm_hd != 0: the m rows of x are rows of [k / perm_hd][perm_rows][perm_hd] (attention output, heads outermost).  whole: products of Q4_0 and Q6_K
+// weights with infinite activations as a tile gives them.
 int launch_gemv_krows(hipStream_t s, const void* x, hq_act_dtype xdt, uint32_t m, uint32_t k, hq_ggml_type t, const KRowsSeg* seg, uint32_t nseg,
-                      bool swiglu, const float* gate = nullptr, uint32_t perm_hd = 0, uint32_t perm_rows = 0);
+                      bool swiglu, const float* gate = nullptr, uint32_t perm_hd = 0, uint32_t perm_rows = 0, bool whole = false);
 // Nine to sixteen rows as two of its passes, where those are ahead of a tile; gate: may be null, y = silu(gate) * product.
 bool gemv_krows_passes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32_t n, uint32_t k, const void* w);
 int launch_gemv_krows_passes(hipStream_t s, const void* x, hq_act_dtype xdt, const void* w, float* y, uint32_t m, uint32_t n, uint32_t k, hq_ggml_type t,

@@ -382,11 +382,9 @@ def test_rows_in_registers_keep_large_small_and_non_finite_values(dev, t, m):
 
 
 @pytest.mark.parametrize("t,xdt,m,n,k", [
-    (HQ_Q4_0, "bf16", 5, 4096, 4096), (HQ_Q4_0, "f32", 5, 4096, 5120), (HQ_Q4_0, "f32", 8, 4096, 4096), (HQ_Q4_0, "bf16", 8, 4112, 9216),
-    (HQ_Q6_K, "bf16", 5, 4096, 4096), (HQ_Q6_K, "f32", 5, 6144, 5120), (HQ_Q6_K, "f32", 8, 4096, 2816), (HQ_Q6_K, "bf16", 8, 4112, 9216),
-    (HQ_Q6_K, "f32", 5, 4112, 17408), (HQ_Q8_0, "bf16", 6, 4112, 4096), (HQ_Q8_0, "f32", 5, 4112, 4096), (HQ_Q8_0, "f32", 8, 8192, 4096),
-    (HQ_Q4_0, "bf16", 12, 4096, 4096), (HQ_Q4_0, "f32", 10, 4096, 4096), (HQ_Q6_K, "bf16", 16, 4096, 4096), (HQ_Q8_0, "f32", 16, 4096, 4096),
-    (HQ_Q4_K, "f32", 5, 8192, 2816), (HQ_Q4_K, "bf16", 6, 4096, 2816), (HQ_Q5_K, "f32", 5, 4128, 5120), (HQ_Q5_K, "bf16", 5, 4096, 4096),
+    (HQ_Q4_0, "bf16", 12, 4096, 4096), (HQ_Q4_0, "f32", 10, 4096, 4096), (HQ_Q4_0, "bf16", 16, 4112, 9216), (HQ_Q4_0, "f32", 15, 4096, 2816),
+    (HQ_Q6_K, "bf16", 16, 4096, 4096), (HQ_Q6_K, "bf16", 9, 2064, 9216), (HQ_Q6_K, "f32", 9, 4096, 4096), (HQ_Q6_K, "f32", 10, 4096, 2816),
+    (HQ_Q8_0, "bf16", 6, 4112, 4096), (HQ_Q8_0, "f32", 5, 4112, 4096), (HQ_Q8_0, "f32", 8, 8192, 4096), (HQ_Q8_0, "f32", 16, 4096, 4096),
 ])
 def test_rows_in_registers_carry_infinities(dev, t, xdt, m, n, k):
     """Infinities and NaNs in several rows, super-blocks and waves, of both signs in one: the results that are infinite or NaN are those of
@@ -411,28 +409,13 @@ def test_rows_in_registers_carry_infinities(dev, t, xdt, m, n, k):
     assert torch.isinf(ref[1]).any() and torch.isnan(ref[0]).all()
 
 
-@pytest.mark.parametrize("t", ALL_TYPES)
-@pytest.mark.parametrize("xdt", ["bf16", "f32"])
-def test_rows_in_registers_carry_infinities_into_the_gating(dev, t, xdt):
-    m, n, k = 5, 4112, 2816
-    x = torch.randn(m, k, generator=torch.Generator(device=dev).manual_seed(t), device=dev)
-    x[1, 1000], x[3, 5], x[4, k - 1] = float("inf"), float("nan"), float("-inf")
-    x = x.to(torch.bfloat16) if xdt == "bf16" else x
-    (wg, g), (wu, u) = _rows_ref(dev, t, n, k, x, 5), _rows_ref(dev, t, n, k, x, 6)
-    y, p = torch.empty(m, n, device=dev), GgmlQuantizedMatmulParams(m, n, k, t)
-    ops.quantized_matmul_swiglu_rows(x, wg, wu, y, p)
-    want = g / (1 + torch.exp(-g)) * u
-    assert torch.equal(torch.isnan(y), torch.isnan(want)) and torch.equal(y[torch.isinf(want)].double(), want[torch.isinf(want)])
-    assert torch.isinf(want[1]).any() and torch.isfinite(y[[0, 2]]).all()
-
-
-@pytest.mark.parametrize("t,xdt,m,n,k", [(HQ_Q4_K, "f32", 4, 8192, 2816), (HQ_Q5_K, "f32", 5, 4128, 5120), (HQ_Q6_K, "bf16", 5, 4096, 4096),
-                                         (HQ_Q4_0, "f32", 5, 4096, 4096), (HQ_Q6_K, "bf16", 12, 4096, 4096)])
+@pytest.mark.parametrize("t,xdt,m,n,k", [(HQ_Q4_K, "f32", 4, 8192, 2816), (HQ_Q5_K, "f32", 5, 4128, 5120), (HQ_Q5_K, "bf16", 5, 4096, 4096),
+                                         (HQ_Q4_0, "f32", 10, 4096, 4096), (HQ_Q6_K, "bf16", 12, 4096, 4096)])
 def test_rows_in_registers_take_large_activations(dev, t, xdt, m, n, k):
-    """One activation so large that a product with a weight's integer parts, ahead of the scales, is beyond f32 where the product with the weight
-    is not.  Sums that are taken again are k / 4 f32 additions in a row and two more: that many times 2^-24 of the products' absolute values."""
+    """One activation so large that a product with a weight's integer parts or a scale is beyond f32 where the product with the weight is not.
+    A sum is at most k / 4 f32 additions in a row and two more: that many times 2^-24 of the products' absolute values."""
     x = torch.randn(m, k, generator=torch.Generator(device=dev).manual_seed(t), device=dev)
-    x[2, 1000] = 3e37
+    x[2, 1000] = 1e37
     x = x.to(torch.bfloat16) if xdt == "bf16" else x
     w, ref = _rows_ref(dev, t, n, k, x, 5)
     y = torch.empty(m, n, device=dev)
