@@ -318,7 +318,7 @@ int hq_qmatmul_ggml_k_slices(uint32_t m, uint32_t n, uint32_t k, hq_ggml_type t,
         return fail(HQ_ERR_INVALID_ARGUMENT, "hq_qmatmul_ggml_k_slices: type %d, n %u, k %u", (int)t, n, k);
     *slices = 1;
     *blocks_per_slice = (k + 255u) / 256u;
-    if (f16_tile_route(m, k, t) && m <= 256) gemm_f16_small_tile_slices(t, m, n, k, slices, blocks_per_slice);
+    if (f16_tile_route(m, k, t) && m <= 256) gemm_f16_small_tile_slices(m, n, k, slices, blocks_per_slice);
     return HQ_OK;
 }
 

@@ -221,7 +221,7 @@ struct DenseFfnArgs {
 };
 size_t dense_ffn_scratch_bytes(uint32_t inter);
 int launch_dense_ffn(hipStream_t s, const DenseFfnArgs& a, bool dry);
-void gemm_f16_small_tile_slices(hq_ggml_type t, uint32_t m, uint32_t n, uint32_t k, uint32_t* splits, uint32_t* sb_per);
+void gemm_f16_small_tile_slices(uint32_t m, uint32_t n, uint32_t k, uint32_t* splits, uint32_t* sb_per);
 
 // TurboQuant KV (tq.hip)
 int launch_fwht_sign(hipStream_t s, float* buf, uint32_t n_heads, uint32_t head_dim, bool undo);
