@@ -105,21 +105,25 @@ HQ_API int hq_quantize_ggml_imatrix(void* stream, const float* src, uint64_t n_e
  * (src/inference/models/qwen35/gpu_ffn.rs:1236-1245; dispatch_qmatmul,
  * src/serve/forward_mlx.rs:9655-9969).  m <= 8 takes the bandwidth-bound GEMV
  * kernels (MM_ROUTING_THRESHOLD, forward_mlx.rs:9791; from two to four rows on, by type, a form that fetches every
- * weight once for all rows), and Q4_K / Q5_K run up to 16 rows as two such passes; larger m takes the MFMA GEMM,
- * whose tiles are 64, 128 or 256 token rows by m; up to 256 rows k is cut into slices where the
+ * weight once for all rows).  Nine to 16 rows run as two such passes, Q4_K / Q5_K always, the other types where that is the
+ * faster; larger m takes the MFMA GEMM, whose tiles are 64, 128 or 256 token rows, the lowest that holds them all up to
+ * 256 rows and above by the workgroups that they make; up to 256 rows k is cut into slices where the
  * weight-row tiles alone would leave CUs idle.
  * A K-quant's k that is not a multiple of 1024 (2816, 3584, 5120 ...) has the small-batch kernel where all of k fits a
  * CU's LDS and the matrix has 8192 rows or more (512 or more from four activation rows on); otherwise up to 16 rows run
  * as per-row GEMVs first.
  * MFMA GEMM.  The K-quant (k % 256 == 0) and Q8_0 / Q4_0 (k % 128 == 0) GEMMs multiply f16-rounded
  * weights and activations like the reference's mul_mm, the other kernels keep
- * every product exact.
+ * every product exact (nine to 16 rows: by the route that the size takes).
  * Requires k % block_elems == 0; Q4_K / Q5_K need a 16-byte aligned `w_blocks`,
- * the other types a 2-byte aligned one. */
+ * the other types a 2-byte aligned one.  Q6_K tiles fetch aligned words and a few Q6_K rows aligned 16-byte pieces, whole ones
+ * also where only a part of one belongs to the matrix: up to two bytes ahead of its first block and 14 behind its last one, in
+ * the word or piece that holds a byte of it, may be read (and are not used). */
 HQ_API int hq_qmatmul_ggml(void* stream, const void* x, hq_act_dtype xdt, const void* w_blocks, float* y,
                     uint32_t m, uint32_t n, uint32_t k, hq_ggml_type t);
 
-/* How hq_qmatmul_ggml[_ws] cuts k for up to 256 activation rows on the tile route: `slices` slices of
+/* How hq_qmatmul_ggml[_ws] cuts k for up to 256 activation rows on the tile route (a size of nine to 16 rows that runs as two
+ * passes by its activations' type and its weights' alignment is not cut, whatever this says): `slices` slices of
  * `blocks_per_slice` 256-element runs each (the last one shorter), every slice a launch-time workgroup set of its own whose
  * partial products a second launch adds in slice order.  slices = 1: no cut.  (slices - 1) * blocks_per_slice < k / 256
  * always holds, so no slice starts past the end of a row.  Pure host arithmetic; a query for tests and for sizing. */
@@ -177,8 +181,8 @@ HQ_API int hq_qmatmul_gated_ggml_ws(void* stream, const void* x, hq_act_dtype xd
  * differently and the results agree to a few units in the last place.  Exists where
  * hq_qmatmul_swiglu_ggml_workspace_bytes() is not 0 (Q4_K /
  * Q5_K on the tile route: more rows than the small-batch kernels take, k % 256 == 0); other calls return
- * HQ_ERR_UNSUPPORTED and the caller issues the separate calls.  The separate calls run 256-row tiles from 257 rows
- * on, which use the matrix cores better: this form pays for few weight rows (the shared expert: 512) or few tokens,
+ * HQ_ERR_UNSUPPORTED and the caller issues the separate calls.  The separate calls run 256-row tiles where those fill
+ * the device, which use the matrix cores better: this form pays for few weight rows (the shared expert: 512) or few tokens,
  * not for a 12288-row layer over thousands of tokens.  gate_row_scales / up_row_scales: both null, or both from
  * hq_weight_row_scales_ggml (n floats each). */
 HQ_API size_t hq_qmatmul_swiglu_ggml_workspace_bytes(uint32_t m, uint32_t n, uint32_t k, hq_act_dtype xdt, hq_ggml_type t);
