@@ -726,8 +726,7 @@ int launch_krows_s(hipStream_t s, KRowsArgs& a, uint32_t cus) {
 template <int TYPE, bool WHOLE>
 int launch_krows_w(hipStream_t s, KRowsArgs& a, bool f32, uint32_t cus) {
     if (!f32) return launch_krows_s<TYPE, false, 2, WHOLE>(s, a, cus);
-    if constexpr (!WHOLE)  // (half of nine rows or more)
-        if (a.m <= 4u) return launch_krows_s<TYPE, true, 3, WHOLE>(s, a, cus);
+    if (a.m <= 4u) return launch_krows_s<TYPE, true, 3, WHOLE>(s, a, cus);  // (nine rows: passes of five and four)
     if (a.m == 5u) return launch_krows_s<TYPE, true, 4, WHOLE>(s, a, cus);
     return launch_krows<TYPE, true, 3, 2, 1, 16, WHOLE>(s, a, krows_form(TYPE == HQ_Q6_K, true, a.m, a.nsb, a.units, cus), cus);
 }

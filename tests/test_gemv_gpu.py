@@ -314,6 +314,23 @@ def test_rows_in_registers_in_two_passes(dev, t, xdt, m, n, k, takes):
         assert torch.equal(gate, sep)
 
 
+@pytest.mark.parametrize("n,k", [(5120, 5120), (4096, 6144), (2816, 9216), (4112, 4352), (4096, 2816)])
+def test_nine_rows_over_long_k_in_two_passes(dev, n, k):
+    """Nine f32 rows of Q4_0 are passes of five and four, also over more than sixteen super-blocks of k, where a wave takes two or three: the bits
+    of the two passes' own calls."""
+    t, m = HQ_Q4_0, 9
+    x = torch.randn(m, k, generator=torch.Generator(device=dev).manual_seed(n), device=dev)
+    w, ref = _rows_ref(dev, t, n, k, x, k)
+    y, parts = torch.full((m, n), float("nan"), device=dev), torch.full((m, n), float("nan"), device=dev)
+    call = lambda: ops.quantized_matmul_ggml(x, w, y, GgmlQuantizedMatmulParams(m, n, k, t))  # noqa: E731
+    call()
+    assert len(launched_kernels(call)) == 2 and all("krows_kernel" in s for s in launched_kernels(call))
+    for r0, r1 in ((0, 5), (5, 9)):
+        ops.quantized_matmul_ggml(x[r0:r1], w, parts[r0:r1], GgmlQuantizedMatmulParams(r1 - r0, n, k, t))
+    assert torch.equal(y, parts)
+    assert ((y - ref).norm() / ref.norm()).item() <= 6.6e-7
+
+
 def test_two_passes_allocate_nothing(dev):
     """hq_qmatmul_ggml without a workspace takes one from the stream's allocator for a tile, and none for two passes."""
     n, k, t = 4096, 4096, HQ_Q8_0
