@@ -16,13 +16,19 @@ namespace hq {
 //   388 / 206, 8192 x 2816 21 / 14) and Q6_K of seven and eight rows (4096 x 4096 17.6 / 12.9), behind over Q4_K and Q5_K (12288 x 4096 16.2 / 18.0).
 // Long k in slices (a launch each, about 4 us ahead of the first product): 4096 x 12288 at five rows f32 Q4_K 28.4 / 21.4, Q6_K 39.8 / 25.9, Q8_0 36 / 22, bf16 Q5_K
 //   22.1 / 18.9; behind for fewer rows over K-quants (Q6_K bf16 at four 17.6 / 21.3) and at six to eight f32 rows (Q4_K 28.8 / 37.6).
+// Rounds: one group of sixteen rows per CU.  K-quants under four f32 rows are ahead in a round that is whole or nearly so and from one and a half rounds
+// on, not with a few more groups than CUs, which take a second round for themselves: four f32 rows, 3840 and 4080 x 5120 Q4_K 10.9 / 9.1, 11.0 / 9.2, x 2816 Q6_K
+// 9.5 / 7.9 (x 1024 6.0 / 6.2).
 bool gemv_krows_takes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32_t n, uint32_t k, const void* w) {
-    if (m < 2 || m > 8 || n % 16u || k % 256u || k < 1024 || !is_aligned(w, 16)) return false;
+    uint32_t cus = 0;
+    if (m < 2 || m > 8 || n % 16u || k % 256u || k < 1024 || !is_aligned(w, 16) || cu_count(&cus)) return false;
     const bool f32 = xdt != HQ_BF16, head = n >= 32768, sliced = krows_slices(k / 256u, f32, m) > 1u;
     const bool b32 = t == HQ_Q8_0 || t == HQ_Q4_0;
     if (!b32 && t != HQ_Q4_K && t != HQ_Q5_K && t != HQ_Q6_K) return false;
     const bool odd_k = k % 1024u != 0;  // k for which the K-quants have no chunked small-batch kernel
     if (t == HQ_Q8_0 && (uint64_t)n * k < 10u << 20) return false;  // (small ones: gemv_q80_rows_walked, gemvr32.hip)
+    const uint32_t units = n / 16u;
+    const bool whole_round = units <= cus && units * 16u >= (t == HQ_Q6_K && k < 2048 ? 16u : 15u) * cus, overhang = units > cus && 2u * units < 3u * cus;
     if (!f32) {
         if (t == HQ_Q4_0) return !head && (n < 16384 || k > 4096) && (m >= 3 || (uint64_t)n * k >= 6u << 20);
         if (t == HQ_Q8_0) return head ? true : sliced ? m >= 4 || (m == 3 && !odd_k) : n >= 16384 && k <= 4096 ? false : m >= 4 || (n >= 8192 && n >= k);
@@ -40,10 +46,10 @@ bool gemv_krows_takes(hq_ggml_type t, hq_act_dtype xdt, uint32_t m, uint32_t n, 
     if (t == HQ_Q8_0) return head || (sliced ? m >= 4 || (m == 3 && !odd_k) : n >= 16384 && k <= 4096 ? m >= 5 : m == 5 || (m == 4 && n >= 4096) || (n >= 8192 && n >= k));
     if (head) return k >= (t == HQ_Q5_K ? 5120u : 4096u);
     if (n >= 16384 && k <= 4096) return t == HQ_Q6_K && m >= 4;
-    if (n < 4096) return sliced ? m >= 4 : m == 5 && k > 4096;
+    if (units <= cus && !whole_round) return sliced ? m >= 4 : m == 5 && k > 4096;
     if (odd_k && n >= 8192 && k <= 4096) return m >= 3;
-    if (t == HQ_Q6_K && !sliced && n < 6144 && n > 4096) return false;
-    return m >= (n >= 16384 && t == HQ_Q4_K ? 3u : t == HQ_Q5_K && sliced && n > 4096 ? 5u : 4u) && (m == 5 || n == 4096 || n >= 6144 || sliced);
+    if (t == HQ_Q6_K && !sliced && overhang) return false;
+    return m >= (n >= 16384 && t == HQ_Q4_K ? 3u : t == HQ_Q5_K && sliced && !whole_round ? 5u : 4u) && (m == 5 || !overhang || sliced);
 }
 
 // Gate + up + SwiGLU of a few rows (n rows a matrix, one slice of k): both matrices' groups by the same workgroup, gate then up.  us, the walk of

@@ -314,6 +314,20 @@ def test_rows_in_registers_in_two_passes(dev, t, xdt, m, n, k, takes):
         assert torch.equal(gate, sep)
 
 
+@pytest.mark.parametrize("t", [HQ_Q4_K, HQ_Q5_K, HQ_Q6_K])
+def test_rows_in_registers_by_rounds_of_groups(dev, t):
+    """Four f32 rows over K-quants: from fifteen sixteenths of a round of groups of sixteen rows to a whole one and from one and a half on."""
+    m, k, m16 = 4, 2048, 16 * torch.cuda.get_device_properties(dev).multi_processor_count
+    x = torch.randn(m, k, generator=torch.Generator(device=dev).manual_seed(t), device=dev)
+    for n, takes in ((m16 * 15 // 16 - 16, False), (m16 * 15 // 16, True), (m16 - 16, True), (m16, True), (m16 + 16, False), (m16 * 3 // 2 - 16, False), (m16 * 3 // 2, True)):
+        w, ref = _rows_ref(dev, t, n, k, x, 5)
+        y = torch.full((m, n), float("nan"), device=dev)
+        call = lambda: ops.quantized_matmul_ggml(x, w, y, GgmlQuantizedMatmulParams(m, n, k, t))  # noqa: E731,B023
+        call()
+        assert all("krows_kernel" in s for s in launched_kernels(call)) == takes, n
+        assert ((y - ref).norm() / ref.norm()).item() <= (6.6e-7 if takes else 1e-5)
+
+
 @pytest.mark.parametrize("n,k", [(5120, 5120), (4096, 6144), (2816, 9216), (4112, 4352), (4096, 2816)])
 def test_nine_rows_over_long_k_in_two_passes(dev, n, k):
     """Nine f32 rows of Q4_0 are passes of five and four, also over more than sixteen super-blocks of k, where a wave takes two or three: the bits
