@@ -328,6 +328,22 @@ def test_rows_in_registers_by_rounds_of_groups(dev, t):
         assert ((y - ref).norm() / ref.norm()).item() <= (6.6e-7 if takes else 1e-5)
 
 
+@pytest.mark.parametrize("t,xdt,m,n,k", [
+    (HQ_Q4_K, "bf16", 5, 8192, 1024), (HQ_Q6_K, "f32", 8, 12288, 1280), (HQ_Q4_0, "f32", 4, 12272, 1024), (HQ_Q8_0, "bf16", 8, 12304, 1280),
+    (HQ_Q5_K, "bf16", 4, 14352, 1536), (HQ_Q4_0, "f32", 5, 20496, 1280), (HQ_Q6_K, "bf16", 7, 8208, 1536), (HQ_Q8_0, "f32", 6, 14320, 1024),
+])
+def test_rows_in_registers_over_few_super_blocks(dev, t, xdt, m, n, k):
+    """Two and three groups of four to six waves side by side, also where the last round is short of groups."""
+    x = torch.randn(m, k, generator=torch.Generator(device=dev).manual_seed(n + m), device=dev)
+    x = x.to(torch.bfloat16) if xdt == "bf16" else x
+    w, ref = _rows_ref(dev, t, n, k, x, k + m)
+    y = torch.full((m + 1, n), float("nan"), device=dev)
+    call = lambda: ops.quantized_matmul_ggml(x, w, y, GgmlQuantizedMatmulParams(m, n, k, t))  # noqa: E731
+    call()
+    assert all("krows_kernel" in s for s in launched_kernels(call))
+    assert torch.isnan(y[m]).all() and ((y[:m] - ref).norm() / ref.norm()).item() <= 6.6e-7
+
+
 @pytest.mark.parametrize("n,k", [(5120, 5120), (4096, 6144), (2816, 9216), (4112, 4352), (4096, 2816)])
 def test_nine_rows_over_long_k_in_two_passes(dev, n, k):
     """Nine f32 rows of Q4_0 are passes of five and four, also over more than sixteen super-blocks of k, where a wave takes two or three: the bits

@@ -58,3 +58,33 @@ def test_every_slice_of_every_length_has_a_split(plan):
     rows once ended in a slice of three super-blocks, for which there is none), and every split is one that the kernel has a form for."""
     r = plan(PROGRAM)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+GROUPS = r"""
+#include <stdio.h>
+#include "gemvk_plan.h"
+int main() {
+    using namespace hq;
+    const uint32_t cus = 256;
+    unsigned more = 0;
+    for (uint32_t nsb = 4; nsb <= 36; ++nsb)
+        for (uint32_t m = 2; m <= 8; ++m)
+            for (uint32_t units = 1; units <= 4200; ++units)
+                for (int f32 = 0; f32 < 2; ++f32) {
+                    if (f32 && m > 5 && nsb > 16) continue;
+                    const KSplit p = krows_form_of(false, f32, m, nsb, units, cus), q = krows_form(false, f32, m, nsb, units, cus);
+                    more += q.rg != p.rg;
+                    auto all = [&](const KSplit& x) { return (units + x.rg * cus - 1) / (x.rg * cus) * krows_load(nsb, x.kp, x.rg); };
+                    if (q.kp != p.kp || q.s != p.s || q.w != p.w || q.rg < p.rg || q.rg > 4 || q.rg * q.kp > q.w || all(q) > all(p) || q.load != krows_load(nsb, q.kp, q.rg) ||
+                        (q.rg > p.rg && units < q.rg * cus))
+                        return printf("%u super-blocks, %u rows, %u groups: kp %u rg %u -> kp %u rg %u\n", nsb, m, units, p.kp, p.rg, q.kp, q.rg), 1;
+                }
+    return more == 0;
+}
+"""
+
+
+def test_groups_side_by_side_leave_the_sums_alone(plan):
+    """More groups side by side: the same waves to a group, no more work on a SIMD over all rounds, no CU without a group, within the kernel's waves."""
+    r = plan(GROUPS)
+    assert r.returncode == 0, r.stdout + r.stderr
