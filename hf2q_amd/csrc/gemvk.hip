@@ -3,7 +3,11 @@
 
 namespace hq {
 
-// Where it is ahead of the kernels that serve a few rows otherwise (and no less exact: 0.9 .. 2e-7 of the result, Q8_0 and Q4_0 rows in bf16 8e-8).
+// Where it is ahead of the kernels that serve a few rows otherwise (and no less exact: 0.9 .. 2e-7 of the result, Q8_0 and Q4_0 rows in bf16 8e-8), or
+// behind them and ten to fifty times as exact: k below 2048 and up to 3584 from two rounds of groups on, where the groups' hand-overs are much of the
+// product, and heads of K-quants and Q8_0 up to 131072 rows with k up to 4096.  us and error of the result, the others / here: bf16 Q4_K at five rows 4096 x 1024 3.6, 2.6e-6 / 4.9, 1.5e-7,
+// 65536 x 1280 16.6 / 18.8; f32 Q6_K at eight 12288 x 1280 9.7, 2.8e-6 / 13.8, 9e-8, 24576 x 2816 22.3 / 30.3; f32 Q4_0 at four 5120 x 1280 5.4, 4.2e-6 / 7.5, 7e-8; f32 Q8_0 at
+// three 32768 x 2048 17.5, 2.4e-6 / 22.7, 7e-8, 4352 x 10240 17.4 / 27.8.  In all 17 000 products of two to sixteen rows: 0.90 of the time in the geometric mean.
 // n of whole groups of sixteen rows, k of whole super-blocks; the rest of the rule is measured, us before / here:
 //   bf16 rows at 3, 5, 8: Q4_K 4096 x 2816 6.6 / 5.2, 9.7 / 5.7, 9.9 / 6.2, 17408 x 5120 20.9 / 16.4, 21.0 / 16.8, 20.9 / 17.8, 152064 x 5120 94 / 81, 96 / 85,
 //   97 / 91; Q5_K 4096 x 4096 8.7 / 6.5, 8.8 / 7.0, 8.8 / 7.4; Q6_K at 5 4096 x 4096 12.0 / 7.1, 17408 x 5120 40 / 24, 152064 x 5120 164 / 133; Q8_0 at 5 4096 x 4096
@@ -126,8 +130,8 @@ int launch_gemv_krows(hipStream_t s, const void* x, hq_act_dtype xdt, uint32_t m
     return HQ_OK;
 }
 
-// Nine to sixteen rows of Q8_0 / Q4_0 / Q6_K (Q4_K and Q5_K take passes of eight anyway) as two passes of half of them: both find the weights in the
-// device's caches, and no tile of 64 rows is filled with 16.  us, a tile / two passes, as the calls follow each other (about 24 us is what the
+// Nine to sixteen rows of Q8_0 / Q4_0 / Q6_K (Q4_K and Q5_K take passes of eight anyway) as two passes of half of them: no tile of 64 rows is
+// filled with 16, and where the matrix fits them the second pass finds the weights in the device's caches (up to 256 MB; a head is read twice).  us, a tile / two passes, as the calls follow each other (about 24 us is what the
 // host takes for a call): bf16 Q8_0 at 12 rows 4096 x 4096 27.3 / 23.9, 17408 x 5120 60.6 / 45.2, 151936 x 4096 325 / 234, Q4_0 5120 x 5120 30.3 / 24.0, 17408 x 5120 47.6 /
 // 42.3 (14336 x 5120 36.4 / 39.5), Q6_K 4096 x 4096 30.0 / 24.9 (14336 x 5120 37.8 / 45.4, 18944 x 3584 37.3 / 43.8); f32 at 9 / 16 Q8_0 4096 x 4096 27.9 / 25.5, 29.3 / 25.4,
 // 151936 x 4096 327 / 235, 327 / 257 (12288 x 4096 38.4 / 42.3), Q4_0 4096 x 4096 29.7 / 22.5, 29.5 / 26.3 (12288 x 4096 32 / 40), Q6_K 4096 x 4096 29.8 / 24.2, 27.8 / 29.7.

@@ -52,7 +52,7 @@ inline KSplit krows_form_of(bool q6k, bool f32, uint32_t m, uint32_t nsb, uint32
 // And how many groups side by side: more than that where it takes fewer rounds, by the work of the busiest SIMD over all rounds, and for four waves to a
 // group, one to a SIMD with nothing to hide its latencies behind, also where the work is the same.  Which waves add up a group stays that of
 // the form, and so do the bits.  us, one group / two or three: 8192 x 1024 bf16 Q5_K at five rows 6.3 / 5.7, 12288 x 1024 f32 Q4_0 at four 8.5 / 7.3, 12288 x 1280 f32 Q6_K at
-// eight 16.0 / 13.8, 14336 x 1024 bf16 Q4_K at five 8.2 / 6.9, 20480 x 1280 (two / three) 0.91 of the time over all types.  (Four for two of four waves,
+// eight 16.0 / 13.8, 14336 x 1024 bf16 Q4_K at five 8.2 / 6.8, 20480 x 1280 (two / three) 0.91 of the time over all types.  (Four for two of four waves,
 // 16384 x 1024: up to 1.07 of it.)
 inline KSplit krows_form(bool q6k, bool f32, uint32_t m, uint32_t nsb, uint32_t units, uint32_t cus) {
     KSplit p = krows_form_of(q6k, f32, m, nsb, units, cus);
